@@ -10,8 +10,8 @@ apply several fused blocks per HBM pass on the FP32 matrix cores, FP64
 renormalisation).  value = gates * 2^30 / step time.
 
 Beside it, in the same process:
-  * the plain FP64 form of the same circuit (complex128, one kernel per gate),
-    for the speedup and for 1 - F / max-abs of the fused state;
+  * the plain FP64 form of the same circuit (complex128, the gates' own
+    arithmetic, many gates per HBM pass), for the speedup and for 1 - F / max-abs of the fused state;
   * the dominant kernel's roofline: average duration of the fused
     matrix-core kernel from HIP events recorded on the state's stream inside
     the timed steps; tile programs are bound by the FP32 matrix cores
@@ -482,6 +482,7 @@ def bench_qft(args):
     st = plain.device_state
     m1, n1, b1, _ = timing(hip, st, qcs_amd.K_1Q)
     m2, n2, b2, _ = timing(hip, st, qcs_amd.K_CU)
+    m3, n3, b3, _ = timing(hip, st, qcs_amd.K_FUSED)
     off = 12345678 % (N - (1 << 16))
     y = np.arange(off, off + (1 << 16), dtype=np.int64)
     ref = np.exp(2j * np.pi * ((int(rev(np.array([b]))[0]) * rev(y)) % N) / N) / math.sqrt(N)
@@ -512,6 +513,8 @@ def bench_qft(args):
         "k_cu_and_swap": {"launches": n2, "avg_ms": m2 / max(n2, 1),
                           "gbs_algorithmic": (b2 / max(n2, 1)) / (m2 / max(n2, 1) * 1e-3) / 1e9
                           if n2 else None},
+        "gate_passes": {"launches": n3, "avg_ms": m3 / max(n3, 1),
+                        "gbs": b3 / (m3 * 1e-3) / 1e9 if n3 else None},
         "fused_fp32_tiles": {"ms_per_step": tf * 1e3, "amp_updates_per_s": G * N / tf,
                              "fused_blocks": blocks, "hbm_passes": passes,
                              "one_minus_f": omf, "max_abs_err": mx},
@@ -1190,6 +1193,7 @@ def main():
         m1, n1, b1, _ = timing(hip, pstate, qcs_amd.K_1Q)
         m2, n2, b2, _ = timing(hip, pstate, qcs_amd.K_CU)
         mv1, mv2 = moved(hip, pstate, qcs_amd.K_1Q), moved(hip, pstate, qcs_amd.K_CU)
+        m3, n3, b3, _ = timing(hip, pstate, qcs_amd.K_FUSED)
         omf, mx = fused.compare_with(plain)
         result["plain_fp64"] = {
             "ms": Tp * 1e3,
@@ -1200,6 +1204,11 @@ def main():
             "k_cu_avg_ms": m2 / max(n2, 1),
             "k_cu_gbs": (b2 / max(n2, 1)) / (m2 / max(n2, 1) * 1e-3) / 1e9 if n2 else None,
         }
+        # many gates per sweep over the state: the passes' own bytes
+        result["plain_fp64"]["gate_passes"] = {
+            "launches": n3, "avg_ms": m3 / max(n3, 1),
+            "gbs": b3 / (m3 * 1e-3) / 1e9 if n3 else None,
+            "hbm_frac": b3 / (m3 * 1e-3) / 1e9 / HBM_PEAK_GBS if n3 else None}
         result["plain_fp64"]["k_1q_hbm_frac"] = (result["plain_fp64"]["k_1q_gbs"] or 0) / HBM_PEAK_GBS
         # the plain form as a whole: algorithmic bytes of every gate over the
         # gate kernels' time, and over the step's wall time

@@ -48,7 +48,8 @@ typedef struct qcs_hip_state qcs_hip_state;
 const char *qcs_hip_last_error(void);
 /* 1 if a HIP device is usable, 0 otherwise (never aborts) */
 int qcs_hip_device_available(void);
-/* hipDeviceSynchronize on the current device */
+/* launches the queued gates of every state on the current device, then
+ * hipDeviceSynchronize */
 int qcs_hip_device_sync(void);
 /* "<gcn arch>:<compute units>" of the current device (e.g. "gfx950:256"),
  * the key of cached autotuning results; no reference counterpart */
@@ -69,7 +70,7 @@ int qcs_hip_state_flags(const qcs_hip_state *s);
 /* |basis>; the compat scratch buffer is zeroed as q_state_init does
  * (src/q_state.c:93-99) */
 int qcs_hip_state_set_basis(qcs_hip_state *s, long basis);
-/* wait for every op queued on the state's stream */
+/* launch the queued gates and wait for everything on the state's stream */
 int qcs_hip_sync(qcs_hip_state *s);
 
 /* ---- host <-> device copies (observation, tests) -----------------------
@@ -86,7 +87,15 @@ int qcs_hip_read_scratch(qcs_hip_state *s, long offset, long count,
  * (out-of-place plus buffer swap in compat mode).  Arithmetic per output is
  * c_add(c_mul(g0, v0), c_mul(g1, v1)) without FMA contraction
  * (src/complex.c:23-57), so c128 results equal the reference's sequential
- * loop bit for bit. */
+ * loop value for value (a zero may differ in sign).
+ *
+ * Textbook states of 7 qubits and up: a gate call checks its arguments and
+ * queues the gate; gates are launched together, several to a sweep over the
+ * state, while later ones are still being queued, and what is left when an
+ * entry point reads or changes the state otherwise, waits for it
+ * (qcs_hip_sync, qcs_hip_device_sync) or destroys it.  A launch failure is
+ * reported by the call that launches.  A program that waits with HIP's own
+ * calls instead of these has to call one of these first. */
 int qcs_hip_apply_1q(qcs_hip_state *s, int target, const double m[8]);
 /* qcs_hip_apply_cu replaces q_apply_2q_gate / q_apply_2q_gate_gpu
  * (src/q_gates.c:158-298, src/gpu_complex.c:704-921): controlled 2x2 on
@@ -305,7 +314,7 @@ int qcs_hip_compare(qcs_hip_state *a, qcs_hip_state *b, double *one_minus_f,
  * recorded on the state's stream; totals are kept per kernel class. */
 #define QCS_HIP_K_1Q 0
 #define QCS_HIP_K_CU 1
-#define QCS_HIP_K_FUSED 2
+#define QCS_HIP_K_FUSED 2 /* fused blocks, tile programs, passes of plain gates */
 #define QCS_HIP_K_COMPOSE 3
 #define QCS_HIP_K_REDUCE 4
 #define QCS_HIP_K_OTHER 5

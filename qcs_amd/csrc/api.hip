@@ -1,5 +1,6 @@
 // extern "C" entry points of the backend (declared in include/qcs_hip.h):
 // argument validation, state lifetime, copies, kernel timers, dispatch.
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdarg>
@@ -62,6 +63,10 @@ int launch_check(const char *what) {
     return fail(QCS_HIP_EDEVICE, "%s: injected failure (QCS_HIP_INJECT_FAULT)", what);
   return check_hip(e, what);
 }
+
+// states whose gates are queued, for qcs_hip_device_sync
+static std::mutex g_states_mu;
+static std::vector<qcs_hip_state *> g_states;
 
 static hipEvent_t take_event(qcs_hip_state *s) {
   if (!s->free_events.empty()) {
@@ -158,6 +163,12 @@ static int check_state(const qcs_hip_state *s) {
   return 0;
 }
 
+// the state as every gate call so far left it: what is queued is launched
+static int ready(qcs_hip_state *s) {
+  const int rc = check_state(s);
+  return rc ? rc : queue_flush(s);
+}
+
 static int check_qubit(const qcs_hip_state *s, int q, const char *what) {
   if (q < 0 || q >= s->n)
     return fail(QCS_HIP_EINVAL, "%s: qubit %d out of range [0,%d)", what, q,
@@ -197,6 +208,16 @@ static int copy_out(qcs_hip_state *s, const void *dev, long off, long count,
     done += m;
   }
   return 0;
+}
+
+static uint64_t or_bits(const double *x, long n) {
+  uint64_t r = 0;
+  for (long i = 0; i < n; ++i) {
+    uint64_t b;
+    std::memcpy(&b, x + i, 8);
+    r |= b;
+  }
+  return r;
 }
 
 int validate_blocks(int n, const qcs_hip_block *blocks, int num_blocks,
@@ -247,6 +268,13 @@ int qcs_hip_device_available(void) {
 }
 
 int qcs_hip_device_sync(void) {
+  int dev = 0, rc;
+  QCS_HIP_TRY(hipGetDevice(&dev));
+  {
+    std::lock_guard<std::mutex> lock(g_states_mu);
+    for (qcs_hip_state *s : g_states)
+      if (s->device == dev && (rc = queue_flush(s))) return rc;
+  }
   QCS_HIP_TRY(hipDeviceSynchronize());
   return 0;
 }
@@ -308,11 +336,28 @@ int qcs_hip_state_create(qcs_hip_state **out, int num_qubits, int precision,
     free_state(s);
     return rc;
   }
+  if (num_qubits >= kPassMinQubits && !(flags & QCS_HIP_COMPAT)) {
+    try {
+      std::lock_guard<std::mutex> lock(g_states_mu);
+      g_states.push_back(s);
+    } catch (const std::exception &) {
+      free_state(s);
+      return fail(QCS_HIP_ENOMEM, "host allocation failed");
+    }
+    s->queued = true;
+  }
   *out = s;
   return 0;
 }
 
-void qcs_hip_state_destroy(qcs_hip_state *s) { free_state(s); }
+void qcs_hip_state_destroy(qcs_hip_state *s) {
+  if (s && s->queued) {
+    std::lock_guard<std::mutex> lock(g_states_mu);
+    g_states.erase(std::find(g_states.begin(), g_states.end(), s));
+  }
+  if (s) (void)queue_flush(s);
+  free_state(s);
+}
 
 int qcs_hip_state_num_qubits(const qcs_hip_state *s) { return s ? s->n : 0; }
 int qcs_hip_state_precision(const qcs_hip_state *s) { return s ? s->precision : -1; }
@@ -320,9 +365,10 @@ int qcs_hip_state_flags(const qcs_hip_state *s) { return s ? s->flags : 0; }
 
 int qcs_hip_state_set_basis(qcs_hip_state *s, long basis) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (basis < 0 || uint64_t(basis) >= s->size)
     return fail(QCS_HIP_EINVAL, "basis %ld outside 2^%d", basis, s->n);
+  bound_reset(s, 0.0);
   if ((rc = launch_fill_basis(s, s->vec, uint64_t(basis), 1))) return rc;
   if (s->scratch && (rc = launch_fill_basis(s, s->scratch, 0, 0))) return rc;
   return 0;
@@ -330,33 +376,35 @@ int qcs_hip_state_set_basis(qcs_hip_state *s, long basis) {
 
 int qcs_hip_sync(qcs_hip_state *s) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   QCS_HIP_TRY(hipStreamSynchronize(s->stream));
   return 0;
 }
 
 int qcs_hip_read(qcs_hip_state *s, long offset, long count, double *out) {
   int rc;
-  if ((rc = check_state(s)) || (rc = check_range(s, offset, count, out))) return rc;
+  if ((rc = ready(s)) || (rc = check_range(s, offset, count, out))) return rc;
   return copy_out(s, s->vec, offset, count, out);
 }
 
 int qcs_hip_read_scratch(qcs_hip_state *s, long offset, long count,
                          double *out) {
   int rc;
-  if ((rc = check_state(s)) || (rc = check_range(s, offset, count, out))) return rc;
+  if ((rc = ready(s)) || (rc = check_range(s, offset, count, out))) return rc;
   if (!s->scratch) return fail(QCS_HIP_EUNSUP, "state has no scratch buffer (not compat)");
   return copy_out(s, s->scratch, offset, count, out);
 }
 
 int qcs_hip_write(qcs_hip_state *s, long offset, long count, const double *in) {
   int rc;
-  if ((rc = check_state(s)) || (rc = check_range(s, offset, count, in))) return rc;
+  if ((rc = ready(s)) || (rc = check_range(s, offset, count, in))) return rc;
   const size_t chunk_amps = size_t(1) << 20;
   if ((rc = ensure_pinned(s, chunk_amps * 16))) return rc;
+  uint64_t exps = 0;  // the exponent bits of every value, or-ed
   for (long done = 0; done < count;) {
     const long m = long(std::min<size_t>(chunk_amps, size_t(count - done)));
     QCS_HIP_TRY(hipStreamSynchronize(s->stream));  // staging buffer free
+    exps |= or_bits(in + 2 * done, 2 * m);
     if (s->precision == QCS_HIP_C128) {
       std::memcpy(s->host, in + 2 * done, size_t(m) * 16);
     } else {
@@ -368,6 +416,20 @@ int qcs_hip_write(qcs_hip_state *s, long offset, long count, const double *in) {
                                hipMemcpyHostToDevice, s->stream));
     done += m;
   }
+  if (count > 0) {
+    // |x| < 2 for every value unless some exponent says otherwise
+    double top = 2.0;
+    if (((exps >> 52) & 0x7ff) >= 0x400) {
+      top = 0.0;
+      for (long i = 0; i < 2 * count; ++i)
+        if (!(std::fabs(in[i]) <= top)) top = std::fabs(in[i]);
+    }
+    const double b = std::log2(top) + 0.5 * std::log2(2.0 * double(count));
+    // the amplitudes left as they were keep their bound
+    const double old = uint64_t(count) == s->size ? b : s->log2_bound;
+    bound_reset(s, (old > b ? old : b) + 0.5);
+    if (!(b < 1e300)) bound_reset(s, b);  // infinite or NaN
+  }
   QCS_HIP_TRY(hipStreamSynchronize(s->stream));
   return 0;
 }
@@ -376,7 +438,7 @@ int qcs_hip_apply_1q(qcs_hip_state *s, int target, const double m[8]) {
   int rc;
   if ((rc = check_state(s)) || (rc = check_qubit(s, target, "apply_1q"))) return rc;
   if (!m) return fail(QCS_HIP_EINVAL, "null gate matrix");
-  return launch_1q(s, target, m);
+  return queue_gate(s, QCS_HIP_G_1Q, target, -1, m);
 }
 
 int qcs_hip_apply_cu(qcs_hip_state *s, int control, int target,
@@ -387,7 +449,7 @@ int qcs_hip_apply_cu(qcs_hip_state *s, int control, int target,
     return rc;
   if (control == target) return fail(QCS_HIP_EINVAL, "apply_cu: control == target");
   if (!m) return fail(QCS_HIP_EINVAL, "null gate matrix");
-  return launch_cu(s, control, target, m);
+  return queue_gate(s, QCS_HIP_G_CU, target, control, m);
 }
 
 int qcs_hip_apply_swap(qcs_hip_state *s, int a, int b) {
@@ -397,12 +459,12 @@ int qcs_hip_apply_swap(qcs_hip_state *s, int a, int b) {
     return rc;
   if (a == b) return 0;
   if (s->flags & QCS_HIP_COMPAT) return fail(QCS_HIP_EUNSUP, "swap in compat mode");
-  return launch_swap(s, a, b);
+  return queue_gate(s, QCS_HIP_G_SWAP, a, b, nullptr);
 }
 
 int qcs_hip_phase_flip(qcs_hip_state *s, long index) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (index < 0 || uint64_t(index) >= s->size)
     return fail(QCS_HIP_EINVAL, "phase flip index %ld outside 2^%d", index, s->n);
   if (s->flags & QCS_HIP_COMPAT) return phase_flip_compat(s, index);
@@ -411,14 +473,14 @@ int qcs_hip_phase_flip(qcs_hip_state *s, long index) {
 
 int qcs_hip_diffusion(qcs_hip_state *s) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (s->flags & QCS_HIP_COMPAT) return diffusion_compat(s);
   return grover_textbook(s, -1, 1);
 }
 
 int qcs_hip_grover(qcs_hip_state *s, long marked, long iterations) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (iterations <= 0) return 0;
   if (marked >= 0 && uint64_t(marked) >= s->size)
     return fail(QCS_HIP_EINVAL, "marked index %ld outside 2^%d", marked, s->n);
@@ -434,25 +496,29 @@ int qcs_hip_grover(qcs_hip_state *s, long marked, long iterations) {
 
 int qcs_hip_norm_sq(qcs_hip_state *s, double *norm_sq) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (!norm_sq) return fail(QCS_HIP_EINVAL, "null output");
   return reduce_norm(s, norm_sq);
 }
 
 int qcs_hip_normalize(qcs_hip_state *s, double *norm_sq_out) {
   int rc;
-  if ((rc = check_state(s))) return rc;
-  if (!norm_sq_out) return normalize_device(s);
+  if ((rc = ready(s))) return rc;
+  if (!norm_sq_out) {
+    bound_normalized(s);
+    return normalize_device(s);
+  }
   double ns = 0.0;
   if ((rc = reduce_norm(s, &ns))) return rc;
   *norm_sq_out = ns;
+  bound_normalized(s);
   if (ns > 1e-12 && ns != 1.0) return scale_state(s, 1.0 / std::sqrt(ns));
   return 0;
 }
 
 int qcs_hip_qubit_probs(qcs_hip_state *s, int qubit, double *p0, double *p1) {
   int rc;
-  if ((rc = check_state(s)) || (rc = check_qubit(s, qubit, "qubit_probs"))) return rc;
+  if ((rc = ready(s)) || (rc = check_qubit(s, qubit, "qubit_probs"))) return rc;
   double a = 0.0, b = 0.0;
   if ((rc = qubit_probs(s, qubit, &a, &b))) return rc;
   if (p0) *p0 = a;
@@ -462,7 +528,7 @@ int qcs_hip_qubit_probs(qcs_hip_state *s, int qubit, double *p0, double *p1) {
 
 int qcs_hip_measure(qcs_hip_state *s, int qubit, double u, int *outcome) {
   int rc;
-  if ((rc = check_state(s)) || (rc = check_qubit(s, qubit, "measure"))) return rc;
+  if ((rc = ready(s)) || (rc = check_qubit(s, qubit, "measure"))) return rc;
   // p0 over the bit = 0 half (src/qcs.c:253-259); p1, the norm the kept
   // half has after zeroing, only when the outcome is 1.  Where the halves'
   // runs are shorter than a line, one pass over the whole state gives both.
@@ -475,6 +541,7 @@ int qcs_hip_measure(qcs_hip_state *s, int qubit, double u, int *outcome) {
   const double ns = o == 0 ? p0 : p1;
   const int do_scale = (ns > 1e-12 && ns != 1.0) ? 1 : 0;
   const double f = do_scale ? 1.0 / std::sqrt(ns) : 1.0;
+  bound_normalized(s);
   if ((rc = collapse(s, qubit, o, f, do_scale))) return rc;
   if (outcome) *outcome = o;
   return 0;
@@ -483,17 +550,18 @@ int qcs_hip_measure(qcs_hip_state *s, int qubit, double u, int *outcome) {
 int qcs_hip_measure_seq(qcs_hip_state *s, int count, const int *qubits,
                         const double *u, int *outcomes) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (count <= 0) return 0;
   if (!qubits || !u || !outcomes) return fail(QCS_HIP_EINVAL, "null buffer");
   for (int i = 0; i < count; ++i)
     if ((rc = check_qubit(s, qubits[i], "measure_seq"))) return rc;
+  bound_normalized(s);
   return measure_seq(s, count, qubits, u, outcomes);
 }
 
 int qcs_hip_probability(qcs_hip_state *s, long index, double *p) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (!p) return fail(QCS_HIP_EINVAL, "null output");
   if (index < 0 || uint64_t(index) >= s->size) {
     *p = 0.0;  // src/qcs.c:392-393
@@ -507,7 +575,7 @@ int qcs_hip_probability(qcs_hip_state *s, long index, double *p) {
 
 int qcs_hip_argmax(qcs_hip_state *s, long *index) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (!index) return fail(QCS_HIP_EINVAL, "null output");
   return argmax(s, index);
 }
@@ -515,7 +583,7 @@ int qcs_hip_argmax(qcs_hip_state *s, long *index) {
 int qcs_hip_sample(qcs_hip_state *s, long shots, const double *u,
                    long *index_out) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (shots <= 0) return 0;
   if (!u || !index_out) return fail(QCS_HIP_EINVAL, "null buffer");
   return sample(s, shots, u, index_out);
@@ -539,7 +607,7 @@ static int check_device_buffer(const void *p, const char *what) {
 int qcs_hip_sample_noalloc(qcs_hip_state *s, long shots, const double *u_dev,
                            long *index_out_dev) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (shots <= 0) return 0;
   if ((rc = check_device_buffer(u_dev, "sample_noalloc uniforms")) ||
       (rc = check_device_buffer(index_out_dev, "sample_noalloc indices")))
@@ -551,17 +619,19 @@ int qcs_hip_apply_fused(qcs_hip_state *s, const qcs_hip_block *blocks,
                         int num_blocks, const qcs_hip_gate *gates,
                         int num_gates) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (s->flags & QCS_HIP_COMPAT)
     return fail(QCS_HIP_EUNSUP, "fusion needs textbook semantics");
   if ((rc = validate_blocks(s->n, blocks, num_blocks, gates, num_gates))) return rc;
+  for (int g = 0; g < num_gates; ++g)
+    if (gates[g].kind != QCS_HIP_G_SWAP) bound_gate(s, gates[g].m);
   return fused_apply(s, blocks, num_blocks, gates, num_gates);
 }
 
 int qcs_hip_apply_unitary(qcs_hip_state *s, int k, const int *targets,
                           const double *u) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (s->flags & QCS_HIP_COMPAT)
     return fail(QCS_HIP_EUNSUP, "fusion needs textbook semantics");
   if (k < 1 || k > QCS_HIP_MAX_FUSE || k > s->n || !targets || !u)
@@ -569,6 +639,7 @@ int qcs_hip_apply_unitary(qcs_hip_state *s, int k, const int *targets,
   for (int q = 0; q < k; ++q)
     if (targets[q] < 0 || targets[q] >= s->n || (q > 0 && targets[q] <= targets[q - 1]))
       return fail(QCS_HIP_EINVAL, "apply_unitary: targets not ascending in range");
+  bound_matrix(s, u, 1L << (2 * k));
   return fused_apply_unitary(s, k, targets, u);
 }
 
@@ -576,7 +647,7 @@ static int check_passes(qcs_hip_state *s, const qcs_hip_pass *passes, int num_pa
                         const qcs_hip_block *blocks, int num_blocks,
                         const qcs_hip_gate *gates, int num_gates) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (s->flags & QCS_HIP_COMPAT)
     return fail(QCS_HIP_EUNSUP, "fusion needs textbook semantics");
   if (s->precision != QCS_HIP_C64)
@@ -617,7 +688,10 @@ static int check_passes(qcs_hip_state *s, const qcs_hip_pass *passes, int num_pa
   }
   if (covered != num_blocks)
     return fail(QCS_HIP_EINVAL, "passes cover %d of %d blocks", covered, num_blocks);
-  return validate_blocks(s->n, blocks, num_blocks, gates, num_gates);
+  if ((rc = validate_blocks(s->n, blocks, num_blocks, gates, num_gates))) return rc;
+  for (int g = 0; g < num_gates; ++g)
+    if (gates[g].kind != QCS_HIP_G_SWAP) bound_gate(s, gates[g].m);
+  return 0;
 }
 
 int qcs_hip_apply_passes(qcs_hip_state *s, const qcs_hip_pass *passes,
@@ -640,6 +714,7 @@ int qcs_hip_apply_passes_normalize(qcs_hip_state *s, const qcs_hip_pass *passes,
   if ((rc = tiles_apply(s, passes, num_passes, blocks, num_blocks, gates, num_gates,
                         &nparts)))
     return rc;
+  bound_normalized(s);
   if (nparts < 0) return 0;  // renormalised by the last pass
   // the last pass summed |x|^2 of what it wrote: no separate read of the state
   return nparts > 0 ? normalize_from_partials(s, nparts) : normalize_device(s);
@@ -708,14 +783,14 @@ int qcs_hip_get_tuning(qcs_hip_state *s, int knob, int *value) {
 int qcs_hip_compare(qcs_hip_state *a, qcs_hip_state *b, double *one_minus_f,
                     double *max_abs) {
   int rc;
-  if ((rc = check_state(a)) || (rc = check_state(b))) return rc;
+  if ((rc = ready(a)) || (rc = ready(b))) return rc;
   if (a->n != b->n) return fail(QCS_HIP_EINVAL, "compare: sizes differ");
   return compare(a, b, one_minus_f, max_abs);
 }
 
 int qcs_hip_timing_enable(qcs_hip_state *s, int enable) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if ((rc = drain_events(s))) return rc;
   for (int c = 0; c < QCS_HIP_K_COUNT; ++c) {
     s->t_ms[c] = 0.0;
@@ -731,7 +806,7 @@ int qcs_hip_timing_enable(qcs_hip_state *s, int enable) {
 int qcs_hip_timing_read(qcs_hip_state *s, int kernel_class, double *total_ms,
                         long *launches, double *bytes, double *flops) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (kernel_class < 0 || kernel_class >= QCS_HIP_K_COUNT)
     return fail(QCS_HIP_EINVAL, "unknown kernel class %d", kernel_class);
   if ((rc = drain_events(s))) return rc;
@@ -744,7 +819,7 @@ int qcs_hip_timing_read(qcs_hip_state *s, int kernel_class, double *total_ms,
 
 int qcs_hip_timing_moved(qcs_hip_state *s, int kernel_class, double *moved_bytes) {
   int rc;
-  if ((rc = check_state(s))) return rc;
+  if ((rc = ready(s))) return rc;
   if (kernel_class < 0 || kernel_class >= QCS_HIP_K_COUNT)
     return fail(QCS_HIP_EINVAL, "unknown kernel class %d", kernel_class);
   if (!moved_bytes) return fail(QCS_HIP_EINVAL, "null output");

@@ -1,0 +1,503 @@
+// Gate passes: many plain gates in one sweep over HBM.
+//
+// A gate by itself reads and writes the state once (gates.hip: bound by HBM,
+// 5.8 TB/s in place).  A pass reads it once, runs the gates of gateplan.h's
+// program on it and writes it once, so the cost of a gate becomes its
+// arithmetic: a pass of the 28-qubit layered circuit (694 gates in 20 passes)
+// takes 2.16 ms, 4.0 TB/s, where each gate by itself took 1.2 ms; the circuit
+// went from 863 to 44.5 ms, the 28-qubit QFT (448 gates) from 270 to 24 ms.
+//
+// k_gate_pass.  One work-group per tile of 2^tb amplitudes; thread t holds 16
+// of them in registers, those that differ in the layout's four register
+// bits.  A layout change exchanges the tile through LDS, complex128 as two
+// planes (all real parts, then all imaginary parts), so a 13-bit tile takes
+// 64 KiB: two work-groups of 512 threads fit a CU, and one computes while
+// the other waits for HBM.  The arithmetic is that of gates.hip without the
+// products by exact-zero entries, which add only signed zeros; the
+// amplitudes compare equal to the per-gate kernels' (bound_gate
+// keeps states whose amplitudes could overflow out).
+#include <algorithm>
+#include <cmath>
+#include <exception>
+#include <mutex>
+#include <vector>
+
+#include "device.h"
+#include "gateplan.h"
+#include "internal.h"
+
+namespace qcs {
+
+// ---- ops on the register group -----------------------------------------------
+//
+// vr[j], vi[j]: the amplitude whose register bits are the bits of j.  Every
+// index is a compile-time constant.
+
+template <typename T>
+using Regs = T[kPAmps];
+
+// Every product of a pair is formed before any sum: each result is then
+// defined after the last use of the inputs and takes an input's register, so
+// every op leaves each amplitude in the register it came in and the joins
+// after the dispatch need no copies.  pair_end keeps the scheduler from
+// interleaving the pairs, which would need more registers than the four
+// waves a SIMD holds leave.
+__device__ __forceinline__ void pair_end() { __builtin_amdgcn_sched_barrier(0); }
+
+template <int Q, typename T>
+__device__ __forceinline__ void p_dense(Regs<T> &vr, Regs<T> &vi, const T (&m)[8]) {
+#pragma unroll
+  for (int j = 0; j < kPAmps; ++j) {
+    if (j & (1 << Q)) continue;
+    const int k = j | (1 << Q);
+    const T x0 = vr[j], y0 = vi[j], x1 = vr[k], y1 = vi[k];
+    const T a0 = m[0] * x0, a1 = m[1] * y0, a2 = m[0] * y0, a3 = m[1] * x0;
+    const T c0 = m[2] * x1, c1 = m[3] * y1, c2 = m[2] * y1, c3 = m[3] * x1;
+    const T b0 = m[4] * x0, b1 = m[5] * y0, b2 = m[4] * y0, b3 = m[5] * x0;
+    const T d0 = m[6] * x1, d1 = m[7] * y1, d2 = m[6] * y1, d3 = m[7] * x1;
+    vr[j] = (a0 - a1) + (c0 - c1);
+    vi[j] = (a2 + a3) + (c2 + c3);
+    vr[k] = (b0 - b1) + (d0 - d1);
+    vi[k] = (b2 + b3) + (d2 + d3);
+    pair_end();
+  }
+}
+
+// every imaginary part 0: {m00, m01, m10, m11}
+template <int Q, typename T>
+__device__ __forceinline__ void p_real(Regs<T> &vr, Regs<T> &vi, T m00, T m01, T m10, T m11) {
+#pragma unroll
+  for (int j = 0; j < kPAmps; ++j) {
+    if (j & (1 << Q)) continue;
+    const int k = j | (1 << Q);
+    const T x0 = vr[j], y0 = vi[j], x1 = vr[k], y1 = vi[k];
+    const T a0 = m00 * x0, a1 = m00 * y0, b0 = m10 * x0, b1 = m10 * y0;
+    const T c0 = m01 * x1, c1 = m01 * y1, d0 = m11 * x1, d1 = m11 * y1;
+    vr[j] = a0 + c0;
+    vi[j] = a1 + c1;
+    vr[k] = b0 + d0;
+    vi[k] = b1 + d1;
+    pair_end();
+  }
+}
+
+// zero diagonal: out0 = (ar, ai) v1, out1 = (br, bi) v0
+template <int Q, typename T>
+__device__ __forceinline__ void p_anti(Regs<T> &vr, Regs<T> &vi, T ar, T ai, T br, T bi) {
+#pragma unroll
+  for (int j = 0; j < kPAmps; ++j) {
+    if (j & (1 << Q)) continue;
+    const int k = j | (1 << Q);
+    const T x0 = vr[j], y0 = vi[j], x1 = vr[k], y1 = vi[k];
+    const T c0 = ar * x1, c1 = ai * y1, c2 = ar * y1, c3 = ai * x1;
+    const T b0 = br * x0, b1 = bi * y0, b2 = br * y0, b3 = bi * x0;
+    vr[j] = c0 - c1;
+    vi[j] = c2 + c3;
+    vr[k] = b0 - b1;
+    vi[k] = b2 + b3;
+    pair_end();
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void p_scale(T &vr, T &vi, T ar, T ai) {
+  const T a0 = ar * vr, a1 = ai * vi, a2 = ar * vi, a3 = ai * vr;
+  vr = a0 - a1;
+  vi = a2 + a3;
+}
+
+// the amplitudes whose register bits include those of SET, times (ar, ai)
+template <int SET, typename T>
+__device__ __forceinline__ void p_phase(Regs<T> &vr, Regs<T> &vi, T ar, T ai) {
+#pragma unroll
+  for (int j = 0; j < kPAmps; ++j) {
+    if ((j & SET) != SET) continue;
+    p_scale(vr[j], vi[j], ar, ai);
+    if (j & 1) pair_end();
+  }
+}
+
+template <int Q, typename T>
+__device__ __forceinline__ void p_diag(Regs<T> &vr, Regs<T> &vi, T ar, T ai, T br, T bi) {
+#pragma unroll
+  for (int j = 0; j < kPAmps; ++j) {
+    if (j & (1 << Q)) continue;
+    const int k = j | (1 << Q);
+    p_scale(vr[j], vi[j], ar, ai);
+    p_scale(vr[k], vi[k], br, bi);
+    pair_end();
+  }
+}
+
+// diag(ar + i ai, conj), [[c, s], [-s, c]], diag(br + i bi, conj), one after
+// the other: the products of the three gates, whose other entries are copies
+// and negations of these
+template <int Q, typename T>
+__device__ __forceinline__ void p_euler(Regs<T> &vr, Regs<T> &vi, T ar, T ai, T c, T s, T br,
+                                        T bi) {
+#pragma unroll
+  for (int j = 0; j < kPAmps; ++j) {
+    if (j & (1 << Q)) continue;
+    const int k = j | (1 << Q);
+    p_scale(vr[j], vi[j], ar, ai);
+    p_scale(vr[k], vi[k], ar, -ai);
+    const T x0 = vr[j], y0 = vi[j], x1 = vr[k], y1 = vi[k];
+    const T a0 = c * x0, a1 = c * y0, b0 = -s * x0, b1 = -s * y0;
+    const T c0 = s * x1, c1 = s * y1, d0 = c * x1, d1 = c * y1;
+    vr[j] = a0 + c0;
+    vi[j] = a1 + c1;
+    vr[k] = b0 + d0;
+    vi[k] = b1 + d1;
+    p_scale(vr[j], vi[j], br, bi);
+    p_scale(vr[k], vi[k], br, -bi);
+    pair_end();
+  }
+}
+
+// The program is read where the launch put it, by scalar loads: as a plain
+// by-value parameter indexed at run time it would be copied to scratch.
+#define QCS_KERNARG __attribute__((address_space(4)))
+typedef const QCS_KERNARG uint32_t *Words;
+typedef const QCS_KERNARG PassLayout *LayoutPtr;
+typedef const QCS_KERNARG PassProgram *ProgramPtr;
+
+// a program word's parameters: T values at a word boundary
+template <typename T>
+__device__ __forceinline__ T par(Words w, int i) {
+  if constexpr (sizeof(T) == 8)
+    return __builtin_bit_cast(T, uint64_t(w[2 * i]) | uint64_t(w[2 * i + 1]) << 32);
+  else
+    return __builtin_bit_cast(T, w[i]);
+}
+
+// XOR of the entries whose bit is set in x
+template <int N, typename V>
+__device__ __forceinline__ V xor_bits(uint32_t x, const QCS_KERNARG V *e) {
+  V r = 0;
+#pragma unroll
+  for (int b = 0; b < N; ++b) r ^= e[b] & (V(0) - V((x >> b) & 1));
+  return r;
+}
+
+// the same value, but not for the compiler: what is computed from it is not
+// kept in registers from an earlier use (here the thread-bit masks, which
+// cost 17 spilled registers across the ops)
+__device__ __forceinline__ uint32_t fresh(uint32_t x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// a where mask is all ones, b where it is 0: by bits, since a select between
+// a loaded value and another becomes a branch around the load
+__device__ __forceinline__ double blend(uint32_t mask, double a, double b) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+  const uint64_t m = uint64_t(mask) << 32 | mask;
+  return __builtin_bit_cast(double, (x & m) | (y & ~m));
+}
+__device__ __forceinline__ float blend(uint32_t mask, float a, float b) {
+  const uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+  return __builtin_bit_cast(float, (x & mask) | (y & ~mask));
+}
+
+template <int Q, typename T>
+__device__ __forceinline__ void p_op(int cls, Regs<T> &vr, Regs<T> &vi, Words w,
+                                     uint32_t on) {
+  switch (cls) {
+    case kPDense: {
+      const T m[8] = {par<T>(w, 0), par<T>(w, 1), par<T>(w, 2), par<T>(w, 3),
+                      par<T>(w, 4), par<T>(w, 5), par<T>(w, 6), par<T>(w, 7)};
+      p_dense<Q, T>(vr, vi, m);
+      break;
+    }
+    case kPReal:
+      p_real<Q, T>(vr, vi, par<T>(w, 0), par<T>(w, 1), par<T>(w, 2), par<T>(w, 3));
+      break;
+    case kPAnti:
+      p_anti<Q, T>(vr, vi, par<T>(w, 0), par<T>(w, 1), par<T>(w, 2), par<T>(w, 3));
+      break;
+    case kPDiag:
+      p_diag<Q, T>(vr, vi, par<T>(w, 0), par<T>(w, 1), par<T>(w, 2), par<T>(w, 3));
+      break;
+    case kPPhase:  // where the condition fails the factor is 1: x * 1 - y * 0 is x
+      p_phase<(1 << Q), T>(vr, vi, blend(on, par<T>(w, 0), T(1)), blend(on, par<T>(w, 1), T(0)));
+      break;
+    default:  // kPEuler
+      p_euler<Q, T>(vr, vi, par<T>(w, 0), par<T>(w, 1), par<T>(w, 2), par<T>(w, 3), par<T>(w, 4),
+                    par<T>(w, 5));
+      break;
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(1 << kPThrBits, 4) void k_gate_pass(
+    const PassProgram by_value, typename Amp<T>::type *a, uint64_t ntiles) {
+  typedef typename Amp<T>::type A;
+  extern __shared__ double lds_pass[];
+  // the first argument starts the kernel-argument segment
+  const ProgramPtr prog = (ProgramPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  const int tid = threadIdx.x;
+  const int tb = int(prog->tb);
+  // a tile of fewer than 1024 amplitudes still takes a whole wave, whose
+  // lanes past the tile compute on copies and store nothing
+  const bool in = tid < (1 << (tb - kPRegBits));
+  // amplitude index of the tile: its number with zeros at the tile's bits
+  uint64_t base = xcd_order(blockIdx.x, ntiles);
+  for (int p = 0; p < tb; ++p) base = insert0(base, int(prog->bits[p]));
+  T vr[kPAmps], vi[kPAmps];
+  {
+    const uint64_t i0 = base | xor_bits<kPThrBits>(uint32_t(tid), prog->load_t);
+    A v[kPAmps];
+    // (lanes past the tile read its first amplitudes: their masks are zero)
+#pragma unroll
+    for (int j = 0; j < kPAmps; ++j)
+      v[j] = ld_stream(a + (i0 | xor_bits<kPRegBits>(uint32_t(j), prog->load_r)));
+#pragma unroll
+    for (int j = 0; j < kPAmps; ++j) {
+      vr[j] = v[j].x;
+      vi[j] = v[j].y;
+    }
+  }
+  Words w = prog->words;
+  for (int l = 0;;) {
+    const LayoutPtr lay = (LayoutPtr)w;
+    w += kPLayoutWords;
+    const Words end = w + lay->opwords;
+    while (w < end) {
+      const uint32_t h = w[0];
+      const Words pw = w + 1;
+      w += h >> 24;
+      const int kind = int(h & 255), c1 = int((h >> 8) & 255), c2 = int((h >> 16) & 255);
+      uint32_t on = ~0u;  // all ones where the op's conditions hold
+      if (c1 != kPNoCond) {
+        // straight-line on purpose: a branch on a lane's value here would
+        // make the compiler treat the whole dispatch as divergent
+        const uint32_t b1 = c1 < 64 ? uint32_t(tid) >> c1 : uint32_t(base >> (c1 & 63));
+        const uint32_t b2 = c2 == kPNoCond ? 1u
+                            : c2 < 64      ? uint32_t(tid) >> c2
+                                           : uint32_t(base >> (c2 & 63));
+        on = 0u - (b1 & b2 & 1u);
+        // nothing to do for any lane of the wave
+        if (kind != kPSelect && __ballot(on != 0) == 0) continue;
+      }
+      if (kind < kPCPhase) {
+        switch (kind & 3) {
+          case 0: p_op<0, T>(kind & ~3, vr, vi, pw, on); break;
+          case 1: p_op<1, T>(kind & ~3, vr, vi, pw, on); break;
+          case 2: p_op<2, T>(kind & ~3, vr, vi, pw, on); break;
+          default: p_op<3, T>(kind & ~3, vr, vi, pw, on); break;
+        }
+        continue;
+      }
+      const T ar = par<T>(pw, 0), ai = par<T>(pw, 1);
+      switch (kind) {
+        case kPCPhase + 0: p_phase<3, T>(vr, vi, ar, ai); break;
+        case kPCPhase + 1: p_phase<5, T>(vr, vi, ar, ai); break;
+        case kPCPhase + 2: p_phase<9, T>(vr, vi, ar, ai); break;
+        case kPCPhase + 3: p_phase<6, T>(vr, vi, ar, ai); break;
+        case kPCPhase + 4: p_phase<10, T>(vr, vi, ar, ai); break;
+        case kPCPhase + 5: p_phase<12, T>(vr, vi, ar, ai); break;
+        case kPSelect:
+          p_phase<0, T>(vr, vi, blend(on, par<T>(pw, 2), ar), blend(on, par<T>(pw, 3), ai));
+          break;
+        default:  // kPScale: by 1 where a condition fails
+          p_phase<0, T>(vr, vi, blend(on, ar, T(1)), blend(on, ai, T(0)));
+      }
+    }
+    if (++l == int(prog->nlayouts)) break;
+    // exchange: written in this layout, through its index map, and read in
+    // the next one
+    const LayoutPtr nxt = (LayoutPtr)w;
+    const uint32_t tx = fresh(uint32_t(tid));
+    uint32_t ws = xor_bits<kPThrBits>(tx, lay->thr) >> 16;
+    const uint32_t rs = xor_bits<kPThrBits>(tx, nxt->thr) & 0xffffu;
+    for (uint32_t k = 0; k < lay->nterm; ++k) {
+      const uint32_t t = lay->term[k];
+      if ((base >> (t & 63)) & 1) ws ^= t >> 16;
+    }
+    auto wslot = [&](int j) { return ws ^ (xor_bits<kPRegBits>(uint32_t(j), lay->reg) >> 16); };
+    auto rslot = [&](int j) { return rs ^ (xor_bits<kPRegBits>(uint32_t(j), nxt->reg) & 0xffffu); };
+    __syncthreads();  // the reads of the exchange before
+    if constexpr (sizeof(T) == 8) {
+      if (in) {
+#pragma unroll
+        for (int j = 0; j < kPAmps; ++j) lds_pass[wslot(j)] = vr[j];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < kPAmps; ++j)
+        vr[j] = lds_pass[rslot(j)];
+      __syncthreads();
+      if (in) {
+#pragma unroll
+        for (int j = 0; j < kPAmps; ++j) lds_pass[wslot(j)] = vi[j];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < kPAmps; ++j)
+        vi[j] = lds_pass[rslot(j)];
+    } else {
+      float2 *L = reinterpret_cast<float2 *>(lds_pass);
+      if (in) {
+#pragma unroll
+        for (int j = 0; j < kPAmps; ++j) L[wslot(j)] = make_float2(vr[j], vi[j]);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < kPAmps; ++j) {
+        const float2 x = L[rslot(j)];
+        vr[j] = x.x;
+        vi[j] = x.y;
+      }
+    }
+  }
+  if (prog->nlayouts == 1) {
+    // no exchange has held the waves together, and the store's index map may
+    // hit amplitudes that another wave loads: every load first
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  }
+  if (!in) return;
+  uint64_t i0 = base ^ xor_bits<kPThrBits>(fresh(uint32_t(tid)), prog->store_t);
+  for (uint32_t k = 0; k < prog->store_nterm; ++k)
+    if ((base >> prog->store_q[k]) & 1) i0 ^= prog->store_term[k];
+#pragma unroll
+  for (int j = 0; j < kPAmps; ++j) {
+    A o;
+    o.x = vr[j];
+    o.y = vi[j];
+    st_stream(a + (i0 ^ xor_bits<kPRegBits>(uint32_t(j), prog->store_r)), o);
+  }
+}
+
+// ---- the queue of plain gates --------------------------------------------------
+
+// Tile of a pass over an n-qubit state.
+static int pass_tile_bits(int n) {
+  return std::min(n, kPMaxTile);
+}
+
+// Two-norm bounds (log2) under which no amplitude can overflow: beyond them
+// the products by exact zeros are no longer zeros and the gates run one by
+// one.
+static double bound_limit(const qcs_hip_state *s) {
+  return s->precision == QCS_HIP_C128 ? 900.0 : 100.0;
+}
+
+void bound_reset(qcs_hip_state *s, double log2_norm) { s->log2_bound = log2_norm; }
+
+void bound_normalized(qcs_hip_state *s) {
+  if (s->log2_bound < bound_limit(s)) s->log2_bound = 1.0;
+}
+
+// growth of the two-norm by a matrix of `count` complex entries: its
+// Frobenius norm
+void bound_matrix(qcs_hip_state *s, const double *m, long count) {
+  double f = 0.0;
+  for (long i = 0; i < 2 * count; ++i) f += m[i] * m[i];
+  f = 0.5 * std::log2(f);
+  s->log2_bound += f > 0.0 || f != f ? f : 0.0;
+}
+
+void bound_gate(qcs_hip_state *s, const double m[8]) {
+  const double a = m[0] * m[0] + m[1] * m[1] + m[4] * m[4] + m[5] * m[5];
+  const double b = m[2] * m[2] + m[3] * m[3] + m[6] * m[6] + m[7] * m[7];
+  const double re = m[0] * m[2] + m[1] * m[3] + m[4] * m[6] + m[5] * m[7];
+  const double im = m[0] * m[3] - m[1] * m[2] + m[4] * m[7] - m[5] * m[6];
+  const double e = 1e-9;
+  if (std::fabs(a - 1.0) < e && std::fabs(b - 1.0) < e && std::fabs(re) < e && std::fabs(im) < e)
+    s->log2_bound += 1e-8;
+  else
+    bound_matrix(s, m, 4);  // never less than before: a controlled gate keeps a half
+}
+
+static int launch_gate(qcs_hip_state *s, int kind, int target, int control, const double *m) {
+  if (kind == QCS_HIP_G_1Q) return launch_1q(s, target, m);
+  if (kind == QCS_HIP_G_CU) return launch_cu(s, control, target, m);
+  return launch_swap(s, target, control);
+}
+
+template <typename T>
+static int launch_pass(qcs_hip_state *s, const PassPick &pick,
+                       const std::vector<PassGroup> &groups, int tb) {
+  typedef typename Amp<T>::type A;
+  PassProgram prog;
+  write_pass<T>(s->queue, pick, groups, tb, &prog);
+  const uint64_t ntiles = s->size >> tb;
+  const int threads = std::max(64, 1 << (tb - kPRegBits));
+  const size_t lds = prog.nlayouts > 1 ? size_t(8) << tb : 0;
+  TimedLaunch tl;
+  timing_begin(s, QCS_HIP_K_FUSED, 2.0 * double(s->size) * sizeof(A),
+               6.0 * double(s->size) * double(pick.gates.size()), &tl);
+  hipLaunchKernelGGL(k_gate_pass<T>, dim3(unsigned(ntiles)), dim3(unsigned(threads)), lds,
+                     s->stream, prog, static_cast<A *>(s->vec), ntiles);
+  int rc = launch_check("k_gate_pass");
+  if (rc) return rc;
+  return timing_end(s, &tl);
+}
+
+// Launches passes from the head of the queue: all of it, or only those that
+// further gates would not change, while enough is left to plan the next.
+static int run_queue(qcs_hip_state *s, bool all) {
+  std::vector<PlanGate> &q = s->queue;
+  PassPick pick;
+  std::vector<PassGroup> groups;
+  int rc = 0;
+  const int tb = pass_tile_bits(s->n);
+  const int words = s->precision == QCS_HIP_C128 ? 2 : 1;
+  while (!q.empty() && (all || q.size() >= kQueueLow)) {
+    plan_pick(q, s->n, tb, kPassLowBits, words, 64, &pick, &groups);
+    if (!all && !pick.full && q.size() < kQueueMax) break;
+    double traffic = 0.0;
+    for (int i : pick.gates) traffic += plan_gate_traffic(q[size_t(i)]);
+    if (pick.gates.size() <= 1 || (s->n >= kPassBigState && traffic <= 2.0)) {
+      // the per-gate kernels move no more than the pass would
+      if (pick.gates.empty()) pick.gates.push_back(0);
+      for (int i : pick.gates) {
+        const PlanGate &g = q[size_t(i)];
+        const int kind = g.cls == kGSwap ? QCS_HIP_G_SWAP : g.c >= 0 ? QCS_HIP_G_CU : QCS_HIP_G_1Q;
+        if ((rc = launch_gate(s, kind, g.t, g.c, g.m))) break;
+      }
+    } else {
+      rc = s->precision == QCS_HIP_C128 ? launch_pass<double>(s, pick, groups, tb)
+                                        : launch_pass<float>(s, pick, groups, tb);
+    }
+    if (rc) {
+      q.clear();  // the state is no longer what the rest would act on
+      break;
+    }
+    size_t keep = 0, x = 0;
+    for (size_t i = 0; i < q.size(); ++i) {
+      if (x < pick.gates.size() && size_t(pick.gates[x]) == i) ++x;
+      else q[keep++] = q[i];
+    }
+    q.resize(keep);
+  }
+  s->queue_mark = q.size() + kQueueStep;
+  return rc;
+}
+
+// (the planner's vectors may throw; the queue is whole either way)
+int queue_flush(qcs_hip_state *s) try {
+  if (!s->queued) return 0;
+  std::lock_guard<std::mutex> lock(s->queue_mu);
+  return s->queue.empty() ? 0 : run_queue(s, true);
+} catch (const std::exception &) {
+  return fail(QCS_HIP_ENOMEM, "planning the queued gates: out of host memory");
+}
+
+int queue_gate(qcs_hip_state *s, int kind, int target, int control, const double *m) try {
+  if (!s->queued) return launch_gate(s, kind, target, control, m);
+  std::lock_guard<std::mutex> lock(s->queue_mu);
+  if (kind != QCS_HIP_G_SWAP) bound_gate(s, m);
+  const PlanGate g = plan_gate(kind, target, control, m);
+  if (g.cls == kGCuDense || !(s->log2_bound < bound_limit(s))) {
+    const int rc = s->queue.empty() ? 0 : run_queue(s, true);
+    return rc ? rc : launch_gate(s, kind, target, control, m);
+  }
+  s->queue.push_back(g);
+  return s->queue.size() >= s->queue_mark ? run_queue(s, false) : 0;
+} catch (const std::exception &) {
+  return fail(QCS_HIP_ENOMEM, "queueing a gate: out of host memory");
+}
+
+}  // namespace qcs

@@ -11,9 +11,11 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <vector>
 
 #include "../../include/qcs_hip.h"
+#include "gateplan.h"
 
 namespace qcs {
 
@@ -22,6 +24,14 @@ constexpr int kRedBlocks = 1024;  // fixed grid of the FP64 reductions
 constexpr int kRedSlots = 8;      // doubles per reduction partial
 constexpr long kChunk = 4096;     // amplitudes per sampling chunk
 constexpr int kMaxQubits = 34;
+// Queue of plain gates (gatepass.hip).  A state of up to 6 qubits fits one
+// amplitude per lane of a wave: its gates launch one by one.
+constexpr int kPassMinQubits = 7;
+constexpr int kPassLowBits = 4;      // tiles always hold these index bits (256-byte runs)
+constexpr int kPassBigState = 18;    // from here on launches cost less than traffic
+constexpr size_t kQueueLow = 96;     // gates kept back to plan the next pass
+constexpr size_t kQueueStep = 64;    // gates between looks at the queue
+constexpr size_t kQueueMax = 1024;   // the queue never grows beyond this
 
 struct TimedLaunch {
   hipEvent_t start;
@@ -77,6 +87,13 @@ struct qcs_hip_state {
   int tile_k4 = QCS_HIP_TILE_K4_GAUSS;     // form of k = 4 blocks in tile programs
   int tile_direct = 1;  // three-product tile programs: first block from HBM,
                         // last block to HBM, where the pass allows
+  // plain gates recorded but not launched yet (every entry point that reads
+  // or changes the state launches them first)
+  bool queued = false;  // gates of this state go through the queue
+  std::mutex queue_mu;  // qcs_hip_device_sync may come from another thread
+  std::vector<qcs::PlanGate> queue;
+  size_t queue_mark = qcs::kQueueLow;
+  double log2_bound = 0.0;  // bound of log2 of the amplitudes' two-norm
   // kernel timing
   int timing = 0;
   std::vector<qcs::TimedLaunch> pending_events;
@@ -120,6 +137,15 @@ int launch_1q(qcs_hip_state *s, int target, const double m[8]);
 int launch_cu(qcs_hip_state *s, int control, int target, const double m[8]);
 int launch_swap(qcs_hip_state *s, int a, int b);
 int launch_fill_basis(qcs_hip_state *s, void *buf, uint64_t basis, int one);
+// kernels in gatepass.hip: a plain gate is queued, and launched together
+// with others on its tile; queue_flush launches what is queued
+int queue_gate(qcs_hip_state *s, int kind, int target, int control, const double *m);
+int queue_flush(qcs_hip_state *s);
+// the bound of the state's two-norm that decides whether gates may be queued
+void bound_reset(qcs_hip_state *s, double log2_norm);
+void bound_normalized(qcs_hip_state *s);
+void bound_matrix(qcs_hip_state *s, const double *m, long count);
+void bound_gate(qcs_hip_state *s, const double m[8]);
 // gate classes of the plain kernels: diag(1, x) (only the bit-1 half
 // changes) and X (a pure exchange)
 bool is_phase1(const double m[8]);

@@ -1,0 +1,351 @@
+// Gate-pass plans run on the CPU.
+//
+// Random gate lists are planned pass by pass (gateplan.h), each pass's
+// program is interpreted the way k_gate_pass runs it -- threads, register
+// amplitudes, LDS slots, conditions, index maps -- and the state is compared,
+// value for value, with the same gates applied one after another by the
+// per-gate arithmetic.  Every LDS slot and every amplitude index is checked
+// for range, and every exchange and every pass for being a permutation.
+#include <cstdio>
+#include <cstdlib>
+
+#include "../../qcs_amd/csrc/gateplan.h"
+
+using namespace qcs;
+
+static uint64_t rng_state;
+static uint64_t rnd() {
+  uint64_t z = (rng_state += 0x9E3779B97F4A7C15ull);
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  return z ^ (z >> 31);
+}
+static double uni() { return double(rnd() >> 11) / 9007199254740992.0; }
+
+static void fail(const char *what) {
+  std::printf("FAIL: %s\n", what);
+  std::exit(1);
+}
+
+struct Gate {
+  int kind, t, c;
+  double m[8];
+};
+
+template <typename T>
+struct Vec {
+  std::vector<T> r, i;
+};
+
+template <typename T>
+static void cmul(T ar, T ai, T br, T bi, T &rr, T &ri) {
+  const T a = ar * br, b = ai * bi, c = ar * bi, d = ai * br;
+  rr = a - b;
+  ri = c + d;
+}
+
+template <typename T>
+static void apply(Vec<T> &v, int n, const Gate &g) {
+  const uint64_t N = uint64_t(1) << n, tb = uint64_t(1) << g.t;
+  T m[8];
+  for (int k = 0; k < 8; ++k) m[k] = T(g.m[k]);
+  for (uint64_t i0 = 0; i0 < N; ++i0) {
+    if (g.kind == QCS_HIP_G_SWAP) {
+      const uint64_t cb = uint64_t(1) << g.c;
+      if ((i0 & tb) && !(i0 & cb)) {
+        std::swap(v.r[i0], v.r[(i0 ^ tb) | cb]);
+        std::swap(v.i[i0], v.i[(i0 ^ tb) | cb]);
+      }
+      continue;
+    }
+    if (i0 & tb) continue;
+    if (g.kind == QCS_HIP_G_CU && !((i0 >> g.c) & 1)) continue;
+    const uint64_t i1 = i0 | tb;
+    T a, b, c, d, e, f, p, q;
+    cmul(m[0], m[1], v.r[i0], v.i[i0], a, b);
+    cmul(m[2], m[3], v.r[i1], v.i[i1], c, d);
+    cmul(m[4], m[5], v.r[i0], v.i[i0], e, f);
+    cmul(m[6], m[7], v.r[i1], v.i[i1], p, q);
+    v.r[i0] = a + c;
+    v.i[i0] = b + d;
+    v.r[i1] = e + p;
+    v.i[i1] = f + q;
+  }
+}
+
+template <typename V>
+static V xor_bits(uint32_t x, const V *e, int n) {
+  V r = 0;
+  for (int b = 0; b < n; ++b)
+    if ((x >> b) & 1) r ^= e[b];
+  return r;
+}
+
+template <typename T>
+static T par(const uint32_t *w, int i) {
+  T x;
+  std::memcpy(&x, reinterpret_cast<const char *>(w) + size_t(i) * sizeof(T), sizeof(T));
+  return x;
+}
+
+template <typename T>
+static void op1(int cls, T *vr, T *vi, int q, const uint32_t *w, bool on) {
+  for (int j = 0; j < kPAmps; ++j) {
+    if ((j >> q) & 1) continue;
+    const int k = j | (1 << q);
+    T x0 = vr[j], y0 = vi[j], x1 = vr[k], y1 = vi[k];
+    T p[8];
+    for (int z = 0; z < 8; ++z) p[z] = z < (cls == kPDense ? 8 : cls == kPEuler ? 6 : cls == kPPhase ? 2 : 4) ? par<T>(w, z) : T(0);
+    switch (cls) {
+      case kPDense: {
+        T a, b, c, d;
+        cmul(p[0], p[1], x0, y0, a, b);
+        cmul(p[2], p[3], x1, y1, c, d);
+        vr[j] = a + c;
+        vi[j] = b + d;
+        cmul(p[4], p[5], x0, y0, a, b);
+        cmul(p[6], p[7], x1, y1, c, d);
+        vr[k] = a + c;
+        vi[k] = b + d;
+        break;
+      }
+      case kPReal:
+        vr[j] = p[0] * x0 + p[1] * x1;
+        vi[j] = p[0] * y0 + p[1] * y1;
+        vr[k] = p[2] * x0 + p[3] * x1;
+        vi[k] = p[2] * y0 + p[3] * y1;
+        break;
+      case kPAnti:
+        cmul(p[0], p[1], x1, y1, vr[j], vi[j]);
+        cmul(p[2], p[3], x0, y0, vr[k], vi[k]);
+        break;
+      case kPDiag:
+        cmul(p[0], p[1], x0, y0, vr[j], vi[j]);
+        cmul(p[2], p[3], x1, y1, vr[k], vi[k]);
+        break;
+      case kPPhase:
+        cmul(on ? p[0] : T(1), on ? p[1] : T(0), x1, y1, vr[k], vi[k]);
+        break;
+      case kPEuler: {
+        cmul(p[0], p[1], x0, y0, x0, y0);
+        cmul(p[0], -p[1], x1, y1, x1, y1);
+        const T u0 = p[2] * x0 + p[3] * x1, v0 = p[2] * y0 + p[3] * y1;
+        const T u1 = -p[3] * x0 + p[2] * x1, v1 = -p[3] * y0 + p[2] * y1;
+        cmul(p[4], p[5], u0, v0, vr[j], vi[j]);
+        cmul(p[4], -p[5], u1, v1, vr[k], vi[k]);
+        break;
+      }
+      default: fail("unknown op");
+    }
+  }
+}
+
+// One pass over the state, as k_gate_pass runs it.
+template <typename T>
+static void run_pass(Vec<T> &v, int n, const PassProgram &pp) {
+  const int tb = int(pp.tb), nthr = 1 << (tb - kPRegBits);
+  const uint64_t N = uint64_t(1) << n, ntiles = N >> tb;
+  std::vector<char> touched(N, 0), stored(N, 0);
+  Vec<T> out = v;
+  for (uint64_t tile = 0; tile < ntiles; ++tile) {
+    uint64_t base = tile;
+    for (int p = 0; p < tb; ++p) {
+      const uint64_t lo = base & ((uint64_t(1) << pp.bits[p]) - 1);
+      base = ((base >> pp.bits[p]) << (pp.bits[p] + 1)) | lo;
+    }
+    std::vector<T> vr(size_t(nthr) * kPAmps), vi(vr.size());
+    for (int t = 0; t < nthr; ++t)
+      for (int j = 0; j < kPAmps; ++j) {
+        const uint64_t i = base | xor_bits<uint64_t>(uint32_t(t), pp.load_t, kPThrBits) |
+                           xor_bits<uint64_t>(uint32_t(j), pp.load_r, kPRegBits);
+        if (i >= N || touched[i]) fail("load index");
+        touched[i] = 1;
+        vr[size_t(t) * kPAmps + j] = v.r[i];
+        vi[size_t(t) * kPAmps + j] = v.i[i];
+      }
+    // whole lines: threads 0..7 on 8 consecutive amplitudes
+    for (int t = 0; t < 8; ++t)
+      if (xor_bits<uint64_t>(uint32_t(t), pp.load_t, kPThrBits) != uint64_t(t)) fail("load line");
+    const uint32_t *w = pp.words;
+    for (uint32_t l = 0;;) {
+      PassLayout lay, nxt;
+      std::memcpy(&lay, w, sizeof(lay));
+      w += kPLayoutWords;
+      const uint32_t *end = w + lay.opwords;
+      while (w < end) {
+        const uint32_t h = w[0];
+        const uint32_t *pw = w + 1;
+        w += h >> 24;
+        const int kind = int(h & 255), c1 = int((h >> 8) & 255), c2 = int((h >> 16) & 255);
+        if ((h >> 24) == 0 || w > end) fail("op length");
+        for (int t = 0; t < nthr; ++t) {
+          T *r = &vr[size_t(t) * kPAmps], *s = &vi[size_t(t) * kPAmps];
+          auto cond = [&](int c) {
+            if (c == kPNoCond) return true;
+            if (c >= 64 && c - 64 >= n) fail("condition");
+            if (c < 64 && c >= tb - kPRegBits) fail("condition");
+            return c < 64 ? ((t >> c) & 1) != 0 : ((base >> (c - 64)) & 1) != 0;
+          };
+          const bool on = cond(c1) && cond(c2);
+          if (kind < kPCPhase) {
+            op1<T>(kind & ~3, r, s, kind & 3, pw, on);
+            continue;
+          }
+          static const int sets[6] = {3, 5, 9, 6, 10, 12};
+          const int set = kind < kPScale ? sets[kind - kPCPhase] : 0;
+          T ar = par<T>(pw, 0), ai = par<T>(pw, 1);
+          if (kind == kPScale && !on) ar = T(1), ai = T(0);
+          if (kind == kPSelect && on) ar = par<T>(pw, 2), ai = par<T>(pw, 3);
+          if (kind > kPSelect) fail("unknown kind");
+          for (int j = 0; j < kPAmps; ++j)
+            if ((j & set) == set) cmul(ar, ai, r[j], s[j], r[j], s[j]);
+        }
+      }
+      if (++l == pp.nlayouts) break;
+      std::memcpy(&nxt, w, sizeof(nxt));
+      std::vector<T> lr(size_t(1) << tb), li(lr.size());
+      std::vector<char> full(lr.size(), 0);
+      for (int t = 0; t < nthr; ++t) {
+        uint32_t ws = xor_bits<uint32_t>(uint32_t(t), lay.thr, kPThrBits) >> 16;
+        for (uint32_t k = 0; k < lay.nterm; ++k)
+          if ((base >> (lay.term[k] & 63)) & 1) ws ^= lay.term[k] >> 16;
+        for (int j = 0; j < kPAmps; ++j) {
+          const uint32_t x = ws ^ (xor_bits<uint32_t>(uint32_t(j), lay.reg, kPRegBits) >> 16);
+          if (x >= full.size() || full[x]) fail("write slot");
+          full[x] = 1;
+          lr[x] = vr[size_t(t) * kPAmps + j];
+          li[x] = vi[size_t(t) * kPAmps + j];
+        }
+      }
+      for (int t = 0; t < nthr; ++t) {
+        const uint32_t rs = xor_bits<uint32_t>(uint32_t(t), nxt.thr, kPThrBits) & 0xffffu;
+        for (int j = 0; j < kPAmps; ++j) {
+          const uint32_t x = rs ^ (xor_bits<uint32_t>(uint32_t(j), nxt.reg, kPRegBits) & 0xffffu);
+          if (x >= full.size() || full[x] != 1) fail("read slot");
+          full[x] = 2;
+          vr[size_t(t) * kPAmps + j] = lr[x];
+          vi[size_t(t) * kPAmps + j] = li[x];
+        }
+      }
+    }
+    if (w - pp.words > kPWords) fail("program length");
+    uint64_t b2 = base;
+    for (uint32_t k = 0; k < pp.store_nterm; ++k)
+      if ((base >> pp.store_q[k]) & 1) b2 ^= pp.store_term[k];
+    for (int t = 0; t < nthr; ++t)
+      for (int j = 0; j < kPAmps; ++j) {
+        const uint64_t i = b2 ^ xor_bits<uint64_t>(uint32_t(t), pp.store_t, kPThrBits) ^
+                           xor_bits<uint64_t>(uint32_t(j), pp.store_r, kPRegBits);
+        if (i >= N || stored[i]) fail("store index");
+        stored[i] = 1;
+        out.r[i] = vr[size_t(t) * kPAmps + j];
+        out.i[i] = vi[size_t(t) * kPAmps + j];
+      }
+  }
+  for (uint64_t i = 0; i < N; ++i)
+    if (!touched[i] || !stored[i]) fail("an amplitude was left out");
+  v = out;
+}
+
+template <typename T>
+static int check(int n, int tb, int low, int count, int style) {
+  const uint64_t N = uint64_t(1) << n;
+  std::vector<Gate> gates;
+  std::vector<PlanGate> q;
+  for (int x = 0; x < count; ++x) {
+    Gate g;
+    std::memset(&g, 0, sizeof(g));
+    g.t = int(rnd() % uint64_t(n));
+    g.c = int(rnd() % uint64_t(n - 1));
+    if (g.c >= g.t) ++g.c;
+    const double a = 6.283185307179586 * uni(), c = std::cos(a / 2), s = std::sin(a / 2);
+    // style 0: every kind; 1: rotations and CNOTs; 2: H and controlled phases
+    int k = int(rnd() % 13);
+    if (style == 1) k = k < 8 ? 6 + k % 2 : 9;
+    if (style == 2) k = k < 3 ? 0 : k < 11 ? 10 : 11;
+    if (style == 1 && k == 7 && x + 3 <= count) {  // RZ RY RZ
+      for (int y = 0; y < 3; ++y) {
+        Gate z;
+        std::memset(&z, 0, sizeof(z));
+        const double b = 6.283185307179586 * uni(), cb = std::cos(b / 2), sb = std::sin(b / 2);
+        z.kind = QCS_HIP_G_1Q;
+        z.t = g.t;
+        const double rz[8] = {cb, -sb, 0, 0, 0, 0, cb, sb}, ry[8] = {cb, 0, -sb, 0, sb, 0, cb, 0};
+        std::memcpy(z.m, y == 1 ? ry : rz, sizeof(z.m));
+        gates.push_back(z);
+      }
+      x += 2;
+      continue;
+    }
+    const double r = 1.0 / std::sqrt(2.0);
+    const double mats[9][8] = {{r, 0, r, 0, r, 0, -r, 0}, {0, 0, 1, 0, 1, 0, 0, 0},
+                               {0, 0, 0, -1, 0, 1, 0, 0}, {1, 0, 0, 0, 0, 0, -1, 0},
+                               {1, 0, 0, 0, 0, 0, c, s},  {c, 0, 0, -s, 0, -s, c, 0},
+                               {c, 0, -s, 0, s, 0, c, 0}, {c, -s, 0, 0, 0, 0, c, s},
+                               {c, s, 0, 0, 0, 0, s, -c}};
+    g.kind = QCS_HIP_G_1Q;
+    if (k < 9) {
+      std::memcpy(g.m, mats[k], sizeof(g.m));
+    } else if (k == 11) {
+      g.kind = QCS_HIP_G_SWAP;
+    } else {
+      g.kind = QCS_HIP_G_CU;
+      std::memcpy(g.m, k == 9 ? mats[1] : k == 10 ? mats[4] : mats[3], sizeof(g.m));
+    }
+    if (g.kind == QCS_HIP_G_1Q && k == 5 && rnd() % 2) {  // a dense matrix
+      for (double &z : g.m) z = 0.5 * (uni() - 0.5);
+    }
+    gates.push_back(g);
+  }
+  Vec<T> a;
+  a.r.resize(N);
+  a.i.resize(N);
+  for (uint64_t i = 0; i < N; ++i) {
+    a.r[i] = T(uni() - 0.5);
+    a.i[i] = T(uni() - 0.5);
+  }
+  Vec<T> b = a;
+  for (const Gate &g : gates) apply(a, n, g);
+  for (const Gate &g : gates) q.push_back(plan_gate(g.kind, g.t, g.c, g.m));
+  int passes = 0;
+  PassPick pick;
+  std::vector<PassGroup> groups;
+  static PassProgram pp;
+  while (!q.empty()) {
+    plan_pick(q, n, tb, low, int(sizeof(T) / 4), 64, &pick, &groups);
+    if (pick.gates.empty()) fail("a pass without gates");
+    if (__builtin_popcountll(pick.bits) != tb) fail("tile bits");
+    write_pass<T>(q, pick, groups, tb, &pp);
+    run_pass<T>(b, n, pp);
+    std::vector<PlanGate> rest;
+    size_t x = 0;
+    for (size_t i = 0; i < q.size(); ++i) {
+      if (x < pick.gates.size() && size_t(pick.gates[x]) == i) ++x;
+      else rest.push_back(q[i]);
+    }
+    q.swap(rest);
+    ++passes;
+  }
+  for (uint64_t i = 0; i < N; ++i)
+    if (!(a.r[i] == b.r[i] && a.i[i] == b.i[i])) fail("amplitudes differ");
+  return passes;
+}
+
+int main() {
+  rng_state = 12345;
+  long total = 0;
+  for (int n = 7; n <= 15; ++n)
+    for (int style = 0; style < 3; ++style)
+      for (int rep = 0; rep < 3; ++rep) {
+        // the whole state in a tile, then tiles smaller than it
+        for (int tb = n < kPMaxTile ? n : kPMaxTile; tb >= 7 && tb >= n - 5; tb -= 2)
+          for (int low = 3; low <= 4; ++low) {
+            if (tb < n && tb < low + 4) continue;
+            const int count = 20 + int(rnd() % 200);
+            total += check<double>(n, tb, low, count, style);
+            total += check<float>(n, tb, low, count, style);
+          }
+      }
+  std::printf("ok %ld passes\n", total);
+  return 0;
+}
