@@ -152,6 +152,7 @@ static void free_state(qcs_hip_state *s) {
   if (s->chunk_inc) (void)hipFree(s->chunk_inc);
   if (s->u_dev) (void)hipFree(s->u_dev);
   if (s->idx_dev) (void)hipFree(s->idx_dev);
+  if (s->marg) (void)hipFree(s->marg);
   if (s->tpass_dev) (void)hipFree(s->tpass_dev);
   if (s->tblock_dev) (void)hipFree(s->tblock_dev);
   if (s->stream) (void)hipStreamDestroy(s->stream);

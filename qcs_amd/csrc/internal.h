@@ -72,6 +72,7 @@ struct qcs_hip_state {
   double *u_dev = nullptr;
   long *idx_dev = nullptr;
   size_t shots_cap = 0;
+  double *marg = nullptr;  // measurement weights (measure_seq), kept once made
   // tile-program buffers and tuning
   void *tpass_dev = nullptr;
   size_t tpass_cap = 0;
