@@ -3,16 +3,16 @@
 // A gate by itself reads and writes the state once (gates.hip: bound by HBM,
 // 5.8 TB/s in place).  A pass reads it once, runs the gates of gateplan.h's
 // program on it and writes it once, so the cost of a gate becomes its
-// arithmetic: a pass of the 28-qubit layered circuit (694 gates in 20 passes)
-// takes 2.16 ms, 4.0 TB/s, where each gate by itself took 1.2 ms; the circuit
-// went from 863 to 44.5 ms, the 28-qubit QFT (448 gates) from 270 to 24 ms.
+// arithmetic: a pass of the 28-qubit layered circuit (694 gates in 21 passes)
+// takes 1.82 ms, 4.7 TB/s, where each gate by itself took 1.2 ms; the circuit
+// went from 863 to 39.5 ms, the 28-qubit QFT (448 gates) from 270 to 24 ms.
 //
 // k_gate_pass.  One work-group per tile of 2^tb amplitudes; thread t holds 16
 // of them in registers, those that differ in the layout's four register
 // bits.  A layout change exchanges the tile through LDS, complex128 as two
-// planes (all real parts, then all imaginary parts), so a 13-bit tile takes
-// 64 KiB: two work-groups of 512 threads fit a CU, and one computes while
-// the other waits for HBM.  The arithmetic is that of gates.hip without the
+// planes (all real parts, then all imaginary parts), so a 12-bit tile takes
+// 32 KiB: four work-groups of 256 threads fit a CU (128 registers a thread),
+// and one computes while another waits for HBM.  The arithmetic is that of gates.hip without the
 // products by exact-zero entries, which add only signed zeros; the
 // amplitudes compare equal to the per-gate kernels' (bound_gate
 // keeps states whose amplitudes could overflow out).
@@ -161,13 +161,29 @@ typedef const QCS_KERNARG uint32_t *Words;
 typedef const QCS_KERNARG PassLayout *LayoutPtr;
 typedef const QCS_KERNARG PassProgram *ProgramPtr;
 
-// a program word's parameters: T values at a word boundary
+// An op's word and the 16 words behind it (its parameters, at most), in
+// scalar registers.  The next op's are loaded before this one runs, so the
+// two waits of a dispatch (the op word, then its parameters) are covered by
+// arithmetic (28 qubits, complex64: 1.10 -> 0.87 ms a pass; 16 qubits,
+// complex128: 21 -> 19 us).
+typedef uint32_t Par __attribute__((ext_vector_type(16), aligned(4)));
+struct Op {
+  uint32_t h;
+  Par p;
+};
+__device__ __forceinline__ Op load_op(Words w) {
+  return Op{w[0], *(const QCS_KERNARG Par *)(w + 1)};
+}
+
+// parameter i of an op
 template <typename T>
-__device__ __forceinline__ T par(Words w, int i) {
-  if constexpr (sizeof(T) == 8)
+__device__ __forceinline__ T par(const Par &w, int i) {
+  if constexpr (sizeof(T) == 8) {
     return __builtin_bit_cast(T, uint64_t(w[2 * i]) | uint64_t(w[2 * i + 1]) << 32);
-  else
-    return __builtin_bit_cast(T, w[i]);
+  } else {
+    const uint32_t x = w[i];  // (a bit cast of the element itself takes element 0)
+    return __builtin_bit_cast(T, x);
+  }
 }
 
 // XOR of the entries whose bit is set in x
@@ -200,7 +216,7 @@ __device__ __forceinline__ float blend(uint32_t mask, float a, float b) {
 }
 
 template <int Q, typename T>
-__device__ __forceinline__ void p_op(int cls, Regs<T> &vr, Regs<T> &vi, Words w,
+__device__ __forceinline__ void p_op(int cls, Regs<T> &vr, Regs<T> &vi, const Par &w,
                                      uint32_t on) {
   switch (cls) {
     case kPDense: {
@@ -262,10 +278,12 @@ __global__ __launch_bounds__(1 << kPThrBits, 4) void k_gate_pass(
     const LayoutPtr lay = (LayoutPtr)w;
     w += kPLayoutWords;
     const Words end = w + lay->opwords;
+    Op nxt_op = load_op(w);
     while (w < end) {
-      const uint32_t h = w[0];
-      const Words pw = w + 1;
+      const uint32_t h = nxt_op.h;
+      const Par pw = nxt_op.p;
       w += h >> 24;
+      nxt_op = load_op(w);
       const int kind = int(h & 255), c1 = int((h >> 8) & 255), c2 = int((h >> 16) & 255);
       uint32_t on = ~0u;  // all ones where the op's conditions hold
       if (c1 != kPNoCond) {
@@ -371,9 +389,15 @@ __global__ __launch_bounds__(1 << kPThrBits, 4) void k_gate_pass(
 
 // ---- the queue of plain gates --------------------------------------------------
 
-// Tile of a pass over an n-qubit state.
+// Tile of a pass over an n-qubit state.  A state of up to 13 qubits is one
+// tile, so a pass ends only where its program is full.  Larger states take
+// 12-bit tiles: 256 threads, four work-groups to a CU, which overlap their
+// HBM and arithmetic phases better than two of 512 (complex128 layered
+// circuit, all passes, 13 / 12 bits: 16 qubits 0.36 / 0.27 ms, 20 qubits
+// 0.54 / 0.48, 24 qubits 1.73 / 1.80, 28 qubits 24.5 / 21.8; 11 bits 0.30 at
+// 16 qubits, 25.7 at 28).
 static int pass_tile_bits(int n) {
-  return std::min(n, kPMaxTile);
+  return n <= kPMaxTile ? n : kPMaxTile - 1;
 }
 
 // Two-norm bounds (log2) under which no amplitude can overflow: beyond them

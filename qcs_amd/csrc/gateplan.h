@@ -33,7 +33,8 @@ constexpr int kPMaxTile = 13;              // tile bits: 512 threads x 16
 constexpr int kPThrBits = kPMaxTile - kPRegBits;
 constexpr int kPLineBits = 3;              // 8 amplitudes: a 128-byte line (complex128)
 constexpr int kPMaxTerms = 6;              // controls outside the tile per exchange
-constexpr int kPWords = 868;               // program words of a pass
+constexpr int kPWords = 848;               // program words of a pass
+constexpr int kPPad = 17;                  // words read past the last op
 
 // A gate as the planner sees it.  kGCuDense (a controlled matrix that is
 // neither X nor a phase; no qc_* gate makes one) is not planned: it runs by
@@ -87,7 +88,7 @@ struct PassProgram {
   uint32_t store_q[kPMaxTerms];
   uint32_t store_nterm;
   uint32_t bits[kPMaxTile];  // tile position -> index bit, ascending
-  uint32_t words[kPWords];
+  uint32_t words[kPWords + kPPad];
 };
 static_assert(sizeof(PassProgram) <= 4096 - 16, "a pass program travels as a kernel argument");
 
