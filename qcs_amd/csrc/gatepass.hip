@@ -111,9 +111,15 @@ template <int SET, typename T>
 __device__ __forceinline__ void p_phase(Regs<T> &vr, Regs<T> &vi, T ar, T ai) {
 #pragma unroll
   for (int j = 0; j < kPAmps; ++j) {
-    if ((j & SET) != SET) continue;
-    p_scale(vr[j], vi[j], ar, ai);
-    if (j & 1) pair_end();
+    if ((j & SET) == SET) {
+      p_scale(vr[j], vi[j], ar, ai);
+      if (j & 1) pair_end();
+    } else {
+      // tied to its register as if it changed: left alone, the amplitudes an
+      // op does not touch were copied at the join (42 moves beside 48
+      // arithmetic instructions)
+      asm volatile("" : "+v"(vr[j]), "+v"(vi[j]));
+    }
   }
 }
 
@@ -287,13 +293,14 @@ __global__ __launch_bounds__(1 << kPThrBits, 4) void k_gate_pass(
       const int kind = int(h & 255), c1 = int((h >> 8) & 255), c2 = int((h >> 16) & 255);
       uint32_t on = ~0u;  // all ones where the op's conditions hold
       if (c1 != kPNoCond) {
-        // straight-line on purpose: a branch on a lane's value here would
-        // make the compiler treat the whole dispatch as divergent
-        const uint32_t b1 = c1 < 64 ? uint32_t(tid) >> c1 : uint32_t(base >> (c1 & 63));
-        const uint32_t b2 = c2 == kPNoCond ? 1u
-                            : c2 < 64      ? uint32_t(tid) >> c2
-                                           : uint32_t(base >> (c2 & 63));
-        on = 0u - (b1 & b2 & 1u);
+        // branches on scalars only (a branch on a lane's value would make the
+        // compiler treat the whole dispatch as divergent)
+        if (c1 < 64) on = 0u - ((uint32_t(tid) >> c1) & 1u);
+        else on = 0u - uint32_t((base >> (c1 & 63)) & 1u);
+        if (c2 != kPNoCond) {
+          if (c2 < 64) on &= 0u - ((uint32_t(tid) >> c2) & 1u);
+          else on &= 0u - uint32_t((base >> (c2 & 63)) & 1u);
+        }
         // nothing to do for any lane of the wave
         if (kind != kPSelect && __ballot(on != 0) == 0) continue;
       }
