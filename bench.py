@@ -696,10 +696,11 @@ def bench_config5(args):
             "h_layer_ms": t_h * 1e3, "rounds": k, "rounds_ms": t_r * 1e3,
             "ms_per_round": t_r / k * 1e3,
             # the reference's round: a sum, then a read+write update (3*N*s);
-            # here the update also forms the next round's sum (2*N*s moved)
+            # here that is what all rounds together move (the sums follow by
+            # recurrence)
             "round_gbs": 3 * N * sb / (t_r / k) / 1e9,
-            "round_moved_gbs": 2 * N * sb / (t_r / k) / 1e9,
-            "round_moved_hbm_frac": 2 * N * sb / (t_r / k) / 1e9 / HBM_PEAK_GBS,
+            "moved_gbs": 3 * N * sb / t_r / 1e9,
+            "moved_hbm_frac": 3 * N * sb / t_r / 1e9 / HBM_PEAK_GBS,
             "marked": m, "p_marked": p, "p_marked_analytic": want,
             "abs_err": abs(p - want)}
     t = t_h + t_r

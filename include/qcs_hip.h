@@ -116,8 +116,9 @@ int qcs_hip_apply_swap(qcs_hip_state *s, int qubit_a, int qubit_b);
 int qcs_hip_phase_flip(qcs_hip_state *s, long index);
 int qcs_hip_diffusion(qcs_hip_state *s);
 /* `iterations` rounds of (phase_flip(marked); diffusion) on the device with
- * no host round trip (textbook: one fused read+write pass per round).  The
- * loop body of qc_grover_search (src/qcs.c:412-418). */
+ * no host round trip (textbook: one reduction, a recurrence for the rounds'
+ * sums, one update of the state, whatever the number of rounds).  The loop
+ * body of qc_grover_search (src/qcs.c:412-418). */
 int qcs_hip_grover(qcs_hip_state *s, long marked, long iterations);
 
 /* ---- reductions and observation (FP64 on the device) -------------------
