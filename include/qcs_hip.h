@@ -298,7 +298,10 @@ int qcs_hip_apply_passes_normalize(qcs_hip_state *s, const qcs_hip_pass *passes,
 #define QCS_HIP_BLOCK_TB12_256_PIPE 1 /* same, next tile's loads pipelined */
 #define QCS_HIP_BLOCK_TB13_256_PIPE 2 /* 8192-amplitude tiles, 256 threads */
 #define QCS_HIP_BLOCK_TB13_512_PIPE 3 /* 8192-amplitude tiles, 512 threads
-                                         (default) */
+                                         (default); states of up to 24
+                                         qubits, which such tiles do not
+                                         fill the device with, run smaller
+                                         work-groups under this value */
 int qcs_hip_set_tuning(qcs_hip_state *s, int knob, int value);
 /* the current value of a knob (what the autotuner chose, or the default) */
 int qcs_hip_get_tuning(qcs_hip_state *s, int knob, int *value);

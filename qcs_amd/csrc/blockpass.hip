@@ -14,10 +14,11 @@
 // complex row s and each 32-row accumulator block holds whole complex
 // outputs.
 //
-// Launch variants (chosen per block by the autotuner, see qcs_hip_set_tuning):
-//   TB 12 / 256 threads, or TB 13 / 256 or 512 threads; with or without
-//   software pipelining (the next tile's loads issued before the current
-//   tile's MFMA work).  All use non-temporal global accesses and, when the
+// Launch variants (chosen per block by the autotuner, see qcs_hip_set_tuning,
+// and by the state's size, block_variant_for): TB 12 / 256 threads, or TB 13 /
+// 256 or 512 threads; with or without software pipelining (the next tile's
+// loads issued before the current tile's MFMA work); TB 10 on one wave for
+// small states.  All use non-temporal global accesses and, when the
 //   state has >= 8 tiles, an XCD-aware tile order (work-group i runs on XCD
 //   i % 8, so XCD x takes the contiguous x-th eighth of the tiles).
 #include "device.h"
@@ -224,6 +225,10 @@ static void launch_k(qcs_hip_state *s, const float *W, const BlockGeom &g,
                      ntiles);
 }
 
+// one-wave tiles, for states too small to fill the chip with larger ones; not
+// among the variants a caller can name
+constexpr int kBlockTb10_64 = 16;
+
 template <int K>
 static void launch_variant(qcs_hip_state *s, const float *W, const int *targets,
                            int variant) {
@@ -237,17 +242,27 @@ static void launch_variant(qcs_hip_state *s, const float *W, const int *targets,
     case QCS_HIP_BLOCK_TB13_256_PIPE:
       launch_k<K, 13, 256, true>(s, W, make_geom(s->n, K, targets, 13), 512);
       break;
+    case kBlockTb10_64:
+      launch_k<K, 10, 64, false>(s, W, make_geom(s->n, K, targets, 10), 4096);
+      break;
     default:
       launch_k<K, 13, 512, true>(s, W, make_geom(s->n, K, targets, 13), 512);
       break;
   }
 }
 
-// variant usable for this state size (13-bit tiles need n >= 13)
+// The variant a state of this size runs.  13-bit tiles on 512 threads need
+// many tiles to fill 256 CUs, and pay their barriers and operand loads for
+// them: whole flushes of the layered circuit, one-wave 10-bit tiles / 13-bit
+// tiles on 256 / on 512 threads: 18 qubits 286 / 499 / 659 us, 20 qubits
+// 521 / 607 / 788, 21 qubits 832 / 722 / 930, 23 qubits 1280 / 1163 / 1392,
+// 26 qubits 5407 / 5258 / 5045, 28 qubits 18.3 / 17.1 / 16.1 ms.  (10 and 11
+// qubits ran k_fused_valu: 10 qubits 358 us.)
 int block_variant_for(const qcs_hip_state *s, int variant) {
-  if (s->n < 13 && (variant == QCS_HIP_BLOCK_TB13_256_PIPE ||
-                    variant == QCS_HIP_BLOCK_TB13_512_PIPE))
-    return QCS_HIP_BLOCK_TB12_256_PIPE;
+  if (s->n < 12) return kBlockTb10_64;
+  if (variant == QCS_HIP_BLOCK_TB13_512_PIPE && s->n < 25)
+    variant = s->n < 21 ? kBlockTb10_64 : QCS_HIP_BLOCK_TB13_256_PIPE;
+  if (variant == QCS_HIP_BLOCK_TB13_256_PIPE && s->n < 13) return QCS_HIP_BLOCK_TB12_256_PIPE;
   return variant;
 }
 

@@ -10,7 +10,7 @@
 //        followed, for k <= 4, by the 2^k x 2^k planes Ur + Ui and Ur - Ui,
 //      - U itself in FP64 for the VALU kernel.
 // 2. Each block is then applied in one HBM pass: complex64 states with
-//    n >= 12 by the matrix-core kernel of blockpass.hip (k_fused_mfma),
+//    n >= 10 by the matrix-core kernel of blockpass.hip (k_fused_mfma),
 //    other states by k_fused_valu below.  Tile programs (tiles.hip) apply
 //    several composed blocks per pass instead.
 #include <cstring>
@@ -25,64 +25,87 @@ constexpr int kUDoubles = 32 * 32 * 2;      // U slot per block (k = 5)
 
 // ---- composition (FP64) -------------------------------------------------------
 
-__global__ __launch_bounds__(64) void k_compose(const qcs_hip_gate *gates,
-                                                const qcs_hip_block *blocks,
-                                                float *wbuf, double *ubuf) {
+// Thread (j, p): column j of U, the p-th eighth of a gate's row pairs.  Gates
+// are staged in LDS with their positions in the block worked out, so a gate
+// costs two LDS round trips and a barrier.  (One thread per column, reading
+// each gate from memory in turn, took 7 us a gate: 184 us for the 18-qubit
+// depth-10 circuit, now 33 us.)
+constexpr int kComposeThreads = 256;
+__global__ __launch_bounds__(kComposeThreads) void k_compose(const qcs_hip_gate *gates,
+                                                             const qcs_hip_block *blocks,
+                                                             float *wbuf, double *ubuf) {
+  constexpr int kStage = 64;  // gates staged at a time
   __shared__ double cr[32][33];
   __shared__ double ci[32][33];
-  const qcs_hip_block blk = blocks[blockIdx.x];
-  const int k = blk.k, R = 1 << k;
-  const int j = threadIdx.x;  // column of U owned by this thread
-  if (j < R)
-    for (int i = 0; i < R; ++i) {
-      cr[j][i] = (i == j) ? 1.0 : 0.0;
-      ci[j][i] = 0.0;
+  __shared__ double sm[kStage][8];
+  __shared__ int sbit[kStage], scond[kStage], sswap[kStage];
+  const qcs_hip_block &blk = blocks[blockIdx.x];
+  const int k = blk.k, R = 1 << k, ng = blk.num_gates;
+  const qcs_hip_gate *src = gates + blk.first_gate;
+  const int j = threadIdx.x & 31, part = threadIdx.x >> 5;
+  for (int i = part; i < R; i += kComposeThreads / 32) {
+    cr[j][i] = (i == j) ? 1.0 : 0.0;
+    ci[j][i] = 0.0;
+  }
+  for (int g0 = 0; g0 < ng; g0 += kStage) {
+    const int c = min(kStage, ng - g0);
+    __syncthreads();
+    for (int w = threadIdx.x; w < c * 8; w += kComposeThreads)
+      sm[w >> 3][w & 7] = src[g0 + (w >> 3)].m[w & 7];
+    if (int(threadIdx.x) < c) {
+      const qcs_hip_gate &gt = src[g0 + threadIdx.x];
+      const int kind = gt.kind, target = gt.target, control = gt.control;
+      int lt = -1, lc = -1;
+      for (int q = 0; q < k; ++q) {
+        const int b = blk.targets[q];
+        if (b == target) lt = q;
+        if (b == control) lc = q;
+      }
+      const bool swap = kind == QCS_HIP_G_SWAP;
+      // (a gate outside its block is refused on the host)
+      sbit[threadIdx.x] = lt < 0 || (swap && lc < 0) ? -1 : lt;
+      scond[threadIdx.x] = (swap || kind == QCS_HIP_G_CU) && lc >= 0 ? 1 << lc : 0;
+      sswap[threadIdx.x] = swap;
     }
-  for (int g = blk.first_gate; g < blk.first_gate + blk.num_gates; ++g) {
-    const qcs_hip_gate gt = gates[g];
-    int lt = -1, lc = -1;
-    for (int q = 0; q < k; ++q) {
-      if (blk.targets[q] == gt.target) lt = q;
-      if (blk.targets[q] == gt.control) lc = q;
-    }
-    if (j >= R || lt < 0) continue;
-    const int tb = 1 << lt;
-    if (gt.kind == QCS_HIP_G_SWAP) {
-      if (lc < 0) continue;
-      const int cb = 1 << lc;
-      for (int i = 0; i < R; ++i) {
-        if ((i & tb) && !(i & cb)) {
-          const int o = i ^ tb ^ cb;
-          const double xr = cr[j][i], xi = ci[j][i];
-          cr[j][i] = cr[j][o];
-          ci[j][i] = ci[j][o];
-          cr[j][o] = xr;
-          ci[j][o] = xi;
+    __syncthreads();
+    for (int g = 0; g < c; ++g) {
+      const int lt = sbit[g], cb = scond[g];
+      if (lt >= 0 && j < R) {
+        const int tb = 1 << lt;
+        for (int p = part; p < R / 2; p += kComposeThreads / 32) {
+          const int i0 = ((p >> lt) << (lt + 1)) | (p & (tb - 1));
+          const int i1 = i0 | tb;
+          if (sswap[g]) {  // rows with (t, c) = (1, 0) and (0, 1)
+            if (i1 & cb) continue;
+            const int o = i0 | cb;
+            const double xr = cr[j][i1], xi = ci[j][i1];
+            cr[j][i1] = cr[j][o];
+            ci[j][i1] = ci[j][o];
+            cr[j][o] = xr;
+            ci[j][o] = xi;
+            continue;
+          }
+          if ((i0 & cb) != cb) continue;
+          const double *m = sm[g];
+          const double v0r = cr[j][i0], v0i = ci[j][i0];
+          const double v1r = cr[j][i1], v1i = ci[j][i1];
+          double o0r, o0i, o1r, o1i;
+          row2(m[0], m[1], m[2], m[3], v0r, v0i, v1r, v1i, o0r, o0i);
+          row2(m[4], m[5], m[6], m[7], v0r, v0i, v1r, v1i, o1r, o1i);
+          cr[j][i0] = o0r;
+          ci[j][i0] = o0i;
+          cr[j][i1] = o1r;
+          ci[j][i1] = o1i;
         }
       }
-      continue;
-    }
-    const int cb = (gt.kind == QCS_HIP_G_CU && lc >= 0) ? (1 << lc) : 0;
-    const double *m = gt.m;
-    for (int i0 = 0; i0 < R; ++i0) {
-      if ((i0 & tb) || ((i0 & cb) != cb)) continue;
-      const int i1 = i0 | tb;
-      const double v0r = cr[j][i0], v0i = ci[j][i0];
-      const double v1r = cr[j][i1], v1i = ci[j][i1];
-      double o0r, o0i, o1r, o1i;
-      row2(m[0], m[1], m[2], m[3], v0r, v0i, v1r, v1i, o0r, o0i);
-      row2(m[4], m[5], m[6], m[7], v0r, v0i, v1r, v1i, o1r, o1i);
-      cr[j][i0] = o0r;
-      ci[j][i0] = o0i;
-      cr[j][i1] = o1r;
-      ci[j][i1] = o1i;
+      __syncthreads();
     }
   }
-  __syncthreads();
+  if (ng == 0) __syncthreads();
   const int RR = 2 * R;
   float *W = wbuf + size_t(blockIdx.x) * kWFloats;
-  for (int idx = threadIdx.x; idx < RR * RR; idx += 64) {
-    const int row = idx / RR, col = idx % RR;
+  for (int idx = threadIdx.x; idx < RR * RR; idx += kComposeThreads) {
+    const int row = idx >> (k + 1), col = idx & (RR - 1);
     const int i = row >> 1, p = row & 1, jj = col >> 1, q = col & 1;
     const double ur = cr[jj][i], ui = ci[jj][i];
     const double v = (p == q) ? ur : (p == 0 ? -ui : ui);
@@ -92,15 +115,15 @@ __global__ __launch_bounds__(64) void k_compose(const qcs_hip_gate *gates,
   // once, after the real form (the three-product form of tile programs
   // reads them)
   if (RR * RR + 2 * R * R <= kWFloats)
-    for (int idx = threadIdx.x; idx < R * R; idx += 64) {
-      const double ur = cr[idx % R][idx / R], ui = ci[idx % R][idx / R];
+    for (int idx = threadIdx.x; idx < R * R; idx += kComposeThreads) {
+      const double ur = cr[idx & (R - 1)][idx >> k], ui = ci[idx & (R - 1)][idx >> k];
       W[RR * RR + idx] = float(ur + ui);
       W[RR * RR + R * R + idx] = float(ur - ui);
     }
   if (!ubuf) return;
   double *U = ubuf + size_t(blockIdx.x) * kUDoubles;
-  for (int idx = threadIdx.x; idx < R * R; idx += 64) {
-    const int i = idx / R, jj = idx % R;
+  for (int idx = threadIdx.x; idx < R * R; idx += kComposeThreads) {
+    const int i = idx >> k, jj = idx & (R - 1);
     U[2 * idx] = cr[jj][i];
     U[2 * idx + 1] = ci[jj][i];
   }
@@ -196,7 +219,7 @@ static int apply_block(qcs_hip_state *s, int k, const int *targets,
   TimedLaunch tl;
   int rc;
   timing_begin(s, QCS_HIP_K_FUSED, bytes, flops, &tl);
-  if (s->precision == QCS_HIP_C64 && s->n >= 12) {
+  if (s->precision == QCS_HIP_C64 && s->n >= 10) {
     if ((rc = launch_block_mfma(s, k, targets, W, s->block_variant[k]))) return rc;
   } else {
     if (s->precision == QCS_HIP_C128) launch_valu<double>(s, k, U, targets);
@@ -245,7 +268,7 @@ int compose_blocks(qcs_hip_state *s, const qcs_hip_block *blocks, int nb,
                              hipMemcpyHostToDevice, s->stream));
   TimedLaunch tl;
   timing_begin(s, QCS_HIP_K_COMPOSE, 0.0, 0.0, &tl);
-  hipLaunchKernelGGL(k_compose, dim3(nb), dim3(64), 0, s->stream,
+  hipLaunchKernelGGL(k_compose, dim3(nb), dim3(kComposeThreads), 0, s->stream,
                      static_cast<const qcs_hip_gate *>(s->gates_dev),
                      static_cast<const qcs_hip_block *>(s->blocks_dev), s->wbuf,
                      s->ubuf);
@@ -257,7 +280,7 @@ int launch_compose(hipStream_t stream, const qcs_hip_gate *gates,
                    const qcs_hip_block *blocks, int nb, float *wbuf,
                    double *ubuf) {
   if (nb <= 0) return 0;
-  hipLaunchKernelGGL(k_compose, dim3(nb), dim3(64), 0, stream, gates, blocks,
+  hipLaunchKernelGGL(k_compose, dim3(nb), dim3(kComposeThreads), 0, stream, gates, blocks,
                      wbuf, ubuf);
   return launch_check("k_compose");
 }
