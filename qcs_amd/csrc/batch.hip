@@ -93,7 +93,7 @@ struct BCirc {
 constexpr uint64_t kNoSlot = ~uint64_t(0);
 
 // One queue item: a circuit, or one of the `nparts` parts of a streamed
-// complex128 circuit that several work-groups share (part j takes tiles
+// circuit that several work-groups share (part j takes tiles
 // j, j + nparts, ... of every pass; the parts meet between passes).
 struct BItem {
   int circ;
@@ -102,8 +102,8 @@ struct BItem {
   int reserved;
 };
 // spins of a part's wait at a pass boundary before it gives up (each spin
-// sleeps ~1000 clocks: several seconds, far beyond any pass)
-constexpr unsigned kPartSpinLimit = 1u << 23;
+// sleeps ~250 clocks: several seconds, far beyond any pass)
+constexpr unsigned kPartSpinLimit = 1u << 25;
 
 struct BPass {
   int first_op;
@@ -800,10 +800,14 @@ __device__ void sample_state(const P &prob, int n, double *tot, double *inc,
 // is set and every wave of the work-group returns false.
 __device__ bool parts_barrier(unsigned *cnt, unsigned target, unsigned *err) {
   __shared__ int ok_s;
-  __threadfence();
+  // every wave's stores have reached its L2; one fence then writes that back
+  // for all of them (18 qubits, depth 40 in 32 parts: 2.86 ms, with a fence
+  // per wave 3.05)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0) {
     int ok = 1;
+    __threadfence();
     atomicAdd(cnt, 1u);
     for (unsigned spins = 0;
          __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target;) {
@@ -813,7 +817,7 @@ __device__ bool parts_barrier(unsigned *cnt, unsigned target, unsigned *err) {
         ok = 0;
         break;
       }
-      __builtin_amdgcn_s_sleep(16);
+      __builtin_amdgcn_s_sleep(4);
     }
     __threadfence();
     ok_s = ok;
@@ -894,7 +898,8 @@ __device__ void run_c128(const BCirc c, int part, int nparts, unsigned *sync,
 }
 
 template <int NTH>
-__device__ void run_c64(const BCirc c, const BPass *__restrict__ passes,
+__device__ void run_c64(const BCirc c, int part, int nparts, unsigned *sync, unsigned *err,
+                        const BPass *__restrict__ passes,
                         const BBlock *__restrict__ blocks,
                         const float *__restrict__ wbuf, char *states, char *lds,
                         double *tot, double *inc, double *red,
@@ -911,10 +916,14 @@ __device__ void run_c64(const BCirc c, const BPass *__restrict__ passes,
   for (int p = 0; p < c.npass; ++p) {
     const BPass &ps = passes[c.first_pass + p];
     const TileBits tbits = load_tile_bits(ps.sbits);
+    // a pass reads tiles the previous pass wrote, possibly in another part
+    if (nparts > 1 && p > 0 && !parts_barrier(sync, unsigned(p) * unsigned(nparts), err))
+      return;
     const uint64_t outside = outside_mask(tbits, tb, n);
-    const uint64_t bstep = outside & (~outside + 1);  // tile 1
-    uint64_t base = 0;
-    for (uint64_t t = 0; t < ntiles; ++t, base = masked_add(base, bstep, outside)) {
+    const uint64_t bstep = tile_base(uint64_t(nparts), tbits, tb);
+    uint64_t base = tile_base(uint64_t(part), tbits, tb);
+    for (uint64_t t = uint64_t(part); t < ntiles;
+         t += uint64_t(nparts), base = masked_add(base, bstep, outside)) {
       if (p == 0 || resident) {
         if (p == 0)
           for (int e = tid; e < tile; e += NTH)
@@ -932,10 +941,14 @@ __device__ void run_c64(const BCirc c, const BPass *__restrict__ passes,
       if (!resident) {
         tile_io_c64<NTH, false>(lds, G, base, tbits, tb);
         // as in run_c128: within a pass each thread reloads its own slots
-        if (p == 0 || t + 1 >= ntiles) __syncthreads();
+        if (p == 0 || t + uint64_t(nparts) >= ntiles) __syncthreads();
       }
     }
   }
+  // the last pass done by every part; part 0 renormalises and samples (the
+  // norm's sum keeps its order whatever the number of parts)
+  if (nparts > 1 && !parts_barrier(sync, unsigned(c.npass) * unsigned(nparts), err)) return;
+  if (part != 0) return;
   // FP64 renormalisation, q_state_normalize's rule (src/q_utils.c:112-118)
   const uint64_t N = uint64_t(1) << n;
   double ns = 0.0;
@@ -1010,7 +1023,7 @@ __global__ __launch_bounds__(NTH) void k_batch(
       run_c128<NTH>(c, it.part, it.nparts, sync + it.circ, queue + 1, passes, gates,
                     groups, states, lds, tot, inc, red, u, out, shots, keep);
     else
-      run_c64<NTH>(c, passes, blocks, wbuf, states, lds, tot, inc, red, u,
+      run_c64<NTH>(c, it.part, it.nparts, sync + it.circ, queue + 1, passes, blocks, wbuf, states, lds, tot, inc, red, u,
                    out, shots, keep);
   }
 }
@@ -1690,7 +1703,11 @@ int batch_run(qcs_hip_batch *b, const qcs_hip_batch_circuit *cs, int nc,
         ops += resident ? 0.0 : 2.0;
       }
     }
-    cost[i] = double(amp) * double(uint64_t(1) << c.num_qubits) * (ops + 1.0);
+    // (a unit of complex64 work takes 2.8 times a unit of complex128 work:
+    // measured per layer at 20 qubits, 2.71 against 5.52 ms for 240 against
+    // 1392 units an amplitude)
+    cost[i] = (c.precision == QCS_HIP_C128 ? 16.0 : 8.0 * 2.8) *
+              double(uint64_t(1) << c.num_qubits) * (ops + 1.0);
   }
   const int nch_cap = int(std::max<uint64_t>(
       1, (uint64_t(1) << max_n) / std::min<uint64_t>(uint64_t(1) << max_n, kChunk)));
@@ -1700,40 +1717,47 @@ int batch_run(qcs_hip_batch *b, const qcs_hip_batch_circuit *cs, int nc,
   int per_cu = 0;
   if ((rc = batch_occupancy(b->nth, lds_bytes, &per_cu))) return rc;
   if (per_cu < 1) return fail(QCS_HIP_EDEVICE, "batch kernel does not fit on a CU");
-  const int grid = std::min(nc, per_cu * b->num_cus);
-  // A streamed complex128 circuit that costs several times a work-group's
-  // share of the batch is shared by that many work-groups (at most 32, its
-  // tile count, and half the grid), so no single circuit sets the launch
-  // time.  QCS_BATCH_MAX_PARTS lowers the cap (1: no sharing).
+  const int resident = per_cu * b->num_cus;
+  // A streamed circuit that costs more than half a work-group's share of the
+  // batch is shared by several work-groups: a power of two of them (so that
+  // the parts take equally many tiles), at most 32, its tile count, and half
+  // the work-groups, so no single circuit sets the launch time.  256 circuits
+  // of 10-18 qubits, kernel: complex128 circuits alone shared, 34.9 ms; every
+  // streamed one, parts up to a whole share 11.2, half a share 7.9, a quarter
+  // 8.5 (each boundary of a pass costs the parts about 15 us).
+  // QCS_BATCH_MAX_PARTS lowers the cap (1: no sharing).
   std::vector<int> shares(size_t(nc), 1);
   {
     int cap = 32;
     if (const char *e = std::getenv("QCS_BATCH_MAX_PARTS")) cap = std::max(1, std::atoi(e));
-    cap = std::min(cap, std::max(1, grid / 2));
+    cap = std::min(cap, std::max(1, resident / 2));
     double total = 0.0;
     for (int i = 0; i < nc; ++i) total += cost[size_t(i)];
-    const double share = total / double(std::max(grid, 1));
+    const double part = 0.5 * total / double(std::max(resident, 1));
     for (int i = 0; i < nc; ++i) {
       const qcs_hip_batch_circuit &c = cs[i];
-      if (c.precision != QCS_HIP_C128 || c.tile_bits >= c.num_qubits) continue;
-      const uint64_t ntiles = uint64_t(1) << (c.num_qubits - c.tile_bits);
-      const int w = int(std::min<double>({cost[size_t(i)] / share, double(cap), double(ntiles)}));
-      if (w >= 2) shares[size_t(i)] = w;
+      if (c.tile_bits >= c.num_qubits) continue;
+      const double most = std::min(double(cap), double(uint64_t(1) << (c.num_qubits - c.tile_bits)));
+      int w = 1;
+      while (2 * w <= most && 1.5 * w * part <= cost[size_t(i)]) w *= 2;
+      shares[size_t(i)] = w;
     }
   }
-  // queue items: circuits by cost, largest first; the parts of a shared
-  // circuit are consecutive
+  // queue items, the longest parts first; the parts of a shared circuit are
+  // consecutive
   std::vector<BItem> items;
   {
     std::vector<int> idx(static_cast<size_t>(nc));
     for (int i = 0; i < nc; ++i) idx[size_t(i)] = i;
+    auto part_cost = [&](int i) { return cost[size_t(i)] / double(shares[size_t(i)]); };
     std::stable_sort(idx.begin(), idx.end(),
-                     [&](int a, int c) { return cost[size_t(a)] > cost[size_t(c)]; });
+                     [&](int a, int c) { return part_cost(a) > part_cost(c); });
     items.reserve(size_t(nc));
     for (int i : idx)
       for (int j = 0; j < shares[size_t(i)]; ++j) items.push_back(BItem{i, j, shares[size_t(i)], 0});
   }
   const int nitems = int(items.size());
+  const int grid = std::min(nitems, resident);
 
   // layout of the descriptor block (device and pinned staging alike)
   BatchLayout L;
