@@ -798,7 +798,7 @@ __device__ void sample_state(const P &prob, int n, double *tot, double *inc,
 // counter; thread 0 then waits for `target` arrivals and acquires.  The wait
 // is bounded: on timeout, or when another part has timed out, the error flag
 // is set and every wave of the work-group returns false.
-__device__ bool parts_barrier(unsigned *cnt, unsigned target, unsigned *err) {
+__device__ bool parts_barrier(unsigned *cnt, unsigned target, unsigned *err, unsigned limit) {
   __shared__ int ok_s;
   // every wave's stores have reached its L2; one fence then writes that back
   // for all of them (18 qubits, depth 40 in 32 parts: 2.86 ms, with a fence
@@ -812,7 +812,7 @@ __device__ bool parts_barrier(unsigned *cnt, unsigned target, unsigned *err) {
     for (unsigned spins = 0;
          __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target;) {
       if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u ||
-          ++spins > kPartSpinLimit) {
+          ++spins > limit) {
         atomicOr(err, 1u);
         ok = 0;
         break;
@@ -828,7 +828,7 @@ __device__ bool parts_barrier(unsigned *cnt, unsigned target, unsigned *err) {
 
 template <int NTH>
 __device__ void run_c128(const BCirc c, int part, int nparts, unsigned *sync,
-                         unsigned *err, const BPass *__restrict__ passes,
+                         unsigned *err, unsigned limit, const BPass *__restrict__ passes,
                          const BGate *__restrict__ gates,
                          const BGroup *__restrict__ groups, char *states,
                          char *lds, double *tot, double *inc, double *red,
@@ -845,7 +845,7 @@ __device__ void run_c128(const BCirc c, int part, int nparts, unsigned *sync,
     const BPass &ps = passes[c.first_pass + p];
     const TileBits tbits = load_tile_bits(ps.sbits);
     // a pass reads tiles the previous pass wrote, possibly in another part
-    if (nparts > 1 && p > 0 && !parts_barrier(sync, unsigned(p) * unsigned(nparts), err))
+    if (nparts > 1 && p > 0 && !parts_barrier(sync, unsigned(p) * unsigned(nparts), err, limit))
       return;
     const uint64_t outside = outside_mask(tbits, tb, n);
     const uint64_t bstep = tile_base(uint64_t(nparts), tbits, tb);
@@ -879,7 +879,7 @@ __device__ void run_c128(const BCirc c, int part, int nparts, unsigned *sync,
     }
   }
   // the last pass done by every part; part 0 samples the state
-  if (nparts > 1 && !parts_barrier(sync, unsigned(c.npass) * unsigned(nparts), err)) return;
+  if (nparts > 1 && !parts_barrier(sync, unsigned(c.npass) * unsigned(nparts), err, limit)) return;
   if (part != 0) return;
   if (resident && keep && G) {
     for (int e = tid; e < tile; e += NTH) G[e] = L[dswz(e)];
@@ -899,7 +899,7 @@ __device__ void run_c128(const BCirc c, int part, int nparts, unsigned *sync,
 
 template <int NTH>
 __device__ void run_c64(const BCirc c, int part, int nparts, unsigned *sync, unsigned *err,
-                        const BPass *__restrict__ passes,
+                        unsigned limit, const BPass *__restrict__ passes,
                         const BBlock *__restrict__ blocks,
                         const float *__restrict__ wbuf, char *states, char *lds,
                         double *tot, double *inc, double *red,
@@ -917,7 +917,7 @@ __device__ void run_c64(const BCirc c, int part, int nparts, unsigned *sync, uns
     const BPass &ps = passes[c.first_pass + p];
     const TileBits tbits = load_tile_bits(ps.sbits);
     // a pass reads tiles the previous pass wrote, possibly in another part
-    if (nparts > 1 && p > 0 && !parts_barrier(sync, unsigned(p) * unsigned(nparts), err))
+    if (nparts > 1 && p > 0 && !parts_barrier(sync, unsigned(p) * unsigned(nparts), err, limit))
       return;
     const uint64_t outside = outside_mask(tbits, tb, n);
     const uint64_t bstep = tile_base(uint64_t(nparts), tbits, tb);
@@ -947,7 +947,7 @@ __device__ void run_c64(const BCirc c, int part, int nparts, unsigned *sync, uns
   }
   // the last pass done by every part; part 0 renormalises and samples (the
   // norm's sum keeps its order whatever the number of parts)
-  if (nparts > 1 && !parts_barrier(sync, unsigned(c.npass) * unsigned(nparts), err)) return;
+  if (nparts > 1 && !parts_barrier(sync, unsigned(c.npass) * unsigned(nparts), err, limit)) return;
   if (part != 0) return;
   // FP64 renormalisation, q_state_normalize's rule (src/q_utils.c:112-118)
   const uint64_t N = uint64_t(1) << n;
@@ -1004,7 +1004,7 @@ __global__ __launch_bounds__(NTH) void k_batch(
     const BGroup *__restrict__ groups, const BBlock *__restrict__ blocks,
     const float *__restrict__ wbuf, char *states, const double *__restrict__ u,
     long *__restrict__ out, uint64_t shots, unsigned *queue, unsigned *sync,
-    int tile_bytes, int nch_cap, int keep) {
+    unsigned limit, int tile_bytes, int nch_cap, int keep) {
   extern __shared__ double4 smem4[];
   char *lds = reinterpret_cast<char *>(smem4);
   double *tot = reinterpret_cast<double *>(lds + tile_bytes);
@@ -1020,10 +1020,10 @@ __global__ __launch_bounds__(NTH) void k_batch(
     const BItem it = items[i];
     const BCirc c = circs[it.circ];
     if (c.prec == QCS_HIP_C128)
-      run_c128<NTH>(c, it.part, it.nparts, sync + it.circ, queue + 1, passes, gates,
+      run_c128<NTH>(c, it.part, it.nparts, sync + it.circ, queue + 1, limit, passes, gates,
                     groups, states, lds, tot, inc, red, u, out, shots, keep);
     else
-      run_c64<NTH>(c, it.part, it.nparts, sync + it.circ, queue + 1, passes, blocks, wbuf, states, lds, tot, inc, red, u,
+      run_c64<NTH>(c, it.part, it.nparts, sync + it.circ, queue + 1, limit, passes, blocks, wbuf, states, lds, tot, inc, red, u,
                    out, shots, keep);
   }
 }
@@ -1437,6 +1437,12 @@ static BBlock make_bblock(const qcs_hip_pass &ps, const qcs_hip_block &bl,
   return o;
 }
 
+// QCS_BATCH_PART_SPINS lowers the limit (tests: 0 gives up at once)
+static unsigned part_spin_limit() {
+  const char *e = std::getenv("QCS_BATCH_PART_SPINS");
+  return e ? unsigned(std::strtoul(e, nullptr, 10)) : kPartSpinLimit;
+}
+
 template <int NTH>
 static int launch_batch(qcs_hip_batch *b, const BatchLayout &L, int nitems,
                         uint64_t shots, int tile_bytes, int nch_cap, int grid) {
@@ -1451,7 +1457,7 @@ static int launch_batch(qcs_hip_batch *b, const BatchLayout &L, int nitems,
                      reinterpret_cast<const BBlock *>(d + L.block), b->d_w,
                      b->d_states, reinterpret_cast<const double *>(d + L.u),
                      b->d_out, shots, b->d_queue, reinterpret_cast<unsigned *>(d + L.sync),
-                     tile_bytes, nch_cap, (b->flags & QCS_HIP_BATCH_KEEP_STATES) ? 1 : 0);
+                     part_spin_limit(), tile_bytes, nch_cap, (b->flags & QCS_HIP_BATCH_KEEP_STATES) ? 1 : 0);
   return launch_check("k_batch");
 }
 
@@ -1559,6 +1565,23 @@ static int submit(qcs_hip_batch *b, bool rerun, int nb, bool build_graph) {
   }
   QCS_HIP_TRY(hipEventRecord(b->ev[3], b->stream));
   QCS_HIP_TRY(hipStreamSynchronize(b->stream));
+  if (*b->h_flag != 0u && b->last_nitems > nc) {
+    // the parts of a circuit were not on the device together (work of other
+    // processes holds it): once more, a work-group per circuit
+    BItem *items = reinterpret_cast<BItem *>(b->h_stage + L.order);
+    int k = 0;
+    for (int i = 0; i < b->last_nitems; ++i)
+      if (items[i].part == 0) items[k++] = BItem{items[i].circ, 0, 1, 0};
+    b->last_nitems = k;
+    b->last_grid = std::min(b->last_grid, k);
+    drop_graph(b);
+    b->replayed = 0;
+    if ((rc = enqueue_run(b, L, nc, 0, shots, b->last_tile_bytes, b->last_nch_cap, b->last_grid,
+                          true, false)))
+      return rc;
+    QCS_HIP_TRY(hipEventRecord(b->ev[3], b->stream));
+    QCS_HIP_TRY(hipStreamSynchronize(b->stream));
+  }
   if (*b->h_flag != 0u)
     return fail(QCS_HIP_EDEVICE, "batch: the work-groups sharing a circuit did not all "
                                  "reach a pass boundary in time");

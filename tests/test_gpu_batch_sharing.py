@@ -40,3 +40,28 @@ def test_shared_circuits_equal_unshared(qlib, monkeypatch, specs):
     assert np.array_equal(res[0][0], res[1][0])
     for x, y in zip(res[0][1], res[1][1]):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("options", [0, qcs_amd.BATCH_GRAPH])
+def test_parts_that_do_not_meet(qlib, monkeypatch, options):
+    """With no patience at all at the pass boundaries the parts give up, every
+    work-group exits, and the run is repeated with a work-group per circuit."""
+    libc = qcs_amd.libc()
+    cs = []
+    for i, fused in enumerate((False, True)):
+        c = qcs_amd.Circuit(17, qcs_amd.DEFERRED | (qcs_amd.FUSED_FP32 if fused else 0))
+        c.apply(C.layered(17, 3, 30 + i))
+        cs.append(c)
+    with qcs_amd.Batch(options) as b:
+        libc.srand(3)
+        want = b.sample(cs, 100)
+        monkeypatch.setenv("QCS_BATCH_PART_SPINS", "0")
+        libc.srand(3)
+        again = b.sample(cs, 100)  # a rerun of the plan
+        cs[0].x(0)
+        cs[0].x(0)                 # planned anew
+        libc.srand(3)
+        anew = b.sample(cs, 100)
+    assert np.array_equal(want, again) and np.array_equal(want, anew)
+    for c in cs:
+        c.close()
