@@ -370,6 +370,8 @@ int qcs_hip_state_set_basis(qcs_hip_state *s, long basis) {
   if (basis < 0 || uint64_t(basis) >= s->size)
     return fail(QCS_HIP_EINVAL, "basis %ld outside 2^%d", basis, s->n);
   bound_reset(s, 0.0);
+  s->support = 0;
+  s->basis = uint64_t(basis);
   if ((rc = launch_fill_basis(s, s->vec, uint64_t(basis), 1))) return rc;
   if (s->scratch && (rc = launch_fill_basis(s, s->scratch, 0, 0))) return rc;
   return 0;
@@ -401,6 +403,7 @@ int qcs_hip_write(qcs_hip_state *s, long offset, long count, const double *in) {
   if ((rc = ready(s)) || (rc = check_range(s, offset, count, in))) return rc;
   const size_t chunk_amps = size_t(1) << 20;
   if ((rc = ensure_pinned(s, chunk_amps * 16))) return rc;
+  if (count > 0) s->support = ~uint64_t(0);
   uint64_t exps = 0;  // the exponent bits of every value, or-ed
   for (long done = 0; done < count;) {
     const long m = long(std::min<size_t>(chunk_amps, size_t(count - done)));
@@ -475,6 +478,7 @@ int qcs_hip_phase_flip(qcs_hip_state *s, long index) {
 int qcs_hip_diffusion(qcs_hip_state *s) {
   int rc;
   if ((rc = ready(s))) return rc;
+  s->support = ~uint64_t(0);
   if (s->flags & QCS_HIP_COMPAT) return diffusion_compat(s);
   return grover_textbook(s, -1, 1);
 }
@@ -485,6 +489,7 @@ int qcs_hip_grover(qcs_hip_state *s, long marked, long iterations) {
   if (iterations <= 0) return 0;
   if (marked >= 0 && uint64_t(marked) >= s->size)
     return fail(QCS_HIP_EINVAL, "marked index %ld outside 2^%d", marked, s->n);
+  s->support = ~uint64_t(0);
   if (s->flags & QCS_HIP_COMPAT) {
     for (long i = 0; i < iterations; ++i) {
       if (marked >= 0 && (rc = phase_flip_compat(s, marked))) return rc;
@@ -626,6 +631,7 @@ int qcs_hip_apply_fused(qcs_hip_state *s, const qcs_hip_block *blocks,
   if ((rc = validate_blocks(s->n, blocks, num_blocks, gates, num_gates))) return rc;
   for (int g = 0; g < num_gates; ++g)
     if (gates[g].kind != QCS_HIP_G_SWAP) bound_gate(s, gates[g].m);
+  s->support = ~uint64_t(0);
   return fused_apply(s, blocks, num_blocks, gates, num_gates);
 }
 
@@ -641,6 +647,7 @@ int qcs_hip_apply_unitary(qcs_hip_state *s, int k, const int *targets,
     if (targets[q] < 0 || targets[q] >= s->n || (q > 0 && targets[q] <= targets[q - 1]))
       return fail(QCS_HIP_EINVAL, "apply_unitary: targets not ascending in range");
   bound_matrix(s, u, 1L << (2 * k));
+  s->support = ~uint64_t(0);
   return fused_apply_unitary(s, k, targets, u);
 }
 
@@ -692,6 +699,7 @@ static int check_passes(qcs_hip_state *s, const qcs_hip_pass *passes, int num_pa
   if ((rc = validate_blocks(s->n, blocks, num_blocks, gates, num_gates))) return rc;
   for (int g = 0; g < num_gates; ++g)
     if (gates[g].kind != QCS_HIP_G_SWAP) bound_gate(s, gates[g].m);
+  s->support = ~uint64_t(0);
   return 0;
 }
 

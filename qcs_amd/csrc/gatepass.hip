@@ -4,8 +4,11 @@
 // 5.8 TB/s in place).  A pass reads it once, runs the gates of gateplan.h's
 // program on it and writes it once, so the cost of a gate becomes its
 // arithmetic: a pass of the 28-qubit layered circuit (694 gates in 21 passes)
-// takes 1.82 ms, 4.7 TB/s, where each gate by itself took 1.2 ms; the circuit
-// went from 863 to 39.5 ms, the 28-qubit QFT (448 gates) from 270 to 24 ms.
+// takes 1.5-2.1 ms, where each gate by itself took 1.2 ms.  The passes are
+// bound by FP64 multiplies and adds (VALU 95 % busy at the 1.9 GHz the card
+// holds under them; 288 of the 344 instructions per RZ RY RZ), HBM below it at
+// 4-5.7 TB/s.  The circuit went from 863 to 36 ms, the 28-qubit QFT (448 gates)
+// from 270 to 20 ms.
 //
 // k_gate_pass.  One work-group per tile of 2^tb amplitudes; thread t holds 16
 // of them in registers, those that differ in the layout's four register
@@ -16,6 +19,11 @@
 // products by exact-zero entries, which add only signed zeros; the
 // amplitudes compare equal to the per-gate kernels' (bound_gate
 // keeps states whose amplitudes could overflow out).
+//
+// A state that starts as a basis state is zero wherever an index bit no gate
+// has mixed yet differs from the basis index; tiles of zeros are left alone
+// (28 qubits, H on every qubit and three layers: 21.5 -> 18.4 ms, with cheaper
+// addresses; the QFT of a basis state 15.4 -> 5.0 ms).
 #include <algorithm>
 #include <cmath>
 #include <exception>
@@ -192,12 +200,33 @@ __device__ __forceinline__ T par(const Par &w, int i) {
   }
 }
 
-// XOR of the entries whose bit is set in x
+// XOR of the entries whose bit is set in x (a lane's value): two or three
+// instructions a bit
+template <int N>
+__device__ __forceinline__ uint32_t xor_lanes(uint32_t x, const QCS_KERNARG uint32_t *e) {
+  uint32_t r = 0;
+#pragma unroll
+  for (int b = 0; b < N; ++b) r ^= e[b] & uint32_t(__builtin_amdgcn_sbfe(int(x), b, 1));
+  return r;
+}
+template <int N>
+__device__ __forceinline__ uint64_t xor_lanes(uint32_t x, const QCS_KERNARG uint64_t *e) {
+  uint32_t lo = 0, hi = 0;
+#pragma unroll
+  for (int b = 0; b < N; ++b) {
+    const uint32_t m = uint32_t(__builtin_amdgcn_sbfe(int(x), b, 1));
+    lo ^= uint32_t(e[b]) & m;
+    hi ^= uint32_t(e[b] >> 32) & m;
+  }
+  return uint64_t(hi) << 32 | lo;
+}
+// the same of a compile-time index (scalar arithmetic)
 template <int N, typename V>
-__device__ __forceinline__ V xor_bits(uint32_t x, const QCS_KERNARG V *e) {
+__device__ __forceinline__ V xor_const(int x, const QCS_KERNARG V *e) {
   V r = 0;
 #pragma unroll
-  for (int b = 0; b < N; ++b) r ^= e[b] & (V(0) - V((x >> b) & 1));
+  for (int b = 0; b < N; ++b)
+    if ((x >> b) & 1) r ^= e[b];
   return r;
 }
 
@@ -254,7 +283,6 @@ template <typename T>
 __global__ __launch_bounds__(1 << kPThrBits, 4) void k_gate_pass(
     const PassProgram by_value, typename Amp<T>::type *a, uint64_t ntiles) {
   typedef typename Amp<T>::type A;
-  extern __shared__ double lds_pass[];
   // the first argument starts the kernel-argument segment
   const ProgramPtr prog = (ProgramPtr)__builtin_amdgcn_kernarg_segment_ptr();
   const int tid = threadIdx.x;
@@ -262,17 +290,25 @@ __global__ __launch_bounds__(1 << kPThrBits, 4) void k_gate_pass(
   // a tile of fewer than 1024 amplitudes still takes a whole wave, whose
   // lanes past the tile compute on copies and store nothing
   const bool in = tid < (1 << (tb - kPRegBits));
-  // amplitude index of the tile: its number with zeros at the tile's bits
-  uint64_t base = xcd_order(blockIdx.x, ntiles);
-  for (int p = 0; p < tb; ++p) base = insert0(base, int(prog->bits[p]));
+  // amplitude index of the tile
+  uint64_t base = prog->fixed;
+  {
+    uint64_t t = xcd_order(blockIdx.x, ntiles);
+    for (uint64_t o = prog->outer; t; o &= o - 1, t >>= 1)
+      if (t & 1) base |= o & (~o + 1);
+  }
   T vr[kPAmps], vi[kPAmps];
   {
-    const uint64_t i0 = base | xor_bits<kPThrBits>(uint32_t(tid), prog->load_t);
+    // one thread address, plus a scalar offset per register (the masks of a
+    // load share no bit); lanes past the tile read its first amplitudes,
+    // their masks being zero
+    const char *p = reinterpret_cast<const char *>(
+        a + (base | xor_lanes<kPThrBits>(uint32_t(tid), prog->load_t)));
     A v[kPAmps];
-    // (lanes past the tile read its first amplitudes: their masks are zero)
 #pragma unroll
     for (int j = 0; j < kPAmps; ++j)
-      v[j] = ld_stream(a + (i0 | xor_bits<kPRegBits>(uint32_t(j), prog->load_r)));
+      v[j] = ld_stream(reinterpret_cast<const A *>(
+          p + xor_const<kPRegBits>(j, prog->load_r) * sizeof(A)));
 #pragma unroll
     for (int j = 0; j < kPAmps; ++j) {
       vr[j] = v[j].x;
@@ -333,43 +369,45 @@ __global__ __launch_bounds__(1 << kPThrBits, 4) void k_gate_pass(
     // the next one
     const LayoutPtr nxt = (LayoutPtr)w;
     const uint32_t tx = fresh(uint32_t(tid));
-    uint32_t ws = xor_bits<kPThrBits>(tx, lay->thr) >> 16;
-    const uint32_t rs = xor_bits<kPThrBits>(tx, nxt->thr) & 0xffffu;
+    uint32_t ws = xor_lanes<kPThrBits>(tx, lay->thr) >> 16;
+    const uint32_t rs = xor_lanes<kPThrBits>(tx, nxt->thr) & 0xffffu;
     for (uint32_t k = 0; k < lay->nterm; ++k) {
       const uint32_t t = lay->term[k];
       if ((base >> (t & 63)) & 1) ws ^= t >> 16;
     }
-    auto wslot = [&](int j) { return ws ^ (xor_bits<kPRegBits>(uint32_t(j), lay->reg) >> 16); };
-    auto rslot = [&](int j) { return rs ^ (xor_bits<kPRegBits>(uint32_t(j), nxt->reg) & 0xffffu); };
+    // byte offsets from the start of LDS, which is all dynamic here
+    typedef __attribute__((address_space(3))) double *LdsDouble;
+    typedef __attribute__((address_space(3))) f2v *LdsFloat2;
+    auto wslot = [&](int j) { return ws ^ (xor_const<kPRegBits>(j, lay->reg) >> 16); };
+    auto rslot = [&](int j) { return rs ^ (xor_const<kPRegBits>(j, nxt->reg) & 0xffffu); };
     __syncthreads();  // the reads of the exchange before
     if constexpr (sizeof(T) == 8) {
       if (in) {
 #pragma unroll
-        for (int j = 0; j < kPAmps; ++j) lds_pass[wslot(j)] = vr[j];
+        for (int j = 0; j < kPAmps; ++j) *(LdsDouble)uintptr_t(wslot(j)) = vr[j];
       }
       __syncthreads();
 #pragma unroll
       for (int j = 0; j < kPAmps; ++j)
-        vr[j] = lds_pass[rslot(j)];
+        vr[j] = *(LdsDouble)uintptr_t(rslot(j));
       __syncthreads();
       if (in) {
 #pragma unroll
-        for (int j = 0; j < kPAmps; ++j) lds_pass[wslot(j)] = vi[j];
+        for (int j = 0; j < kPAmps; ++j) *(LdsDouble)uintptr_t(wslot(j)) = vi[j];
       }
       __syncthreads();
 #pragma unroll
       for (int j = 0; j < kPAmps; ++j)
-        vi[j] = lds_pass[rslot(j)];
+        vi[j] = *(LdsDouble)uintptr_t(rslot(j));
     } else {
-      float2 *L = reinterpret_cast<float2 *>(lds_pass);
       if (in) {
 #pragma unroll
-        for (int j = 0; j < kPAmps; ++j) L[wslot(j)] = make_float2(vr[j], vi[j]);
+        for (int j = 0; j < kPAmps; ++j) *(LdsFloat2)uintptr_t(wslot(j)) = f2v{vr[j], vi[j]};
       }
       __syncthreads();
 #pragma unroll
       for (int j = 0; j < kPAmps; ++j) {
-        const float2 x = L[rslot(j)];
+        const f2v x = *(LdsFloat2)uintptr_t(rslot(j));
         vr[j] = x.x;
         vi[j] = x.y;
       }
@@ -382,15 +420,25 @@ __global__ __launch_bounds__(1 << kPThrBits, 4) void k_gate_pass(
     __syncthreads();
   }
   if (!in) return;
-  uint64_t i0 = base ^ xor_bits<kPThrBits>(fresh(uint32_t(tid)), prog->store_t);
+  uint64_t i0 = base ^ xor_lanes<kPThrBits>(fresh(uint32_t(tid)), prog->store_t);
   for (uint32_t k = 0; k < prog->store_nterm; ++k)
     if ((base >> prog->store_q[k]) & 1) i0 ^= prog->store_term[k];
-#pragma unroll
-  for (int j = 0; j < kPAmps; ++j) {
+  auto amp = [&](int j) {
     A o;
     o.x = vr[j];
     o.y = vi[j];
-    st_stream(a + (i0 ^ xor_bits<kPRegBits>(uint32_t(j), prog->store_r)), o);
+    return o;
+  };
+  if (prog->store_add) {
+    char *p = reinterpret_cast<char *>(a + i0);
+#pragma unroll
+    for (int j = 0; j < kPAmps; ++j)
+      st_stream(reinterpret_cast<A *>(p + xor_const<kPRegBits>(j, prog->store_r) * sizeof(A)),
+                amp(j));
+  } else {
+#pragma unroll
+    for (int j = 0; j < kPAmps; ++j)
+      st_stream(a + (i0 ^ xor_const<kPRegBits>(j, prog->store_r)), amp(j));
   }
 }
 
@@ -452,13 +500,14 @@ static int launch_pass(qcs_hip_state *s, const PassPick &pick,
                        const std::vector<PassGroup> &groups, int tb) {
   typedef typename Amp<T>::type A;
   PassProgram prog;
-  write_pass<T>(s->queue, pick, groups, tb, &prog);
-  const uint64_t ntiles = s->size >> tb;
+  write_pass<T>(s->queue, pick, groups, s->n, tb, s->support, s->basis, &prog);
+  const uint64_t ntiles = uint64_t(1) << __builtin_popcountll(prog.outer);
   const int threads = std::max(64, 1 << (tb - kPRegBits));
   const size_t lds = prog.nlayouts > 1 ? size_t(8) << tb : 0;
   TimedLaunch tl;
-  timing_begin(s, QCS_HIP_K_FUSED, 2.0 * double(s->size) * sizeof(A),
-               6.0 * double(s->size) * double(pick.gates.size()), &tl);
+  const double amps = double(ntiles << tb);
+  timing_begin(s, QCS_HIP_K_FUSED, 2.0 * amps * sizeof(A),
+               6.0 * amps * double(pick.gates.size()), &tl);
   hipLaunchKernelGGL(k_gate_pass<T>, dim3(unsigned(ntiles)), dim3(unsigned(threads)), lds,
                      s->stream, prog, static_cast<A *>(s->vec), ntiles);
   int rc = launch_check("k_gate_pass");
@@ -496,6 +545,7 @@ static int run_queue(qcs_hip_state *s, bool all) {
       q.clear();  // the state is no longer what the rest would act on
       break;
     }
+    for (int i : pick.gates) s->support |= plan_spread(q[size_t(i)]);
     size_t keep = 0, x = 0;
     for (size_t i = 0; i < q.size(); ++i) {
       if (x < pick.gates.size() && size_t(pick.gates[x]) == i) ++x;
@@ -523,6 +573,7 @@ int queue_gate(qcs_hip_state *s, int kind, int target, int control, const double
   const PlanGate g = plan_gate(kind, target, control, m);
   if (g.cls == kGCuDense || !(s->log2_bound < bound_limit(s))) {
     const int rc = s->queue.empty() ? 0 : run_queue(s, true);
+    s->support = ~uint64_t(0);  // 0 times infinity
     return rc ? rc : launch_gate(s, kind, target, control, m);
   }
   s->queue.push_back(g);

@@ -68,12 +68,12 @@ enum : uint8_t {
 // condition byte: thread bit b (< 16), or 64 + an index bit outside the tile
 constexpr int kPNoCond = 255;
 
-// Layout record, in whole words (scalar loads are 32 bits and up).  A slot
-// pair holds the LDS slot of a thread or register bit when the layout is
-// read, and in the upper half the slot it is written to for the next layout.
+// Layout record, in whole words (scalar loads are 32 bits and up).  A pair
+// holds the LDS byte offset of a thread or register bit when the layout is
+// read, and in the upper half the one it is written to for the next layout.
 struct PassLayout {
   uint32_t thr[kPThrBits], reg[kPRegBits];
-  uint32_t term[kPMaxTerms];  // index bit | slot << 16: written slots change where the bit is set
+  uint32_t term[kPMaxTerms];  // index bit | offset << 16: written offsets change where the bit is set
   uint32_t nterm;
   uint32_t opwords;           // words of the ops that follow the record
 };
@@ -82,12 +82,15 @@ constexpr int kPLayoutWords = int(sizeof(PassLayout) / 4);
 struct PassProgram {
   uint32_t tb;
   uint32_t nlayouts;
+  // Tiles: number t has its bits at the set bits of `outer` (ascending), and
+  // `fixed` elsewhere outside the tile.
+  uint64_t outer, fixed;
   uint64_t load_t[kPThrBits], load_r[kPRegBits];    // index masks of the first layout
   uint64_t store_t[kPThrBits], store_r[kPRegBits];  // index masks (XOR) of the last layout
   uint64_t store_term[kPMaxTerms];                  // XOR where index bit store_q is set
   uint32_t store_q[kPMaxTerms];
   uint32_t store_nterm;
-  uint32_t bits[kPMaxTile];  // tile position -> index bit, ascending
+  uint32_t store_add;  // the registers' masks share no bit with others: XOR is addition
   uint32_t words[kPWords + kPPad];
 };
 static_assert(sizeof(PassProgram) <= 4096 - 16, "a pass program travels as a kernel argument");
@@ -172,6 +175,11 @@ inline int plan_op_words(const PlanGate &g, int param_words) {  // an upper boun
     case kGPhase: case kGCPhase: return 1 + 2 * param_words;
     default: return 0;
   }
+}
+
+// Qubits along which a gate can move weight to amplitudes that were zero.
+inline uint64_t plan_spread(const PlanGate &g) {
+  return g.cls == kGSwap ? g.qubits : g.cls == kGCuDense ? uint64_t(1) << g.t : g.need;
 }
 
 // What a pass takes from the head of a gate list.
@@ -456,19 +464,24 @@ inline void write_ops(const std::vector<PlanGate> &gates, const std::vector<int>
   }
 }
 
-// The program of a pass.
+// The program of a pass.  Amplitudes whose index differs from `basis` in a bit
+// outside `support` are zero (and stay so): the pass runs the other tiles.
 template <typename T>
 inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
-                       const std::vector<PassGroup> &groups, int tb, PassProgram *pp) {
+                       const std::vector<PassGroup> &groups, int n, int tb, uint64_t support,
+                       uint64_t basis, PassProgram *pp) {
   std::memset(pp, 0, offsetof(PassProgram, words));
   pp->tb = uint32_t(tb);
-  int pos[64];
+  const uint64_t all = n < 64 ? (uint64_t(1) << n) - 1 : ~uint64_t(0);
+  pp->outer = support & all & ~pick.bits;
+  pp->fixed = basis & all & ~(support | pick.bits);
+  int pos[64], bits[kPMaxTile];
   for (int &p : pos) p = -1;
   int np = 0;
   for (int q = 0; q < 64; ++q)
     if ((pick.bits >> q) & 1) {
       pos[q] = np;
-      pp->bits[np++] = uint32_t(q);
+      bits[np++] = q;
     }
   auto positions = [&](uint64_t qubits) {
     unsigned r = 0;
@@ -502,7 +515,7 @@ inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
   auto index_mask = [&](int e) {
     uint64_t r = 0;
     for (int p = 0; p < tb; ++p)
-      if ((e >> p) & 1) r |= uint64_t(1) << pp->bits[p];
+      if ((e >> p) & 1) r |= uint64_t(1) << bits[p];
     return r;
   };
   const Step &first = steps.front(), &last = steps.back();
@@ -515,16 +528,26 @@ inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
     pp->store_q[k] = last.a.termq[k];
     pp->store_term[k] = index_mask(last.a.termv[k]);
   }
+  uint64_t seen = 0;
+  for (uint64_t m : pp->store_t) seen |= m;
+  for (uint64_t m : pp->store_term) seen |= m;
+  pp->store_add = 1;
+  for (uint64_t m : pp->store_r) {
+    if (seen & m) pp->store_add = 0;
+    seen |= m;
+  }
   uint32_t *w = pp->words;
   for (const Step &s : steps) {
     PassLayout l;
     std::memset(&l, 0, sizeof(l));
-    auto pair = [&](int p) { return uint32_t(pass_slot(1 << p)) | uint32_t(pass_slot(s.a.col[p])) << 16; };
+    auto pair = [&](int p) {
+      return uint32_t(8 * pass_slot(1 << p)) | uint32_t(8 * pass_slot(s.a.col[p])) << 16;
+    };
     for (int b = 0; b < s.m.nthr; ++b) l.thr[b] = pair(s.m.thr[b]);
     for (int b = 0; b < kPRegBits; ++b) l.reg[b] = pair(s.m.reg[b]);
     l.nterm = uint32_t(s.a.nterm);
     for (int k = 0; k < s.a.nterm; ++k)
-      l.term[k] = uint32_t(s.a.termq[k]) | uint32_t(pass_slot(s.a.termv[k])) << 16;
+      l.term[k] = uint32_t(s.a.termq[k]) | uint32_t(8 * pass_slot(s.a.termv[k])) << 16;
     uint32_t *rec = w;
     w += kPLayoutWords;
     if (s.g) write_ops<T>(gates, s.g->ops, s.m, pos, pick.bits, w);

@@ -95,6 +95,9 @@ struct qcs_hip_state {
   std::mutex queue_mu;  // qcs_hip_device_sync may come from another thread
   std::vector<qcs::PlanGate> queue;
   size_t queue_mark = qcs::kQueueLow;
+  // amplitudes whose index differs from `basis` in a bit outside `support`
+  // are zero (all bits: nothing is known); gate passes skip their tiles
+  uint64_t support = 0, basis = 0;
   double log2_bound = 0.0;  // bound of log2 of the amplitudes' two-norm
   // kernel timing
   int timing = 0;

@@ -144,15 +144,14 @@ static void op1(int cls, T *vr, T *vi, int q, const uint32_t *w, bool on) {
 template <typename T>
 static void run_pass(Vec<T> &v, int n, const PassProgram &pp) {
   const int tb = int(pp.tb), nthr = 1 << (tb - kPRegBits);
-  const uint64_t N = uint64_t(1) << n, ntiles = N >> tb;
+  const uint64_t N = uint64_t(1) << n;
+  const uint64_t ntiles = uint64_t(1) << __builtin_popcountll(pp.outer);
   std::vector<char> touched(N, 0), stored(N, 0);
   Vec<T> out = v;
   for (uint64_t tile = 0; tile < ntiles; ++tile) {
-    uint64_t base = tile;
-    for (int p = 0; p < tb; ++p) {
-      const uint64_t lo = base & ((uint64_t(1) << pp.bits[p]) - 1);
-      base = ((base >> pp.bits[p]) << (pp.bits[p] + 1)) | lo;
-    }
+    uint64_t base = pp.fixed, t = tile;
+    for (uint64_t o = pp.outer; t; o &= o - 1, t >>= 1)
+      if (t & 1) base |= o & (~o + 1);
     std::vector<T> vr(size_t(nthr) * kPAmps), vi(vr.size());
     for (int t = 0; t < nthr; ++t)
       for (int j = 0; j < kPAmps; ++j) {
@@ -210,7 +209,9 @@ static void run_pass(Vec<T> &v, int n, const PassProgram &pp) {
         for (uint32_t k = 0; k < lay.nterm; ++k)
           if ((base >> (lay.term[k] & 63)) & 1) ws ^= lay.term[k] >> 16;
         for (int j = 0; j < kPAmps; ++j) {
-          const uint32_t x = ws ^ (xor_bits<uint32_t>(uint32_t(j), lay.reg, kPRegBits) >> 16);
+          uint32_t x = ws ^ (xor_bits<uint32_t>(uint32_t(j), lay.reg, kPRegBits) >> 16);
+          if (x & 7) fail("write offset");
+          x /= 8;
           if (x >= full.size() || full[x]) fail("write slot");
           full[x] = 1;
           lr[x] = vr[size_t(t) * kPAmps + j];
@@ -220,7 +221,9 @@ static void run_pass(Vec<T> &v, int n, const PassProgram &pp) {
       for (int t = 0; t < nthr; ++t) {
         const uint32_t rs = xor_bits<uint32_t>(uint32_t(t), nxt.thr, kPThrBits) & 0xffffu;
         for (int j = 0; j < kPAmps; ++j) {
-          const uint32_t x = rs ^ (xor_bits<uint32_t>(uint32_t(j), nxt.reg, kPRegBits) & 0xffffu);
+          uint32_t x = rs ^ (xor_bits<uint32_t>(uint32_t(j), nxt.reg, kPRegBits) & 0xffffu);
+          if (x & 7) fail("read offset");
+          x /= 8;
           if (x >= full.size() || full[x] != 1) fail("read slot");
           full[x] = 2;
           vr[size_t(t) * kPAmps + j] = lr[x];
@@ -234,8 +237,10 @@ static void run_pass(Vec<T> &v, int n, const PassProgram &pp) {
       if ((base >> pp.store_q[k]) & 1) b2 ^= pp.store_term[k];
     for (int t = 0; t < nthr; ++t)
       for (int j = 0; j < kPAmps; ++j) {
-        const uint64_t i = b2 ^ xor_bits<uint64_t>(uint32_t(t), pp.store_t, kPThrBits) ^
-                           xor_bits<uint64_t>(uint32_t(j), pp.store_r, kPRegBits);
+        const uint64_t i0 = b2 ^ xor_bits<uint64_t>(uint32_t(t), pp.store_t, kPThrBits);
+        const uint64_t i = i0 ^ xor_bits<uint64_t>(uint32_t(j), pp.store_r, kPRegBits);
+        if (pp.store_add && i != i0 + xor_bits<uint64_t>(uint32_t(j), pp.store_r, kPRegBits))
+          fail("store sum");
         if (i >= N || stored[i]) fail("store index");
         stored[i] = 1;
         out.r[i] = vr[size_t(t) * kPAmps + j];
@@ -243,12 +248,13 @@ static void run_pass(Vec<T> &v, int n, const PassProgram &pp) {
       }
   }
   for (uint64_t i = 0; i < N; ++i)
-    if (!touched[i] || !stored[i]) fail("an amplitude was left out");
+    if (touched[i] != stored[i] || (!touched[i] && (v.r[i] != T(0) || v.i[i] != T(0))))
+      fail("an amplitude was left out");
   v = out;
 }
 
 template <typename T>
-static int check(int n, int tb, int low, int count, int style) {
+static int check(int n, int tb, int low, int count, int style, bool basis_state) {
   const uint64_t N = uint64_t(1) << n;
   std::vector<Gate> gates;
   std::vector<PlanGate> q;
@@ -304,6 +310,13 @@ static int check(int n, int tb, int low, int count, int style) {
     a.r[i] = T(uni() - 0.5);
     a.i[i] = T(uni() - 0.5);
   }
+  // a basis state, or any state
+  const uint64_t basis = rnd() & (N - 1);
+  uint64_t support = basis_state ? 0 : ~uint64_t(0);
+  for (uint64_t i = 0; basis_state && i < N; ++i) {
+    a.r[i] = T(i == basis ? 1 : 0);
+    a.i[i] = T(0);
+  }
   Vec<T> b = a;
   for (const Gate &g : gates) apply(a, n, g);
   for (const Gate &g : gates) q.push_back(plan_gate(g.kind, g.t, g.c, g.m));
@@ -315,8 +328,9 @@ static int check(int n, int tb, int low, int count, int style) {
     plan_pick(q, n, tb, low, int(sizeof(T) / 4), 64, &pick, &groups);
     if (pick.gates.empty()) fail("a pass without gates");
     if (__builtin_popcountll(pick.bits) != tb) fail("tile bits");
-    write_pass<T>(q, pick, groups, tb, &pp);
+    write_pass<T>(q, pick, groups, n, tb, support, basis, &pp);
     run_pass<T>(b, n, pp);
+    for (int i : pick.gates) support |= plan_spread(q[size_t(i)]);
     std::vector<PlanGate> rest;
     size_t x = 0;
     for (size_t i = 0; i < q.size(); ++i) {
@@ -342,8 +356,8 @@ int main() {
           for (int low = 3; low <= 4; ++low) {
             if (tb < n && tb < low + 4) continue;
             const int count = 20 + int(rnd() % 200);
-            total += check<double>(n, tb, low, count, style);
-            total += check<float>(n, tb, low, count, style);
+            total += check<double>(n, tb, low, count, style, rep == 1);
+            total += check<float>(n, tb, low, count, style, rep == 1);
           }
       }
   std::printf("ok %ld passes\n", total);
