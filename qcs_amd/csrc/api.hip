@@ -631,7 +631,7 @@ int qcs_hip_apply_fused(qcs_hip_state *s, const qcs_hip_block *blocks,
   if ((rc = validate_blocks(s->n, blocks, num_blocks, gates, num_gates))) return rc;
   for (int g = 0; g < num_gates; ++g)
     if (gates[g].kind != QCS_HIP_G_SWAP) bound_gate(s, gates[g].m);
-  s->support = ~uint64_t(0);
+  if (!bounded(s)) s->support = ~uint64_t(0);  // 0 times infinity
   return fused_apply(s, blocks, num_blocks, gates, num_gates);
 }
 
@@ -699,7 +699,7 @@ static int check_passes(qcs_hip_state *s, const qcs_hip_pass *passes, int num_pa
   if ((rc = validate_blocks(s->n, blocks, num_blocks, gates, num_gates))) return rc;
   for (int g = 0; g < num_gates; ++g)
     if (gates[g].kind != QCS_HIP_G_SWAP) bound_gate(s, gates[g].m);
-  s->support = ~uint64_t(0);
+  if (!bounded(s)) s->support = ~uint64_t(0);  // 0 times infinity
   return 0;
 }
 

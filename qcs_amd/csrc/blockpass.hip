@@ -49,7 +49,8 @@ __device__ __forceinline__ void bp_st(float2 *p, float4 x) {
 template <int K, int TB, int NTH, bool PIPE>
 __global__ __launch_bounds__(NTH) void k_fused_mfma(float2 *__restrict__ a,
                                                     const float *__restrict__ W,
-                                                    BlockGeom g, uint64_t ntiles) {
+                                                    BlockGeom g, uint64_t ntiles,
+                                                    uint64_t outer, uint64_t fixed) {
   constexpr int R = 1 << K, RR = 2 * R;
   constexpr int C = 1 << (TB - K);            // columns per tile
   constexpr int CS = C + 1;                   // LDS row stride (float2), padded
@@ -113,16 +114,20 @@ __global__ __launch_bounds__(NTH) void k_fused_mfma(float2 *__restrict__ a,
     step = gridDim.x;
     end = ntiles;
   }
-  auto tile_base = [&](uint64_t t) {
-    uint64_t b = t;
-#pragma unroll
-    for (int j = 0; j < TB; ++j) b = insert0(b, g.sbits[j]);
+  // tile t's base deposits t on the bits of `outer` (TileRange); the next
+  // one's follows by adding the deposited step
+  a += fixed;
+  auto deposit = [&](uint64_t t) {
+    uint64_t b = 0;
+    for (uint64_t o = outer; t; o &= o - 1, t >>= 1)
+      if (t & 1) b |= o & (~o + 1);
     return b;
   };
+  const uint64_t dstep = deposit(step);
 
   float4 v[IT];
   uint64_t tile = first;
-  uint64_t base = tile_base(tile);
+  uint64_t base = deposit(tile);
   if (PIPE && tile < end) {
 #pragma unroll
     for (int it = 0; it < IT; ++it) v[it] = bp_ld(a + (base | addr_it[it]));
@@ -142,7 +147,7 @@ __global__ __launch_bounds__(NTH) void k_fused_mfma(float2 *__restrict__ a,
     }
     __syncthreads();
     const uint64_t next = tile + step;
-    const uint64_t nbase = tile_base(next);
+    const uint64_t nbase = ((base | ~outer) + dstep) & outer;
     if (PIPE && next < end) {
 #pragma unroll
       for (int it = 0; it < IT; ++it) v[it] = bp_ld(a + (nbase | addr_it[it]));
@@ -215,14 +220,20 @@ static BlockGeom make_geom(int n, int k, const int *targets, int tb) {
   return g;
 }
 
+static uint64_t geom_mask(const BlockGeom &g, int tb) {
+  uint64_t m = 0;
+  for (int j = 0; j < tb; ++j) m |= uint64_t(1) << g.sbits[j];
+  return m;
+}
+
 template <int K, int TB, int NTH, bool PIPE>
 static void launch_k(qcs_hip_state *s, const float *W, const BlockGeom &g,
                      unsigned grid_cap) {
-  const uint64_t ntiles = s->size >> TB;
-  const uint64_t grid = ntiles < grid_cap ? ntiles : grid_cap;
+  const TileRange r = tile_range(s, geom_mask(g, TB), true);
+  const uint64_t grid = r.count < grid_cap ? r.count : grid_cap;
   hipLaunchKernelGGL((k_fused_mfma<K, TB, NTH, PIPE>), dim3(unsigned(grid)),
                      dim3(NTH), 0, s->stream, static_cast<float2 *>(s->vec), W, g,
-                     ntiles);
+                     r.count, r.outer, r.fixed);
 }
 
 // one-wave tiles, for states too small to fill the chip with larger ones; not
@@ -264,6 +275,14 @@ int block_variant_for(const qcs_hip_state *s, int variant) {
     variant = s->n < 21 ? kBlockTb10_64 : QCS_HIP_BLOCK_TB13_256_PIPE;
   if (variant == QCS_HIP_BLOCK_TB13_256_PIPE && s->n < 13) return QCS_HIP_BLOCK_TB12_256_PIPE;
   return variant;
+}
+
+// amplitudes that launch_block_mfma would read and write
+double block_mfma_amps(const qcs_hip_state *s, int k, const int *targets, int variant) {
+  const int v = block_variant_for(s, variant);
+  const int tb = v == kBlockTb10_64 ? 10
+                 : v == QCS_HIP_BLOCK_TB12_256 || v == QCS_HIP_BLOCK_TB12_256_PIPE ? 12 : 13;
+  return double(tile_range(s, geom_mask(make_geom(s->n, k, targets, tb), tb), true).count << tb);
 }
 
 int launch_block_mfma(qcs_hip_state *s, int k, const int *targets,

@@ -213,12 +213,13 @@ static void launch_valu(qcs_hip_state *s, int k, const double *U, const int *t) 
 // one HBM pass applying a composed block (W for MFMA, U for the VALU kernel)
 static int apply_block(qcs_hip_state *s, int k, const int *targets,
                        const float *W, const double *U) {
-  const double N = double(s->size);
-  const double bytes = 2.0 * N * double(s->amp_bytes);
-  const double flops = 8.0 * double(1 << k) * N;
   TimedLaunch tl;
   int rc;
-  timing_begin(s, QCS_HIP_K_FUSED, bytes, flops, &tl);
+  double amps = double(s->size);
+  if (s->precision == QCS_HIP_C64 && s->n >= 10)
+    amps = block_mfma_amps(s, k, targets, s->block_variant[k]);
+  timing_begin(s, QCS_HIP_K_FUSED, 2.0 * amps * double(s->amp_bytes),
+               8.0 * double(1 << k) * amps, &tl);
   if (s->precision == QCS_HIP_C64 && s->n >= 10) {
     if ((rc = launch_block_mfma(s, k, targets, W, s->block_variant[k]))) return rc;
   } else {
@@ -226,6 +227,7 @@ static int apply_block(qcs_hip_state *s, int k, const int *targets,
     else launch_valu<float>(s, k, U, targets);
     if ((rc = launch_check("k_fused_valu"))) return rc;
   }
+  for (int q = 0; q < k; ++q) s->support |= uint64_t(1) << targets[q];
   return timing_end(s, &tl);
 }
 

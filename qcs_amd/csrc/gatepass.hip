@@ -462,10 +462,12 @@ static double bound_limit(const qcs_hip_state *s) {
   return s->precision == QCS_HIP_C128 ? 900.0 : 100.0;
 }
 
+bool bounded(const qcs_hip_state *s) { return s->log2_bound < bound_limit(s); }
+
 void bound_reset(qcs_hip_state *s, double log2_norm) { s->log2_bound = log2_norm; }
 
 void bound_normalized(qcs_hip_state *s) {
-  if (s->log2_bound < bound_limit(s)) s->log2_bound = 1.0;
+  if (bounded(s)) s->log2_bound = 1.0;
 }
 
 // growth of the two-norm by a matrix of `count` complex entries: its
@@ -571,7 +573,7 @@ int queue_gate(qcs_hip_state *s, int kind, int target, int control, const double
   std::lock_guard<std::mutex> lock(s->queue_mu);
   if (kind != QCS_HIP_G_SWAP) bound_gate(s, m);
   const PlanGate g = plan_gate(kind, target, control, m);
-  if (g.cls == kGCuDense || !(s->log2_bound < bound_limit(s))) {
+  if (g.cls == kGCuDense || !bounded(s)) {
     const int rc = s->queue.empty() ? 0 : run_queue(s, true);
     s->support = ~uint64_t(0);  // 0 times infinity
     return rc ? rc : launch_gate(s, kind, target, control, m);

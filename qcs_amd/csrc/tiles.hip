@@ -824,7 +824,8 @@ template <int TB, int NTH, bool SPLIT, int K4>
 __global__ __launch_bounds__(NTH) void k_tile_program(
     float2 *__restrict__ a, const TilePass *__restrict__ passes, int pass_index,
     const TileBlock *__restrict__ blocks, const float *__restrict__ wbuf,
-    uint64_t ntiles, double *__restrict__ norm, const double *__restrict__ fsum) {
+    uint64_t ntiles, uint64_t outer, uint64_t fixed, double *__restrict__ norm,
+    const double *__restrict__ fsum) {
   constexpr int TILE = 1 << TB;
   constexpr bool DIR = K4 == 3;
   constexpr int KF = DIR ? 2 : K4;  // the block form
@@ -935,19 +936,17 @@ __global__ __launch_bounds__(NTH) void k_tile_program(
   const uint64_t xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
   uint64_t tile = xcd * T8 + slot;
   const uint64_t tend = (xcd + 1) * T8;
-  // tile t's base address deposits t on the index bits outside the tile
-  // (cmask); the next tile's, t + G8, is found by adding the deposited G8 in
-  // the deposited space: ((x | ~cmask) + dinc) & cmask
+  // tile t's base address deposits t on the index bits `outer` (those outside
+  // the tile that may be set in a non-zero amplitude; the others are `fixed`);
+  // the next tile's, t + G8, is found by adding the deposited G8 in the
+  // deposited space: ((x | ~outer) + dinc) & outer
+  a += fixed;
   auto deposit = [&](uint64_t t) {
-    uint64_t b = t;
-#pragma unroll
-    for (int j = 0; j < TB; ++j) b = insert0(b, ps.sbits[j]);
+    uint64_t b = 0;
+    for (uint64_t o = outer; t; o &= o - 1, t >>= 1)
+      if (t & 1) b |= o & (~o + 1);
     return b;
   };
-  uint64_t tmask = 0;
-#pragma unroll
-  for (int j = 0; j < TB; ++j) tmask |= uint64_t(1) << ps.sbits[j];
-  const uint64_t cmask = ((ntiles << TB) - 1) & ~tmask;
   const uint64_t dinc = deposit(G8);
 
   if constexpr (DIR) {
@@ -980,7 +979,7 @@ __global__ __launch_bounds__(NTH) void k_tile_program(
       for (int t = 0; t < 4; ++t)
         x[t] = ld_nt(a + (b | fo | ((t & 1) ? fr2 : 0) | ((t & 2) ? fr3 : 0)));
     };
-    auto step_base = [&](uint64_t b) { return ((b | ~cmask) + dinc) & cmask; };
+    auto step_base = [&](uint64_t b) { return ((b | ~outer) + dinc) & outer; };
     uint64_t base = deposit(tile);
     uint64_t nbase = step_base(base), nbase2 = step_base(nbase);
     // two tiles in flight, in two register sets taken in turn; past the
@@ -1042,7 +1041,7 @@ __global__ __launch_bounds__(NTH) void k_tile_program(
   constexpr int DEPTH = (!SPLIT && KF == 2) ? 2 : 1;
   float4 v0[IT], v1[IT];
   uint64_t base = deposit(tile);
-  auto step_base = [&](uint64_t b) { return ((b | ~cmask) + dinc) & cmask; };
+  auto step_base = [&](uint64_t b) { return ((b | ~outer) + dinc) & outer; };
   uint64_t nbase = step_base(base), nbase2 = step_base(nbase);
   if (tile < tend) {
 #pragma unroll
@@ -1222,7 +1221,7 @@ static int grow_dev(qcs_hip_state *s, void **p, size_t *cap, size_t need) {
 
 template <int NTH, bool SPLIT, int K4>
 static int launch_tp(qcs_hip_state *s, const TilePass *dpass, int pi,
-                     const TileBlock *dblocks, uint64_t ntiles, int nblocks,
+                     const TileBlock *dblocks, const TileRange &tiles, int nblocks,
                      double *norm = nullptr, int *grid_out = nullptr,
                      const double *fsum = nullptr) {
   // once per kernel instance (states may launch from separate threads)
@@ -1253,13 +1252,13 @@ static int launch_tp(qcs_hip_state *s, const TilePass *dpass, int pi,
       kTileLdsTile + size_t(SPLIT ? kTileStrideSplit : kTileStrideFp32) * size_t(nblocks);
   const uint64_t per_cu = kLdsPerCu / lds;  // work-groups that fit per CU
   uint64_t grid = uint64_t(s->tile_grid) * (per_cu > 1 ? 2 : 1);
-  if (grid > ntiles) grid = ntiles;
+  if (grid > tiles.count) grid = tiles.count;
   // the pass's norm: one partial per work-group in the reduction buffer
   if (norm && grid > uint64_t(kRedBlocks)) norm = nullptr;
   if (grid_out) *grid_out = norm ? int(grid) : 0;
   hipLaunchKernelGGL((k_tile_program<kTileBitsFixed, NTH, SPLIT, K4>), dim3(unsigned(grid)),
                      dim3(NTH), lds, s->stream, static_cast<float2 *>(s->vec),
-                     dpass, pi, dblocks, s->wbuf, ntiles, norm, fsum);
+                     dpass, pi, dblocks, s->wbuf, tiles.count, tiles.outer, tiles.fixed, norm, fsum);
   return launch_check("k_tile_program");
 }
 
@@ -1664,7 +1663,6 @@ int tiles_apply(qcs_hip_state *s, const qcs_hip_pass *passes, int np,
   const TilePass *dp = static_cast<const TilePass *>(s->tpass_dev);
   const TileBlock *db = static_cast<const TileBlock *>(s->tblock_dev);
   const bool split = s->tile_math == QCS_HIP_TILE_MATH_SPLIT_BF16;
-  const double N = double(s->size);
   int last_pass = -1, prev_pass = -1;
   for (int p = 0; p < np; ++p)
     if (passes[p].num_blocks > 0) {
@@ -1685,13 +1683,20 @@ int tiles_apply(qcs_hip_state *s, const qcs_hip_pass *passes, int np,
     // the kernel runs its pass's first block unconditionally: an empty pass
     // (which the planner does not make) would change nothing anyway
     if (passes[p].num_blocks <= 0) continue;
-    const uint64_t ntiles = s->size >> passes[p].tile_bits;
+    uint64_t pbits = 0, targets = 0;
+    for (int j = 0; j < passes[p].tile_bits; ++j) pbits |= uint64_t(1) << passes[p].bits[j];
+    // (the norm is summed over every tile, in the same order for any state)
+    const bool sums = norm_partials && (p == last_pass || (scale_ahead && p == prev_pass));
+    const TileRange tiles = tile_range(s, pbits, !sums);
+    const double amps = double(tiles.count << passes[p].tile_bits);
     double flops = 0.0;
     for (int b = passes[p].first_block;
-         b < passes[p].first_block + passes[p].num_blocks; ++b)
-      flops += 8.0 * double(1 << blocks[b].k) * N;
+         b < passes[p].first_block + passes[p].num_blocks; ++b) {
+      flops += 8.0 * double(1 << blocks[b].k) * amps;
+      for (int q = 0; q < blocks[b].k; ++q) targets |= uint64_t(1) << blocks[b].targets[q];
+    }
     TimedLaunch tl;
-    timing_begin(s, QCS_HIP_K_FUSED, 2.0 * N * double(s->amp_bytes), flops, &tl);
+    timing_begin(s, QCS_HIP_K_FUSED, 2.0 * amps * double(s->amp_bytes), flops, &tl);
     const int nbp = passes[p].num_blocks;
     double *nrm = nullptr;
     const double *fs = nullptr;
@@ -1703,17 +1708,18 @@ int tiles_apply(qcs_hip_state *s, const qcs_hip_pass *passes, int np,
     }
     int parts = 0;
     if (s->tile_threads == 1024)
-      rc = split ? launch_tp<1024, true, 0>(s, dp, p, db, ntiles, nbp)
-           : !k4p ? launch_tp<1024, false, 0>(s, dp, p, db, ntiles, nbp)
+      rc = split ? launch_tp<1024, true, 0>(s, dp, p, db, tiles, nbp)
+           : !k4p ? launch_tp<1024, false, 0>(s, dp, p, db, tiles, nbp)
            : s->tile_k4 == QCS_HIP_TILE_K4_GAUSS
                ? (tp[p].direct
-                      ? launch_tp<1024, false, 3>(s, dp, p, db, ntiles, nbp, nrm, &parts, fs)
-                      : launch_tp<1024, false, 2>(s, dp, p, db, ntiles, nbp, nrm, &parts, fs))
-               : launch_tp<1024, false, 1>(s, dp, p, db, ntiles, nbp);
+                      ? launch_tp<1024, false, 3>(s, dp, p, db, tiles, nbp, nrm, &parts, fs)
+                      : launch_tp<1024, false, 2>(s, dp, p, db, tiles, nbp, nrm, &parts, fs))
+               : launch_tp<1024, false, 1>(s, dp, p, db, tiles, nbp);
     else
-      rc = split ? launch_tp<512, true, 0>(s, dp, p, db, ntiles, nbp)
-                 : launch_tp<512, false, 0>(s, dp, p, db, ntiles, nbp);
+      rc = split ? launch_tp<512, true, 0>(s, dp, p, db, tiles, nbp)
+                 : launch_tp<512, false, 0>(s, dp, p, db, tiles, nbp);
     if (rc) return rc;
+    s->support |= targets;
     if ((rc = timing_end(s, &tl))) return rc;
     if (norm_partials && p == last_pass) *norm_partials = fs ? -1 : parts;
     if (scale_ahead && p == prev_pass && parts > 0 &&

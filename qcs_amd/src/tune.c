@@ -175,6 +175,11 @@ static int time_tile_plan(t_q_circuit *c, int k, int max_blocks, double *ms_out)
   int nb = 0, np = 0, b, rc;
   double ms = 0.0, bytes = 0.0, flops = 0.0;
   long launches = 0;
+  /* the identity as an explicit unitary: afterwards nothing is known to be
+   * zero any more, so every candidate's passes run all their tiles */
+  const double id[8] = {1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 1.0, 0.0};
+  const int q0 = 0;
+  if ((rc = qcs_hip_apply_unitary(c->state, 1, &q0, id)) != 0) return rc;
   if (qcs_pass_plan(c->pending, c->pending_size, c->num_qubits, QCS_HIP_TILE_BITS,
                     QCS_HIP_TILE_LOW_BITS, k, max_blocks, &passes, &np, &blocks, &nb,
                     &ordered) != 0)
