@@ -82,6 +82,25 @@ void qc_cphase(t_q_circuit *circuit, int control, int target, double angle);
 /* SWAP of two qubits (QFT with final swaps). */
 void qc_swap(t_q_circuit *circuit, int qubit_a, int qubit_b);
 
+/* Gate codes of qc_apply_gates. */
+#define QCS_OP_H 0
+#define QCS_OP_X 1
+#define QCS_OP_Y 2
+#define QCS_OP_Z 3
+#define QCS_OP_P 4
+#define QCS_OP_RX 5
+#define QCS_OP_RY 6
+#define QCS_OP_RZ 7
+#define QCS_OP_CNOT 8
+#define QCS_OP_CPHASE 9
+#define QCS_OP_SWAP 10
+/* Apply a gate list in order: gate i is the qc_* call of ops[i] on
+ * targets[i], with controls[i] (CNOT, CPHASE; the other qubit of a SWAP) and
+ * params[i] (the angle), as if called one by one.  Stops at the first
+ * unknown code; returns the number of gates applied. */
+long qc_apply_gates(t_q_circuit *circuit, const int *ops, const int *targets,
+                    const int *controls, const double *params, long count);
+
 /* Circuit options for qc_create_ex (bit flags). */
 #define QCS_PLAIN_FP64 0x0      /* complex128, gate by gate (default) */
 #define QCS_FUSED_FP32 0x1      /* complex64 state; gates are recorded and,

@@ -6,6 +6,8 @@ binds them with ctypes so Python tests and the bench can drive the same
 ``qc_*`` calls a C program makes.
 """
 import ctypes
+from array import array
+from itertools import islice
 
 import numpy as np
 
@@ -89,9 +91,22 @@ class Circuit:
 
     # gates ----------------------------------------------------------------------
     def apply(self, ops):
-        """Apply a circuits.Ops list through the qc_* entry points."""
-        d = self._dispatch
-        for op, t, c, p in zip(ops.op, ops.tq, ops.cq, ops.par):
+        """Apply a circuits.Ops list: one qc_apply_gates call, or the qc_*
+        entry points gate by gate for a list that C arrays cannot hold."""
+        op, tq, cq, par = ops.op, ops.tq, ops.cq, ops.par
+        try:
+            n = min(len(op), len(tq), len(cq), len(par))
+            lists = (array("i", list(op)), array("i", list(tq)), array("i", list(cq)),
+                     array("d", list(par)))
+        except (TypeError, ValueError, OverflowError):
+            n = 0
+        i = 0
+        if n:
+            i = self.lib.qc_apply_gates(self._c, *(x.buffer_info()[0] for x in lists), n)
+            if i == n:
+                return
+        d = self._dispatch  # from a gate that is no known one, too
+        for op, t, c, p in islice(zip(op, tq, cq, par), i, None):
             d[op](int(t), int(c), float(p))
 
     def __getattr__(self, name):

@@ -158,6 +158,7 @@ _QCS_PROTOS = {
     "qc_optimize": (None, [_Q]),
     "qc_cphase": (None, [_Q, c_int, c_int, c_double]),
     "qc_swap": (None, [_Q, c_int, c_int]),
+    "qc_apply_gates": (c_long, [_Q, c_void_p, c_void_p, c_void_p, c_void_p, c_long]),
     "qc_create_ex": (_Q, [c_int, c_int]),
     "qc_get_options": (c_int, [_Q]),
     "qc_flush": (None, [_Q]),
