@@ -164,10 +164,11 @@ static int check_state(const qcs_hip_state *s) {
   return 0;
 }
 
-// the state as every gate call so far left it: what is queued is launched
+// the state as every gate call so far left it, all of it in memory: what is
+// queued is launched
 static int ready(qcs_hip_state *s) {
   const int rc = check_state(s);
-  return rc ? rc : queue_flush(s);
+  return rc ? rc : queue_flush(s, true);
 }
 
 static int check_qubit(const qcs_hip_state *s, int q, const char *what) {
@@ -274,7 +275,7 @@ int qcs_hip_device_sync(void) {
   {
     std::lock_guard<std::mutex> lock(g_states_mu);
     for (qcs_hip_state *s : g_states)
-      if (s->device == dev && (rc = queue_flush(s))) return rc;
+      if (s->device == dev && (rc = queue_flush(s, false))) return rc;
   }
   QCS_HIP_TRY(hipDeviceSynchronize());
   return 0;
@@ -356,7 +357,7 @@ void qcs_hip_state_destroy(qcs_hip_state *s) {
     std::lock_guard<std::mutex> lock(g_states_mu);
     g_states.erase(std::find(g_states.begin(), g_states.end(), s));
   }
-  if (s) (void)queue_flush(s);
+  if (s) (void)queue_flush(s, false);
   free_state(s);
 }
 
@@ -366,13 +367,13 @@ int qcs_hip_state_flags(const qcs_hip_state *s) { return s ? s->flags : 0; }
 
 int qcs_hip_state_set_basis(qcs_hip_state *s, long basis) {
   int rc;
-  if ((rc = ready(s))) return rc;
+  if ((rc = check_state(s)) || (rc = queue_flush(s, false))) return rc;
   if (basis < 0 || uint64_t(basis) >= s->size)
     return fail(QCS_HIP_EINVAL, "basis %ld outside 2^%d", basis, s->n);
   bound_reset(s, 0.0);
   s->support = 0;
   s->basis = uint64_t(basis);
-  if ((rc = launch_fill_basis(s, s->vec, uint64_t(basis), 1))) return rc;
+  if ((rc = launch_basis_start(s))) return rc;
   if (s->scratch && (rc = launch_fill_basis(s, s->scratch, 0, 0))) return rc;
   return 0;
 }

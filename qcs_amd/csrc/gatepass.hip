@@ -302,13 +302,24 @@ __global__ __launch_bounds__(1 << kPThrBits, 4) void k_gate_pass(
     // one thread address, plus a scalar offset per register (the masks of a
     // load share no bit); lanes past the tile read its first amplitudes,
     // their masks being zero
-    const char *p = reinterpret_cast<const char *>(
-        a + (base | xor_lanes<kPThrBits>(uint32_t(tid), prog->load_t)));
+    const uint64_t i0 = base | xor_lanes<kPThrBits>(uint32_t(tid), prog->load_t);
+    const char *p = reinterpret_cast<const char *>(a + i0);
     A v[kPAmps];
+    if ((prog->skip_t | prog->skip_r) == 0) {
 #pragma unroll
-    for (int j = 0; j < kPAmps; ++j)
-      v[j] = ld_stream(reinterpret_cast<const A *>(
-          p + xor_const<kPRegBits>(j, prog->load_r) * sizeof(A)));
+      for (int j = 0; j < kPAmps; ++j)
+        v[j] = ld_stream(reinterpret_cast<const A *>(
+            p + xor_const<kPRegBits>(j, prog->load_r) * sizeof(A)));
+    } else {
+      const bool lane = ((i0 ^ prog->basis) & prog->skip_t) == 0;
+#pragma unroll
+      for (int j = 0; j < kPAmps; ++j) {
+        const uint64_t off = xor_const<kPRegBits>(j, prog->load_r);
+        v[j].x = v[j].y = T(0);
+        if (((off ^ prog->basis) & prog->skip_r) == 0 && lane)
+          v[j] = ld_stream(reinterpret_cast<const A *>(p + off * sizeof(A)));
+      }
+    }
 #pragma unroll
     for (int j = 0; j < kPAmps; ++j) {
       vr[j] = v[j].x;
@@ -502,18 +513,23 @@ static int launch_pass(qcs_hip_state *s, const PassPick &pick,
                        const std::vector<PassGroup> &groups, int tb) {
   typedef typename Amp<T>::type A;
   PassProgram prog;
-  write_pass<T>(s->queue, pick, groups, s->n, tb, s->support, s->basis, &prog);
+  write_pass<T>(s->queue, pick, groups, s->n, tb, s->support, s->basis, &prog, s->filled);
   const uint64_t ntiles = uint64_t(1) << __builtin_popcountll(prog.outer);
   const int threads = std::max(64, 1 << (tb - kPRegBits));
   const size_t lds = prog.nlayouts > 1 ? size_t(8) << tb : 0;
   TimedLaunch tl;
   const double amps = double(ntiles << tb);
-  timing_begin(s, QCS_HIP_K_FUSED, 2.0 * amps * sizeof(A),
+  const double read = amps / double(uint64_t(1) << __builtin_popcountll(prog.skip_t | prog.skip_r));
+  timing_begin(s, QCS_HIP_K_FUSED, (amps + read) * sizeof(A),
                6.0 * amps * double(pick.gates.size()), &tl);
   hipLaunchKernelGGL(k_gate_pass<T>, dim3(unsigned(ntiles)), dim3(unsigned(threads)), lds,
                      s->stream, prog, static_cast<A *>(s->vec), ntiles);
   int rc = launch_check("k_gate_pass");
   if (rc) return rc;
+  if (s->filled != ~uint64_t(0)) {
+    s->filled |= pick.bits;
+    if ((~s->filled & (s->size - 1)) == 0) s->filled = ~uint64_t(0);
+  }
   return timing_end(s, &tl);
 }
 
@@ -534,10 +550,12 @@ static int run_queue(qcs_hip_state *s, bool all) {
     if (pick.gates.size() <= 1 || (s->n >= kPassBigState && traffic <= 2.0)) {
       // the per-gate kernels move no more than the pass would
       if (pick.gates.empty()) pick.gates.push_back(0);
+      rc = launch_fill_rest(s);
       for (int i : pick.gates) {
+        if (rc) break;
         const PlanGate &g = q[size_t(i)];
         const int kind = g.cls == kGSwap ? QCS_HIP_G_SWAP : g.c >= 0 ? QCS_HIP_G_CU : QCS_HIP_G_1Q;
-        if ((rc = launch_gate(s, kind, g.t, g.c, g.m))) break;
+        rc = launch_gate(s, kind, g.t, g.c, g.m);
       }
     } else {
       rc = s->precision == QCS_HIP_C128 ? launch_pass<double>(s, pick, groups, tb)
@@ -560,10 +578,11 @@ static int run_queue(qcs_hip_state *s, bool all) {
 }
 
 // (the planner's vectors may throw; the queue is whole either way)
-int queue_flush(qcs_hip_state *s) try {
+int queue_flush(qcs_hip_state *s, bool fill) try {
   if (!s->queued) return 0;
   std::lock_guard<std::mutex> lock(s->queue_mu);
-  return s->queue.empty() ? 0 : run_queue(s, true);
+  const int rc = s->queue.empty() ? 0 : run_queue(s, true);
+  return rc || !fill ? rc : launch_fill_rest(s);
 } catch (const std::exception &) {
   return fail(QCS_HIP_ENOMEM, "planning the queued gates: out of host memory");
 }
@@ -574,7 +593,8 @@ int queue_gate(qcs_hip_state *s, int kind, int target, int control, const double
   if (kind != QCS_HIP_G_SWAP) bound_gate(s, m);
   const PlanGate g = plan_gate(kind, target, control, m);
   if (g.cls == kGCuDense || !bounded(s)) {
-    const int rc = s->queue.empty() ? 0 : run_queue(s, true);
+    int rc = s->queue.empty() ? 0 : run_queue(s, true);
+    if (!rc) rc = launch_fill_rest(s);
     s->support = ~uint64_t(0);  // 0 times infinity
     return rc ? rc : launch_gate(s, kind, target, control, m);
   }

@@ -85,6 +85,10 @@ struct PassProgram {
   // Tiles: number t has its bits at the set bits of `outer` (ascending), and
   // `fixed` elsewhere outside the tile.
   uint64_t outer, fixed;
+  // Amplitudes of the tile that are zero without being so in memory: where
+  // the index differs from `basis` in a bit of skip_t (thread bits) or skip_r
+  // (register bits).
+  uint64_t skip_t, skip_r, basis;
   uint64_t load_t[kPThrBits], load_r[kPRegBits];    // index masks of the first layout
   uint64_t store_t[kPThrBits], store_r[kPRegBits];  // index masks (XOR) of the last layout
   uint64_t store_term[kPMaxTerms];                  // XOR where index bit store_q is set
@@ -466,13 +470,17 @@ inline void write_ops(const std::vector<PlanGate> &gates, const std::vector<int>
 
 // The program of a pass.  Amplitudes whose index differs from `basis` in a bit
 // outside `support` are zero (and stay so): the pass runs the other tiles.
+// Where `filled` is not all ones, memory holds only the amplitudes that agree
+// with `basis` outside `filled` (which includes `support`): the pass runs
+// their tiles and reads nothing else; afterwards the tile bits are filled too.
 template <typename T>
 inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
                        const std::vector<PassGroup> &groups, int n, int tb, uint64_t support,
-                       uint64_t basis, PassProgram *pp) {
+                       uint64_t basis, PassProgram *pp, uint64_t filled = ~uint64_t(0)) {
   std::memset(pp, 0, offsetof(PassProgram, words));
   pp->tb = uint32_t(tb);
   const uint64_t all = n < 64 ? (uint64_t(1) << n) - 1 : ~uint64_t(0);
+  if (~filled & all) support = filled;
   pp->outer = support & all & ~pick.bits;
   pp->fixed = basis & all & ~(support | pick.bits);
   int pos[64], bits[kPMaxTile];
@@ -521,6 +529,9 @@ inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
   const Step &first = steps.front(), &last = steps.back();
   for (int b = 0; b < first.m.nthr; ++b) pp->load_t[b] = index_mask(1 << first.m.thr[b]);
   for (int b = 0; b < kPRegBits; ++b) pp->load_r[b] = index_mask(1 << first.m.reg[b]);
+  for (uint64_t m : pp->load_t) pp->skip_t |= m & ~filled;
+  for (uint64_t m : pp->load_r) pp->skip_r |= m & ~filled;
+  pp->basis = basis;
   for (int b = 0; b < last.m.nthr; ++b) pp->store_t[b] = index_mask(last.a.col[last.m.thr[b]]);
   for (int b = 0; b < kPRegBits; ++b) pp->store_r[b] = index_mask(last.a.col[last.m.reg[b]]);
   pp->store_nterm = uint32_t(last.a.nterm);

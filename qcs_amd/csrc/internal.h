@@ -98,6 +98,10 @@ struct qcs_hip_state {
   // amplitudes whose index differs from `basis` in a bit outside `support`
   // are zero (all bits: nothing is known); gate passes skip their tiles
   uint64_t support = 0, basis = 0;
+  // memory holds only the amplitudes that agree with `basis` outside `filled`,
+  // the others being zero; gate passes fill the rest as they grow the support,
+  // anything else has it filled first
+  uint64_t filled = ~uint64_t(0);
   double log2_bound = 0.0;  // bound of log2 of the amplitudes' two-norm
   // kernel timing
   int timing = 0;
@@ -142,10 +146,12 @@ int launch_1q(qcs_hip_state *s, int target, const double m[8]);
 int launch_cu(qcs_hip_state *s, int control, int target, const double m[8]);
 int launch_swap(qcs_hip_state *s, int a, int b);
 int launch_fill_basis(qcs_hip_state *s, void *buf, uint64_t basis, int one);
+int launch_basis_start(qcs_hip_state *s);
+int launch_fill_rest(qcs_hip_state *s);
 // kernels in gatepass.hip: a plain gate is queued, and launched together
 // with others on its tile; queue_flush launches what is queued
 int queue_gate(qcs_hip_state *s, int kind, int target, int control, const double *m);
-int queue_flush(qcs_hip_state *s);
+int queue_flush(qcs_hip_state *s, bool fill);
 // the bound of the state's two-norm that decides whether gates may be queued
 void bound_reset(qcs_hip_state *s, double log2_norm);
 void bound_normalized(qcs_hip_state *s);

@@ -89,3 +89,62 @@ def test_calls_that_fill_the_state(qlib, option):
                 c.apply(ops)
             assert np.array_equal(a.amplitudes(), b.amplitudes()), between.__name__
             assert abs(a.norm_sq() - b.norm_sq()) == 0.0
+
+
+@pytest.mark.parametrize("option,n", [(qcs_amd.PLAIN_FP64, 21), (qcs_amd.PLAIN_FP32, 22),
+                                      (qcs_amd.FUSED_FP32 | qcs_amd.FUSE_TILES, 22)])
+def test_zeros_that_no_pass_wrote(qlib, option, n):
+    """A large basis state starts without its zeros in memory (here full of
+    another state's amplitudes): every call sees them all the same."""
+    hip, _ = qlib
+    basis = 0x155A5A & ((1 << n) - 1)
+    v = np.zeros(1 << n, np.complex128)
+    v[basis] = 1.0
+    full = C.Ops()
+    for q in range(n):
+        full.add(C.H, q)
+
+    def near(c, ops):
+        c.apply(ops)
+        return c.amplitudes()
+
+    some = few_qubits(n, [1, 2, 9, 17], 3)
+    swap = C.Ops().add(C.SWAP, 0, n - 1)
+    calls = {
+        "read": lambda c: c.amplitudes(),
+        "part": lambda c: c.amplitudes((1 << n) - 5000, 5000),
+        "norm": lambda c: np.array([c.norm_sq()]),
+        "probability": lambda c: np.array([c.get_probability_l(basis), c.get_probability_l(3)]),
+        "most likely": lambda c: np.array([c.find_most_likely_state_l()]),
+        "sample": lambda c: c.sample_indices(16),
+        "one pass": lambda c: near(c, some),
+        "one gate": lambda c: near(c, C.Ops().add(C.H, n - 1)),
+        "swap": lambda c: near(c, swap),
+        "all qubits": lambda c: near(c, full),
+        "measure": lambda c: np.concatenate([c.measure_all_list(), c.amplitudes().view(float)]),
+        "pass, measure": lambda c: (c.apply(some), c.measure_all_list(), c.amplitudes())[2],
+        "write": lambda c: (c.set_amplitudes(np.ones(3, complex), 77), c.amplitudes())[1],
+        "grover": lambda c: np.array([hip.qcs_hip_grover(c.device_state, 5, 2), *c.amplitudes(0, 9)]),
+        "overflow": lambda c: (huge(hip, c), c.amplitudes())[1],
+    }
+    with qcs_amd.Circuit(n, option) as a, qcs_amd.Circuit(n, option) as b:
+        for name, call in calls.items():
+            for c in (a, b):
+                c.apply(full)
+                c.lib.qc_flush(c.handle)
+            a.set_basis_state(basis)
+            b.set_amplitudes(v)
+            libc = qcs_amd.libc()
+            libc.srand(7)
+            x = call(a)
+            libc.srand(7)
+            y = call(b)
+            assert np.array_equal(x, y, equal_nan=True), name
+
+
+def huge(hip, c):
+    import ctypes
+    m = (ctypes.c_double * 8)(1e200, 0, 0, 0, 0, 0, 1e200, 0)
+    if c.options & 1 == 0:  # (a matrix beyond the bound of queued gates)
+        for _ in range(2):
+            assert hip.qcs_hip_apply_1q(c.device_state, 1, m) == 0
