@@ -106,6 +106,48 @@ __device__ __forceinline__ double wave_incl_scan(double x, int lane) {
   return x;
 }
 
+// What wave_incl_scan leaves in lane 63, bit for bit, in every lane: its
+// additions are those of a binary tree over aligned blocks of lanes, which
+// within 16 lanes run on DPP moves and then on lane reads, without the scan's
+// twelve trips through the LDS crossbar.
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double x) {
+  const uint64_t v = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(v)), CTRL, 15, 15, true));
+  const uint32_t hi = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(v >> 32)), CTRL, 15, 15, true));
+  return x + __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+}
+__device__ __forceinline__ double read_lane(double x, int lane) {
+  const uint64_t v = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(v)), lane));
+  const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(v >> 32)), lane));
+  return __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+}
+__device__ __forceinline__ double wave_scan_total(double x) {
+  x = dpp_add<0xB1>(x);   // lanes 1 apart (quad_perm 1 0 3 2)
+  x = dpp_add<0x4E>(x);   // 2 apart (quad_perm 2 3 0 1)
+  x = dpp_add<0x141>(x);  // the other four of eight (row_half_mirror)
+  x = dpp_add<0x140>(x);  // the other eight of sixteen (row_mirror)
+  const double lo = read_lane(x, 16) + read_lane(x, 0);
+  const double hi = read_lane(x, 48) + read_lane(x, 32);
+  return hi + lo;
+}
+
+// One row of 64 amplitudes against a uniform: the mask of the lanes whose
+// cumulative probability (e: of the chunks before, running: of the rows
+// before) exceeds u at a non-zero amplitude; x is the lane's probability.
+__device__ __forceinline__ unsigned long long row_hits(double x, int lane, double e,
+                                                       double running, double u) {
+  const double local = running + wave_incl_scan(x, lane);
+  const double cdf = e + local;
+  return __ballot(cdf > u && x > 0.0);
+}
+// false only where no lane of the row can exceed u: its lanes' sums are at
+// most the row's total but for roundings of 1e-15 (NaN: not skipped)
+__device__ __forceinline__ bool row_may_hit(double tot, double e, double running, double u) {
+  return !((e + (running + tot)) * (1.0 + 1e-12) < u);
+}
+
 // Sum of v over the work-group; `lds` holds blockDim.x/64 doubles.
 // The result is valid in thread 0.
 __device__ __forceinline__ double block_sum(double v, double *lds) {

@@ -465,22 +465,46 @@ __global__ __launch_bounds__(kThreads) void k_argmax_final(
 // The sampling kernel recomputes local(i) with the same operations, so
 // cdf(last of chunk c) == P[c] bit for bit.
 
+//
+// The rows' totals do not depend on one another, only their chain does: a
+// work-group takes a chunk, its waves the rows, and one lane runs the chain.
+// (A wave per chunk, row after row, waited for memory and for the scan's
+// lane crossings 64 times over: at 20 qubits 43 -> 6 us; at 28 qubits, bound by
+// HBM either way, 0.73 -> 0.71 ms.)
+constexpr int kRowWaves = kThreads / 64;
+constexpr int kRowsMax = int(kChunk / 64);
+
+// totals of the chunk's rows (as wave_incl_scan's last lane) into rows[]
+template <typename A>
+__device__ __forceinline__ void chunk_rows(const A *p, uint64_t len, double *rows) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int U = kRowsMax / kRowWaves;
+  A v[U];
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    const uint64_t i = uint64_t(k * kRowWaves + wave) * 64 + lane;
+    v[k].x = v[k].y = 0;
+    if (i < len) v[k] = p[i];
+  }
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    const double t = wave_scan_total(norm2(v[k]));
+    if (lane == 0) rows[k * kRowWaves + wave] = t;
+  }
+}
 
 template <typename T>
-__global__ __launch_bounds__(kThreads) void k_chunk_tot(
-    const typename Amp<T>::type *a, uint64_t nchunks, uint64_t len,
-    double *tot) {
-  const int lane = threadIdx.x & 63;
-  const uint64_t c = uint64_t(blockIdx.x) * (kThreads / 64) + (threadIdx.x >> 6);
-  if (c >= nchunks) return;
-  const typename Amp<T>::type *p = a + c * len;
+__global__ __launch_bounds__(kThreads) void k_chunk_tot(const typename Amp<T>::type *a,
+                                                        uint64_t len, double *tot) {
+  __shared__ double rows[kRowsMax];
+  const uint64_t c = blockIdx.x;
+  chunk_rows(a + c * len, len, rows);
+  __syncthreads();
+  if (threadIdx.x != 0) return;
   double running = 0.0;
-  for (uint64_t r = 0; r < len; r += 64) {
-    const double x = (r + lane < len) ? norm2(p[r + lane]) : 0.0;
-    const double s = wave_incl_scan(x, lane);
-    running = running + __shfl(s, 63, 64);
-  }
-  if (lane == 0) tot[c] = running;
+#pragma unroll 16
+  for (int r = 0; r < kRowsMax; ++r) running = running + rows[r];
+  tot[c] = running;
 }
 
 // One work-group: excl[c] (in place over tot) and inc[c] = excl[c] + tot[c].
@@ -509,7 +533,9 @@ __global__ __launch_bounds__(1024) void k_chunk_scan(double *tot, double *inc,
   __syncthreads();
   if (threadIdx.x == 0) {
     double run = 0.0;
-    for (int t0 = 0; t0 < 1024; t0 += U) {
+    // (the threads past the last chunk hold zeros)
+    const int used = int(ceil_div(nchunks, per));
+    for (int t0 = 0; t0 < used; t0 += U) {
       double v[U];
 #pragma unroll
       for (int j = 0; j < U; ++j) v[j] = base[t0 + j];
@@ -542,6 +568,17 @@ __global__ __launch_bounds__(1024) void k_chunk_scan(double *tot, double *inc,
   }
 }
 
+// first chunk whose inclusive prefix exceeds u (inc is non-decreasing)
+__device__ __forceinline__ uint64_t find_chunk(const double *inc, uint64_t nchunks, double u) {
+  uint64_t lo = 0, hi = nchunks;
+  while (lo < hi) {
+    const uint64_t mid = (lo + hi) >> 1;
+    if (inc[mid] > u) hi = mid; else lo = mid + 1;
+  }
+  return lo;
+}
+
+// A wave per shot, its chunk row by row.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void k_sample(
     const typename Amp<T>::type *a, uint64_t nchunks, uint64_t len,
@@ -551,17 +588,11 @@ __global__ __launch_bounds__(kThreads) void k_sample(
   const uint64_t s = uint64_t(blockIdx.x) * (kThreads / 64) + (threadIdx.x >> 6);
   if (s >= shots) return;
   const double us = u[s];
-  // first chunk with inc > u (inc is non-decreasing)
-  uint64_t lo = 0, hi = nchunks;
-  while (lo < hi) {
-    const uint64_t mid = (lo + hi) >> 1;
-    if (inc[mid] > us) hi = mid; else lo = mid + 1;
-  }
-  if (lo >= nchunks) {  // u not below the total: dropped, as the reference
+  const uint64_t c = find_chunk(inc, nchunks, us);
+  if (c >= nchunks) {  // u not below the total: dropped, as the reference
     if (lane == 0) out[s] = -1;
     return;
   }
-  const uint64_t c = lo;
   const double e = excl[c];
   const typename Amp<T>::type *p = a + c * len;
   double running = 0.0;
@@ -584,6 +615,64 @@ __global__ __launch_bounds__(kThreads) void k_sample(
   // non-zero amplitude seen in the chunk
   if (found < 0) found = last_nz;
   if (lane == 0) out[s] = found;
+}
+
+// A work-group per shot, while there are few: the chunk's rows are summed at
+// once and only those that may hold the shot are scanned, by one wave.  It
+// reads all of the chunk, which a wave per shot leaves half-way on average: at
+// 20 qubits 14 us for 1024 shots and 44 for 8192 where a wave per shot takes
+// 45 and 69, but at 28 qubits, from HBM, 20 and 86 against 23 and 78.
+constexpr long kWideShots = 4096;
+
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_sample_wide(
+    const typename Amp<T>::type *a, uint64_t nchunks, uint64_t len, const double *excl,
+    const double *inc, const double *u, long *out) {
+  constexpr int kHeld = 1024;
+  __shared__ double held[kHeld], rows[kRowsMax];
+  const int lane = threadIdx.x & 63;
+  const double us = u[blockIdx.x];
+  uint64_t c;
+  if (nchunks <= kHeld) {  // the search's dependent reads from LDS
+    for (uint64_t k = threadIdx.x; k < nchunks; k += kThreads) held[k] = inc[k];
+    __syncthreads();
+    c = find_chunk(held, nchunks, us);
+  } else {
+    c = find_chunk(inc, nchunks, us);
+  }
+  if (c >= nchunks) {
+    if (threadIdx.x == 0) out[blockIdx.x] = -1;
+    return;
+  }
+  const typename Amp<T>::type *p = a + c * len;
+  chunk_rows(p, len, rows);
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  const double e = excl[c];
+  double running = 0.0, mine = 0.0;  // lane r: the sum of the rows before r
+#pragma unroll 16
+  for (int r = 0; r < kRowsMax; ++r) {
+    if (r == lane) mine = running;
+    running = running + rows[r];
+  }
+  const uint64_t nrows = ceil_div(len, 64);
+  long found = -1;
+  unsigned long long may =
+      __ballot(uint64_t(lane) < nrows && row_may_hit(rows[lane], e, mine, us));
+  for (; may && found < 0; may &= may - 1) {
+    const int r = __ffsll(may) - 1;
+    const uint64_t i = uint64_t(r) * 64 + lane;
+    const double x = i < len ? norm2(p[i]) : 0.0;
+    const unsigned long long hit = row_hits(x, lane, e, read_lane(mine, r), us);
+    if (hit) found = long(c * len + uint64_t(r) * 64) + __ffsll(hit) - 1;
+  }
+  // (as in k_sample)
+  for (uint64_t r = nrows; r-- > 0 && found < 0;) {
+    const uint64_t i = r * 64 + lane;
+    const unsigned long long nz = __ballot((i < len ? norm2(p[i]) : 0.0) > 0.0);
+    if (nz) found = long(c * len + r * 64) + 63 - __clzll(nz);
+  }
+  if (lane == 0) out[blockIdx.x] = found;
 }
 
 // ---- Grover (textbook) ----------------------------------------------------
@@ -1159,6 +1248,29 @@ int argmax(qcs_hip_state *s, long *idx) {
 }
 
 template <typename T>
+static int launch_sample(qcs_hip_state *s, uint64_t nchunks, uint64_t len, const double *excl,
+                         const double *inc, long shots, const double *u, long *out) {
+  const auto *a = static_cast<const typename Amp<T>::type *>(s->vec);
+  if (shots <= 0) return 0;
+  if (shots <= kWideShots) {
+    hipLaunchKernelGGL(k_sample_wide<T>, dim3(unsigned(shots)), dim3(kThreads), 0, s->stream, a,
+                       nchunks, len, excl, inc, u, out);
+    return launch_check("k_sample_wide");
+  }
+  // one wave per shot; at most 2^24 shots per dispatch keeps the
+  // work-item count below 2^32
+  for (uint64_t s0 = 0; s0 < uint64_t(shots); s0 += uint64_t(1) << 24) {
+    const uint64_t ns = std::min<uint64_t>(uint64_t(shots) - s0, uint64_t(1) << 24);
+    hipLaunchKernelGGL(k_sample<T>, dim3(unsigned(ceil_div(ns, kThreads / 64))),
+                       dim3(kThreads), 0, s->stream, a, nchunks, len, excl, inc, u + s0, ns,
+                       out + s0);
+    const int rc = launch_check("k_sample");
+    if (rc) return rc;
+  }
+  return 0;
+}
+
+template <typename T>
 static int sample_impl(qcs_hip_state *s, long shots, const double *u,
                        long *out) {
   typedef typename Amp<T>::type A;
@@ -1189,8 +1301,8 @@ static int sample_impl(qcs_hip_state *s, long shots, const double *u,
   TimedLaunch tl;
   timing_begin(s, QCS_HIP_K_REDUCE, double(s->size) * sizeof(A), 3.0 * s->size,
                &tl);
-  hipLaunchKernelGGL(k_chunk_tot<T>, dim3(unsigned(ceil_div(nchunks, kThreads / 64))),
-                     dim3(kThreads), 0, s->stream, a, nchunks, len, s->chunk_tot);
+  hipLaunchKernelGGL(k_chunk_tot<T>, dim3(unsigned(nchunks)), dim3(kThreads), 0, s->stream, a,
+                     len, s->chunk_tot);
   int rc = launch_check("k_chunk_tot");
   if (rc) return rc;
   if ((rc = timing_end(s, &tl))) return rc;
@@ -1198,16 +1310,9 @@ static int sample_impl(qcs_hip_state *s, long shots, const double *u,
                      s->chunk_tot, s->chunk_inc, nchunks);
   if ((rc = launch_check("k_chunk_scan"))) return rc;
   timing_begin(s, QCS_HIP_K_OTHER, double(shots) * len * sizeof(A), 0.0, &tl);
-  // one wave per shot; at most 2^24 shots per dispatch keeps the
-  // work-item count below 2^32
-  for (uint64_t s0 = 0; s0 < uint64_t(shots); s0 += uint64_t(1) << 24) {
-    const uint64_t ns = std::min<uint64_t>(uint64_t(shots) - s0, uint64_t(1) << 24);
-    hipLaunchKernelGGL(k_sample<T>, dim3(unsigned(ceil_div(ns, kThreads / 64))),
-                       dim3(kThreads), 0, s->stream, a, nchunks, len,
-                       s->chunk_tot, s->chunk_inc, s->u_dev + s0, ns,
-                       s->idx_dev + s0);
-    if ((rc = launch_check("k_sample"))) return rc;
-  }
+  if ((rc = launch_sample<T>(s, nchunks, len, s->chunk_tot, s->chunk_inc, shots, s->u_dev,
+                             s->idx_dev)))
+    return rc;
   if ((rc = timing_end(s, &tl))) return rc;
   QCS_HIP_TRY(hipMemcpyAsync(out, s->idx_dev, size_t(shots) * sizeof(long),
                              hipMemcpyDeviceToHost, s->stream));
@@ -1265,20 +1370,13 @@ static int sample_noalloc_impl(qcs_hip_state *s, double *scr, long shots,
   const uint64_t nchunks = s->size / len;
   double *tot = scr, *inc = scr + kNoAllocChunks;
   const A *a = static_cast<const A *>(s->vec);
-  hipLaunchKernelGGL(k_chunk_tot<T>, dim3(unsigned(ceil_div(nchunks, kThreads / 64))),
-                     dim3(kThreads), 0, s->stream, a, nchunks, len, tot);
+  hipLaunchKernelGGL(k_chunk_tot<T>, dim3(unsigned(nchunks)), dim3(kThreads), 0, s->stream, a,
+                     len, tot);
   int rc = launch_check("k_chunk_tot");
   if (rc) return rc;
   hipLaunchKernelGGL(k_chunk_scan, dim3(1), dim3(1024), 0, s->stream, tot, inc, nchunks);
   if ((rc = launch_check("k_chunk_scan"))) return rc;
-  for (uint64_t s0 = 0; s0 < uint64_t(shots); s0 += uint64_t(1) << 24) {
-    const uint64_t ns = std::min<uint64_t>(uint64_t(shots) - s0, uint64_t(1) << 24);
-    hipLaunchKernelGGL(k_sample<T>, dim3(unsigned(ceil_div(ns, kThreads / 64))),
-                       dim3(kThreads), 0, s->stream, a, nchunks, len, tot, inc,
-                       u_dev + s0, ns, idx_dev + s0);
-    if ((rc = launch_check("k_sample"))) return rc;
-  }
-  return 0;
+  return launch_sample<T>(s, nchunks, len, tot, inc, shots, u_dev, idx_dev);
 }
 
 int sample_noalloc(qcs_hip_state *s, long shots, const double *u_dev, long *idx_dev) {
