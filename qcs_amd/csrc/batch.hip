@@ -735,12 +735,23 @@ __device__ void sample_state(const P &prob, int n, double *tot, double *inc,
   const uint64_t N = uint64_t(1) << n;
   const uint64_t len = N < uint64_t(kChunk) ? N : uint64_t(kChunk);
   const uint64_t nch = N / len;
+  // U rows at a time: their loads and sums overlap, only the chain of their
+  // totals is sequential
+  constexpr int U = 8;
+  double x[U], t[U];
+  auto rows = [&](uint64_t base, uint64_t r) {
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+      x[k] = r + uint64_t(64 * k + lane) < len ? prob(base + r + uint64_t(64 * k + lane)) : 0.0;
+#pragma unroll
+    for (int k = 0; k < U; ++k) t[k] = wave_scan_total(x[k]);
+  };
   for (uint64_t ch = wave; ch < nch; ch += NW) {
     double running = 0.0;
-    for (uint64_t r = 0; r < len; r += 64) {
-      const double x = (r + lane < len) ? prob(ch * len + r + lane) : 0.0;
-      const double s = wave_incl_scan(x, lane);
-      running = running + __shfl(s, 63, 64);
+    for (uint64_t r = 0; r < len; r += 64 * U) {
+      rows(ch * len, r);
+#pragma unroll
+      for (int k = 0; k < U; ++k) running = running + t[k];
     }
     if (lane == 0) tot[ch] = running;
   }
@@ -769,22 +780,25 @@ __device__ void sample_state(const P &prob, int n, double *tot, double *inc,
     const uint64_t c = lo;
     const double e = tot[c];
     double running = 0.0;
-    long found = -1, last_nz = -1;
-    for (uint64_t r = 0; r < len; r += 64) {
-      const double x = (r + lane < len) ? prob(c * len + r + lane) : 0.0;
-      const double sc = wave_incl_scan(x, lane);
-      const double local = running + sc;
-      const double cdf = e + local;
-      const unsigned long long hit = __ballot(cdf > us && x > 0.0);
-      const unsigned long long nz = __ballot(x > 0.0);
-      if (nz) last_nz = long(c * len + r) + 63 - __clzll(nz);
-      if (hit) {
-        found = long(c * len + r) + __ffsll(hit) - 1;
-        break;
+    long found = -1;
+    for (uint64_t r = 0; r < len && found < 0; r += 64 * U) {
+      rows(c * len, r);
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        if (found < 0 && row_may_hit(t[k], e, running, us)) {
+          const unsigned long long hit = row_hits(x[k], lane, e, running, us);
+          if (hit) found = long(c * len + r) + 64 * k + __ffsll(hit) - 1;
+        }
+        running = running + t[k];
       }
-      running = running + __shfl(sc, 63, 64);
     }
-    if (found < 0) found = last_nz;
+    // only reachable at an ulp-level seam of the chunk scan: the last
+    // non-zero amplitude of the chunk
+    for (uint64_t r = (len + 63) & ~uint64_t(63); r > 0 && found < 0; r -= 64) {
+      const uint64_t i = r - 64 + lane;
+      const unsigned long long nz = __ballot((i < len ? prob(c * len + i) : 0.0) > 0.0);
+      if (nz) found = long(c * len + r) - 1 - __clzll(nz);
+    }
     if (lane == 0) out[s] = found;
   }
   __syncthreads();
@@ -955,7 +969,15 @@ __device__ void run_c64(const BCirc c, int part, int nparts, unsigned *sync, uns
   if (resident)
     for (int e = tid; e < tile; e += NTH) ns += norm2(L[e]);
   else
-    for (uint64_t i = tid; i < N; i += NTH) ns += norm2(G[i]);
+    // each thread's sum left to right, the loads ahead of it
+    for (uint64_t i = tid; i < N; i += 16 * NTH) {
+      float2 v[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k)
+        v[k] = i + uint64_t(k * NTH) < N ? G[i + uint64_t(k * NTH)] : make_float2(0.0f, 0.0f);
+#pragma unroll
+      for (int k = 0; k < 16; ++k) ns += norm2(v[k]);
+    }
   ns = wg_sum<NTH>(ns, red);
   if (ns > 1e-12 && ns != 1.0) {
     const double f = 1.0 / sqrt(ns);
@@ -967,11 +989,18 @@ __device__ void run_c64(const BCirc c, int part, int nparts, unsigned *sync, uns
         L[e] = x;
       }
     } else {
-      for (uint64_t i = tid; i < N; i += NTH) {
-        float2 x = G[i];
-        x.x = float(double(x.x) * f);
-        x.y = float(double(x.y) * f);
-        G[i] = x;
+      for (uint64_t i = tid; i < N; i += 16 * NTH) {
+        float2 v[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+          if (i + uint64_t(k * NTH) < N) v[k] = G[i + uint64_t(k * NTH)];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+          if (i + uint64_t(k * NTH) >= N) break;
+          v[k].x = float(double(v[k].x) * f);
+          v[k].y = float(double(v[k].y) * f);
+          G[i + uint64_t(k * NTH)] = v[k];
+        }
       }
     }
     __syncthreads();
