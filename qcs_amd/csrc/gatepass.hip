@@ -24,9 +24,16 @@
 // has mixed yet differs from the basis index; tiles of zeros are left alone
 // (28 qubits, H on every qubit and three layers: 21.5 -> 18.4 ms, with cheaper
 // addresses; the QFT of a basis state 15.4 -> 5.0 ms).
+// A SWAP of two bits outside the tile moves whole tiles: a work-group of two
+// halves reads a tile and the one it changes places with and stores each in
+// the other's place, so a bit reversal, which took four passes, takes one (28
+// qubits: the QFT's last gates and its 14 SWAPs 6.3 -> 3.7 ms).  Every pair has
+// one work-group: with one per tile and half of them leaving, the XCDs' shares
+// differed by 1.5 to 2 times (5.4 ms).
 #include <algorithm>
 #include <cmath>
 #include <exception>
+#include <iterator>
 #include <mutex>
 #include <vector>
 
@@ -280,22 +287,28 @@ __device__ __forceinline__ void p_op(int cls, Regs<T> &vr, Regs<T> &vi, const Pa
 }
 
 template <typename T>
-__global__ __launch_bounds__(1 << kPThrBits, 4) void k_gate_pass(
-    const PassProgram by_value, typename Amp<T>::type *a, uint64_t ntiles) {
+__global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
+    const PassProgram by_value, typename Amp<T>::type *a) {
   typedef typename Amp<T>::type A;
   // the first argument starts the kernel-argument segment
   const ProgramPtr prog = (ProgramPtr)__builtin_amdgcn_kernarg_segment_ptr();
-  const int tid = threadIdx.x;
   const int tb = int(prog->tb);
+  // With SWAPs of bits outside the tile a work-group takes a tile in its lower
+  // half and the one it changes places with in its upper: both are read before
+  // either is stored, in the other's place.  (A tile that stays where it is is
+  // taken by both halves, which store the same.)
+  const int half = prog->nswaps == 0
+                       ? 0
+                       : __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> (tb - kPRegBits));
+  const int tid = int(threadIdx.x) - (half << (tb - kPRegBits));
   // a tile of fewer than 1024 amplitudes still takes a whole wave, whose
   // lanes past the tile compute on copies and store nothing
   const bool in = tid < (1 << (tb - kPRegBits));
-  // amplitude index of the tile
-  uint64_t base = prog->fixed;
-  {
-    uint64_t t = xcd_order(blockIdx.x, ntiles);
-    for (uint64_t o = prog->outer; t; o &= o - 1, t >>= 1)
-      if (t & 1) base |= o & (~o + 1);
+  // amplitude index of the tile, and of the place it is stored in
+  uint64_t base = pass_tile(prog, xcd_order(blockIdx.x, gridDim.x)), home = base;
+  if (prog->nswaps != 0) {
+    const uint64_t other = pass_home(prog, base);
+    (half != 0 ? base : home) = other;
   }
   T vr[kPAmps], vi[kPAmps];
   {
@@ -379,9 +392,9 @@ __global__ __launch_bounds__(1 << kPThrBits, 4) void k_gate_pass(
     // exchange: written in this layout, through its index map, and read in
     // the next one
     const LayoutPtr nxt = (LayoutPtr)w;
-    const uint32_t tx = fresh(uint32_t(tid));
-    uint32_t ws = xor_lanes<kPThrBits>(tx, lay->thr) >> 16;
-    const uint32_t rs = xor_lanes<kPThrBits>(tx, nxt->thr) & 0xffffu;
+    const uint32_t tx = fresh(uint32_t(tid)), lds0 = uint32_t(half) << (tb + 3);
+    uint32_t ws = xor_lanes<kPThrBits>(tx, lay->thr) >> 16 | lds0;
+    const uint32_t rs = (xor_lanes<kPThrBits>(tx, nxt->thr) & 0xffffu) | lds0;
     for (uint32_t k = 0; k < lay->nterm; ++k) {
       const uint32_t t = lay->term[k];
       if ((base >> (t & 63)) & 1) ws ^= t >> 16;
@@ -431,7 +444,7 @@ __global__ __launch_bounds__(1 << kPThrBits, 4) void k_gate_pass(
     __syncthreads();
   }
   if (!in) return;
-  uint64_t i0 = base ^ xor_lanes<kPThrBits>(fresh(uint32_t(tid)), prog->store_t);
+  uint64_t i0 = home ^ xor_lanes<kPThrBits>(fresh(uint32_t(tid)), prog->store_t);
   for (uint32_t k = 0; k < prog->store_nterm; ++k)
     if ((base >> prog->store_q[k]) & 1) i0 ^= prog->store_term[k];
   auto amp = [&](int j) {
@@ -514,20 +527,21 @@ static int launch_pass(qcs_hip_state *s, const PassPick &pick,
   typedef typename Amp<T>::type A;
   PassProgram prog;
   write_pass<T>(s->queue, pick, groups, s->n, tb, s->support, s->basis, &prog, s->filled);
-  const uint64_t ntiles = uint64_t(1) << __builtin_popcountll(prog.outer);
-  const int threads = std::max(64, 1 << (tb - kPRegBits));
-  const size_t lds = prog.nlayouts > 1 ? size_t(8) << tb : 0;
+  const int outer_bits = __builtin_popcountll(prog.outer);
+  const int halves = prog.nswaps > 0 ? 2 : 1;
+  const int threads = std::max(64, halves << (tb - kPRegBits));
+  const size_t lds = prog.nlayouts > 1 ? size_t(8 * halves) << tb : 0;
   TimedLaunch tl;
-  const double amps = double(ntiles << tb);
+  const double amps = double(uint64_t(1) << (outer_bits + 2 * int(prog.nswaps) + tb));
   const double read = amps / double(uint64_t(1) << __builtin_popcountll(prog.skip_t | prog.skip_r));
   timing_begin(s, QCS_HIP_K_FUSED, (amps + read) * sizeof(A),
                6.0 * amps * double(pick.gates.size()), &tl);
-  hipLaunchKernelGGL(k_gate_pass<T>, dim3(unsigned(ntiles)), dim3(unsigned(threads)), lds,
-                     s->stream, prog, static_cast<A *>(s->vec), ntiles);
+  hipLaunchKernelGGL(k_gate_pass<T>, dim3(unsigned(pass_work_groups(&prog, outer_bits))),
+                     dim3(unsigned(threads)), lds, s->stream, prog, static_cast<A *>(s->vec));
   int rc = launch_check("k_gate_pass");
   if (rc) return rc;
   if (s->filled != ~uint64_t(0)) {
-    s->filled |= pick.bits;
+    s->filled |= pick.bits | pick.swapped;
     if ((~s->filled & (s->size - 1)) == 0) s->filled = ~uint64_t(0);
   }
   return timing_end(s, &tl);
@@ -539,19 +553,23 @@ static int run_queue(qcs_hip_state *s, bool all) {
   std::vector<PlanGate> &q = s->queue;
   PassPick pick;
   std::vector<PassGroup> groups;
+  std::vector<int> taken;  // the pick's gates and SWAPs
   int rc = 0;
   const int tb = pass_tile_bits(s->n);
   const int words = s->precision == QCS_HIP_C128 ? 2 : 1;
   while (!q.empty() && (all || q.size() >= kQueueLow)) {
-    plan_pick(q, s->n, tb, kPassLowBits, words, 64, &pick, &groups);
+    plan_pick(q, s->n, tb, kPassLowBits, words, 64, &pick, &groups, s->n > tb);
     if (!all && !pick.full && q.size() < kQueueMax) break;
+    taken.clear();
+    std::merge(pick.gates.begin(), pick.gates.end(), pick.swaps.begin(), pick.swaps.end(),
+               std::back_inserter(taken));
     double traffic = 0.0;
-    for (int i : pick.gates) traffic += plan_gate_traffic(q[size_t(i)]);
-    if (pick.gates.size() <= 1 || (s->n >= kPassBigState && traffic <= 2.0)) {
+    for (int i : taken) traffic += plan_gate_traffic(q[size_t(i)]);
+    if (taken.size() <= 1 || (s->n >= kPassBigState && traffic <= 2.0)) {
       // the per-gate kernels move no more than the pass would
-      if (pick.gates.empty()) pick.gates.push_back(0);
+      if (taken.empty()) taken.push_back(0);
       rc = launch_fill_rest(s);
-      for (int i : pick.gates) {
+      for (int i : taken) {
         if (rc) break;
         const PlanGate &g = q[size_t(i)];
         const int kind = g.cls == kGSwap ? QCS_HIP_G_SWAP : g.c >= 0 ? QCS_HIP_G_CU : QCS_HIP_G_1Q;
@@ -565,10 +583,10 @@ static int run_queue(qcs_hip_state *s, bool all) {
       q.clear();  // the state is no longer what the rest would act on
       break;
     }
-    for (int i : pick.gates) s->support |= plan_spread(q[size_t(i)]);
+    for (int i : taken) s->support |= plan_spread(q[size_t(i)]);
     size_t keep = 0, x = 0;
     for (size_t i = 0; i < q.size(); ++i) {
-      if (x < pick.gates.size() && size_t(pick.gates[x]) == i) ++x;
+      if (x < taken.size() && size_t(taken[x]) == i) ++x;
       else q[keep++] = q[i];
     }
     q.resize(keep);

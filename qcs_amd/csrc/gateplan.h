@@ -32,6 +32,7 @@ constexpr int kPAmps = 1 << kPRegBits;     // amplitudes per thread
 constexpr int kPMaxTile = 13;              // tile bits: 512 threads x 16
 constexpr int kPThrBits = kPMaxTile - kPRegBits;
 constexpr int kPLineBits = 3;              // 8 amplitudes: a 128-byte line (complex128)
+constexpr int kPMaxSwaps = 16;             // SWAPs of two bits outside the tile per pass
 constexpr int kPMaxTerms = 6;              // controls outside the tile per exchange
 constexpr int kPWords = 848;               // program words of a pass
 constexpr int kPPad = 17;                  // words read past the last op
@@ -82,8 +83,8 @@ constexpr int kPLayoutWords = int(sizeof(PassLayout) / 4);
 struct PassProgram {
   uint32_t tb;
   uint32_t nlayouts;
-  // Tiles: number t has its bits at the set bits of `outer` (ascending), and
-  // `fixed` elsewhere outside the tile.
+  // Tiles: number t has its bits at the set bits of `outer` (ascending) and on
+  // the bits of `swaps`, and `fixed` elsewhere outside the tile (pass_tile).
   uint64_t outer, fixed;
   // Amplitudes of the tile that are zero without being so in memory: where
   // the index differs from `basis` in a bit of skip_t (thread bits) or skip_r
@@ -93,11 +94,59 @@ struct PassProgram {
   uint64_t store_t[kPThrBits], store_r[kPRegBits];  // index masks (XOR) of the last layout
   uint64_t store_term[kPMaxTerms];                  // XOR where index bit store_q is set
   uint32_t store_q[kPMaxTerms];
+  // SWAPs of two index bits outside the tile (pairs of tiles change places)
+  uint32_t nswaps, swaps[kPMaxSwaps];  // low bit | high bit << 8
   uint32_t store_nterm;
   uint32_t store_add;  // the registers' masks share no bit with others: XOR is addition
   uint32_t words[kPWords + kPPad];
 };
 static_assert(sizeof(PassProgram) <= 4096 - 16, "a pass program travels as a kernel argument");
+
+// Work-groups of a pass.  Without SWAPs outside the tile each takes a tile.
+// With p of them it takes a tile and the one it changes places with, and there
+// is one for each such pair: numbered, above the bits of `outer`, by the first
+// SWAP whose two bits differ (of the pair, the tile with its low bit set is
+// the work-group's first), the equal bits of the SWAPs before it and any bits
+// of those after it; last come the tiles that stay where they are.
+// (constexpr: host and device code)
+template <typename P>
+constexpr uint64_t pass_work_groups(const P prog, int outer_bits) {
+  const int p = int(prog->nswaps);
+  uint64_t g = uint64_t(1) << p;
+  for (int k = 0; k < p; ++k) g += uint64_t(1) << (2 * p - 2 - k);
+  return g << outer_bits;
+}
+template <typename P>
+constexpr uint64_t pass_tile(const P prog, uint64_t t) {
+  uint64_t base = prog->fixed;
+  for (uint64_t o = prog->outer; o; o &= o - 1, t >>= 1)
+    if (t & 1) base |= o & (~o + 1);
+  const int p = int(prog->nswaps);
+  int first = 0;
+  for (; first < p; ++first) {
+    const uint64_t count = uint64_t(1) << (2 * p - 2 - first);
+    if (t < count) break;
+    t -= count;
+  }
+  for (int k = 0; k < p; ++k) {
+    const uint32_t lo = prog->swaps[k] & 255, hi = prog->swaps[k] >> 8;
+    uint64_t bits = 1;  // low bit, then high bit
+    if (k < first) bits = (t & 1) * 3, t >>= 1;
+    else if (k > first) bits = t & 3, t >>= 2;
+    base |= (bits & 1) << lo | bits >> 1 << hi;
+  }
+  return base;
+}
+// where the tile is stored
+template <typename P>
+constexpr uint64_t pass_home(const P prog, uint64_t base) {
+  for (uint32_t k = 0; k < prog->nswaps; ++k) {
+    const uint32_t lo = prog->swaps[k] & 255, hi = prog->swaps[k] >> 8;
+    const uint64_t d = (base >> lo ^ base >> hi) & 1;
+    base ^= d << lo | d << hi;
+  }
+  return base;
+}
 
 // XOR swizzle of an LDS slot (8 bytes): bits 5.. fold onto the low five, so
 // that 32 lanes whose positions have independent vectors use 32 slots that
@@ -191,6 +240,8 @@ struct PassPick {
   std::vector<int> gates;  // indices, in the order they run
   uint64_t bits;           // tile bits
   bool full;               // the next gate does not fit: more gates would not change the pick
+  std::vector<int> swaps;  // SWAPs of two qubits outside the tile, after the others
+  uint64_t swapped;        // their qubits
 };
 
 // One group: ops on at most kPRegBits register qubits, then index maps.
@@ -239,9 +290,13 @@ inline bool plan_add(std::vector<PassGroup> &gs, const std::vector<PlanGate> &ga
 
 // The gates of the next pass: in order, each that fits the tile and may run
 // before the ones left behind.  `scan` bounds how far past the first gate
-// left behind the list is searched for gates that may overtake it.
+// left behind the list is searched for gates that may overtake it.  With
+// `pairs`, a SWAP of two qubits outside the tile needs no tile bits: the pass
+// stores the tiles it relates in each other's place, and leaves later gates on
+// its qubits behind.
 inline void plan_pick(const std::vector<PlanGate> &gates, int n, int tb, int low,
-                      int param_words, int scan, PassPick *out, std::vector<PassGroup> *groups) {
+                      int param_words, int scan, PassPick *out, std::vector<PassGroup> *groups,
+                      bool pairs = false) {
   uint64_t tile = (uint64_t(1) << (low < n ? low : n)) - 1;
   if (tb >= n) tile = (uint64_t(1) << n) - 1;
   uint64_t left = 0;  // qubits of the gates left behind
@@ -249,12 +304,20 @@ inline void plan_pick(const std::vector<PlanGate> &gates, int n, int tb, int low
   int words = 0, past = 0;
   out->gates.clear();
   out->full = false;
+  out->swaps.clear();
+  out->swapped = 0;
   groups->clear();
   // the layouts of the load and the store besides the groups'
   const int budget = kPWords - 2 * kPLayoutWords;
   for (size_t i = 0; i < gates.size(); ++i) {
     const PlanGate &g = gates[i];
-    bool take = !(g.qubits & left) && (g.exact || !left_inexact);
+    bool take = !(g.qubits & (left | out->swapped)) && (g.exact || !left_inexact);
+    if (take && pairs && g.cls == kGSwap && !(g.qubits & tile) &&
+        int(out->swaps.size()) < kPMaxSwaps) {
+      out->swaps.push_back(int(i));
+      out->swapped |= g.qubits;
+      continue;
+    }
     if (take) {
       const int w = words + plan_op_words(g, param_words);
       const int room = budget - w - int(groups->size()) * kPLayoutWords;
@@ -275,7 +338,12 @@ inline void plan_pick(const std::vector<PlanGate> &gates, int n, int tb, int low
   }
   out->full = left_inexact;
   // fill the tile with the lowest unused bits (longer runs)
-  for (int q = 0; q < n && __builtin_popcountll(tile) < tb; ++q) tile |= uint64_t(1) << q;
+  for (int q = 0; q < n && __builtin_popcountll(tile) < tb; ++q)
+    tile |= (uint64_t(1) << q) & ~out->swapped;
+  if (__builtin_popcountll(tile) < (tb < n ? tb : n)) {  // the swapped qubits have to fill it
+    plan_pick(gates, n, tb, low, param_words, scan, out, groups, false);
+    return;
+  }
   out->bits = tile;
   // groups, with the final tile
   size_t used = 0;
@@ -292,7 +360,14 @@ inline void plan_pick(const std::vector<PlanGate> &gates, int n, int tb, int low
   // gates that no longer fit: only the ones before them in the run order go.
   // The rest stay in the list in their order; what was taken ran before them
   // legally, since it ran before them in `gates` order of the pick as well.
+  // A SWAP set aside may have followed one of them.
+  while (used < out->gates.size() && !out->swaps.empty() &&
+         out->swaps.back() > out->gates[used]) {
+    out->swapped &= ~gates[size_t(out->swaps.back())].qubits;
+    out->swaps.pop_back();
+  }
   out->gates.resize(used);
+  if (groups->empty()) groups->emplace_back();
 }
 
 // ---- writing the program ---------------------------------------------------
@@ -481,7 +556,13 @@ inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
   pp->tb = uint32_t(tb);
   const uint64_t all = n < 64 ? (uint64_t(1) << n) - 1 : ~uint64_t(0);
   if (~filled & all) support = filled;
-  pp->outer = support & all & ~pick.bits;
+  support |= pick.swapped;
+  pp->nswaps = uint32_t(pick.swaps.size());
+  for (size_t k = 0; k < pick.swaps.size(); ++k) {
+    const PlanGate &g = gates[size_t(pick.swaps[k])];
+    pp->swaps[k] = uint32_t(g.t) | uint32_t(g.c) << 8;
+  }
+  pp->outer = support & all & ~(pick.bits | pick.swapped);
   pp->fixed = basis & all & ~(support | pick.bits);
   int pos[64], bits[kPMaxTile];
   for (int &p : pos) p = -1;
@@ -530,6 +611,7 @@ inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
   for (int b = 0; b < first.m.nthr; ++b) pp->load_t[b] = index_mask(1 << first.m.thr[b]);
   for (int b = 0; b < kPRegBits; ++b) pp->load_r[b] = index_mask(1 << first.m.reg[b]);
   for (uint64_t m : pp->load_t) pp->skip_t |= m & ~filled;
+  pp->skip_t |= pick.swapped & ~filled;  // (whole tiles)
   for (uint64_t m : pp->load_r) pp->skip_r |= m & ~filled;
   pp->basis = basis;
   for (int b = 0; b < last.m.nthr; ++b) pp->store_t[b] = index_mask(last.a.col[last.m.thr[b]]);

@@ -6,6 +6,7 @@
 // value for value, with the same gates applied one after another by the
 // per-gate arithmetic.  Every LDS slot and every amplitude index is checked
 // for range, and every exchange and every pass for being a permutation.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 
@@ -21,6 +22,8 @@ static uint64_t rnd() {
   return z ^ (z >> 31);
 }
 static double uni() { return double(rnd() >> 11) / 9007199254740992.0; }
+
+static long swaps_set_aside;
 
 static void fail(const char *what) {
   std::printf("FAIL: %s\n", what);
@@ -145,13 +148,19 @@ template <typename T>
 static void run_pass(Vec<T> &v, int n, const PassProgram &pp, uint64_t filled) {
   const int tb = int(pp.tb), nthr = 1 << (tb - kPRegBits);
   const uint64_t N = uint64_t(1) << n;
-  const uint64_t ntiles = uint64_t(1) << __builtin_popcountll(pp.outer);
+  // the work-groups' tiles: with SWAPs outside the tile, pairs that change
+  // places and tiles that stay
+  std::vector<uint64_t> tiles;
+  const uint64_t work_groups = pass_work_groups(&pp, __builtin_popcountll(pp.outer));
+  for (uint64_t g = 0; g < work_groups; ++g) {
+    const uint64_t first = pass_tile(&pp, g), other = pass_home(&pp, first);
+    if (pass_home(&pp, other) != first) fail("a pair of tiles");
+    tiles.push_back(first);
+    if (other != first) tiles.push_back(other);
+  }
   std::vector<char> touched(N, 0), stored(N, 0);
   Vec<T> out = v;
-  for (uint64_t tile = 0; tile < ntiles; ++tile) {
-    uint64_t base = pp.fixed, t = tile;
-    for (uint64_t o = pp.outer; t; o &= o - 1, t >>= 1)
-      if (t & 1) base |= o & (~o + 1);
+  for (const uint64_t base : tiles) {
     std::vector<T> vr(size_t(nthr) * kPAmps), vi(vr.size());
     for (int t = 0; t < nthr; ++t)
       for (int j = 0; j < kPAmps; ++j) {
@@ -233,7 +242,17 @@ static void run_pass(Vec<T> &v, int n, const PassProgram &pp, uint64_t filled) {
       }
     }
     if (w - pp.words > kPWords) fail("program length");
-    uint64_t b2 = base;
+    uint64_t b2 = base, used = 0;
+    for (uint32_t k = 0; k < pp.nswaps; ++k) {
+      // distinct bits outside the tile: the tiles change places in pairs
+      const uint32_t lo = pp.swaps[k] & 255, hi = pp.swaps[k] >> 8;
+      const uint64_t both = uint64_t(1) << lo | uint64_t(1) << hi;
+      if (lo == hi || (both & used) || (both & pp.outer) || (base >> lo ^ b2 >> lo) & 1)
+        fail("swapped bits");
+      used |= both;
+      const uint64_t d = (b2 >> lo ^ b2 >> hi) & 1;
+      b2 ^= d << lo | d << hi;
+    }
     for (uint32_t k = 0; k < pp.store_nterm; ++k)
       if ((base >> pp.store_q[k]) & 1) b2 ^= pp.store_term[k];
     for (int t = 0; t < nthr; ++t)
@@ -256,7 +275,7 @@ static void run_pass(Vec<T> &v, int n, const PassProgram &pp, uint64_t filled) {
 }
 
 template <typename T>
-static int check(int n, int tb, int low, int count, int style, bool basis_state, bool unfilled) {
+static int check(int n, int tb, int low, int count, int style, bool basis_state, bool unfilled, bool pairs) {
   const uint64_t N = uint64_t(1) << n;
   std::vector<Gate> gates;
   std::vector<PlanGate> q;
@@ -267,10 +286,12 @@ static int check(int n, int tb, int low, int count, int style, bool basis_state,
     g.c = int(rnd() % uint64_t(n - 1));
     if (g.c >= g.t) ++g.c;
     const double a = 6.283185307179586 * uni(), c = std::cos(a / 2), s = std::sin(a / 2);
-    // style 0: every kind; 1: rotations and CNOTs; 2: H and controlled phases
+    // style 0: every kind; 1: rotations and CNOTs; 2: H and controlled phases;
+    // 3: mostly SWAPs
     int k = int(rnd() % 13);
     if (style == 1) k = k < 8 ? 6 + k % 2 : 9;
     if (style == 2) k = k < 3 ? 0 : k < 11 ? 10 : 11;
+    if (style == 3) k = k < 2 ? 0 : k < 4 ? 9 : k < 6 ? 10 : 11;
     if (style == 1 && k == 7 && x + 3 <= count) {  // RZ RY RZ
       for (int y = 0; y < 3; ++y) {
         Gate z;
@@ -330,17 +351,22 @@ static int check(int n, int tb, int low, int count, int style, bool basis_state,
   std::vector<PassGroup> groups;
   static PassProgram pp;
   while (!q.empty()) {
-    plan_pick(q, n, tb, low, int(sizeof(T) / 4), 64, &pick, &groups);
-    if (pick.gates.empty()) fail("a pass without gates");
+    plan_pick(q, n, tb, low, int(sizeof(T) / 4), 64, &pick, &groups, pairs);
+    if (!pairs && !pick.swaps.empty()) fail("swaps");
+    std::vector<int> taken = pick.gates;
+    taken.insert(taken.end(), pick.swaps.begin(), pick.swaps.end());
+    std::sort(taken.begin(), taken.end());
+    if (taken.empty()) fail("a pass without gates");
     if (__builtin_popcountll(pick.bits) != tb) fail("tile bits");
     write_pass<T>(q, pick, groups, n, tb, support, basis, &pp, filled);
     run_pass<T>(b, n, pp, filled);
-    filled |= pick.bits;
-    for (int i : pick.gates) support |= plan_spread(q[size_t(i)]);
+    filled |= pick.bits | pick.swapped;
+    swaps_set_aside += long(pick.swaps.size());
+    for (int i : taken) support |= plan_spread(q[size_t(i)]);
     std::vector<PlanGate> rest;
     size_t x = 0;
     for (size_t i = 0; i < q.size(); ++i) {
-      if (x < pick.gates.size() && size_t(pick.gates[x]) == i) ++x;
+      if (x < taken.size() && size_t(taken[x]) == i) ++x;
       else rest.push_back(q[i]);
     }
     q.swap(rest);
@@ -359,18 +385,19 @@ static int check(int n, int tb, int low, int count, int style, bool basis_state,
 int main() {
   rng_state = 12345;
   long total = 0;
-  for (int n = 7; n <= 15; ++n)
-    for (int style = 0; style < 3; ++style)
-      for (int rep = 0; rep < 4; ++rep) {
+  for (int n = 7; n <= 14; ++n)
+    for (int style = 0; style < 4; ++style)
+      for (int rep = 0; rep < 6; ++rep) {
         // the whole state in a tile, then tiles smaller than it
         for (int tb = n < kPMaxTile ? n : kPMaxTile; tb >= 7 && tb >= n - 5; tb -= 2)
           for (int low = 3; low <= 4; ++low) {
             if (tb < n && tb < low + 4) continue;
             const int count = 20 + int(rnd() % 200);
-            total += check<double>(n, tb, low, count, style, rep > 0, rep > 1);
-            total += check<float>(n, tb, low, count, style, rep > 0, rep > 1);
+            total += check<double>(n, tb, low, count, style, rep % 3 > 0, rep % 3 > 1, rep > 2);
+            total += check<float>(n, tb, low, count, style, rep % 3 > 0, rep % 3 > 1, rep > 2);
           }
       }
+  if (swaps_set_aside < 100) fail("no pass moved its tiles");
   std::printf("ok %ld passes\n", total);
   return 0;
 }

@@ -109,3 +109,41 @@ def test_values_that_could_overflow_take_the_per_gate_kernels(qlib):
                 if each:
                     c.flush()
         assert np.array_equal(a.amplitudes(), b.amplitudes(), equal_nan=True)
+
+
+@pytest.mark.parametrize("option", [qcs_amd.PLAIN_FP64, qcs_amd.PLAIN_FP32])
+@pytest.mark.parametrize("n", [14, 15, 18, 23])
+def test_swaps_of_qubits_outside_the_tile(qlib, n, option):
+    """Passes that store their tiles in each other's place: from a basis state
+    and from any state, against the gates launched one by one."""
+    rng = np.random.default_rng(n)
+    start = rng.normal(size=1 << n) + 1j * rng.normal(size=1 << n)
+    start /= np.linalg.norm(start)
+    for rep in range(6):
+        ops = C.Ops()
+        for _ in range(40):
+            k, t = rng.integers(0, 8), int(rng.integers(0, n))
+            c = int((t + rng.integers(1, n)) % n)
+            if k < 5:
+                ops.add(C.SWAP, t, c)
+            elif k == 5:
+                ops.add(C.H, t)
+            elif k == 6:
+                ops.add(C.CNOT, t, c)
+            else:
+                ops.add(C.CPHASE, t, c, float(rng.uniform(-3, 3)))
+        if rep == 0:  # a bit reversal
+            ops = C.Ops()
+            for q in range(n // 2):
+                ops.add(C.SWAP, q, n - 1 - q)
+        with qcs_amd.Circuit(n, option) as a, qcs_amd.Circuit(n, option) as b:
+            for c in (a, b):
+                if rep < 4:
+                    c.set_amplitudes(start)
+                else:
+                    c.set_basis_state(rep * 1234 % (1 << n))
+            a.apply(ops)
+            for op, t, c, p in zip(ops.op, ops.tq, ops.cq, ops.par):
+                b.apply(C.Ops().add(op, t, c, p))
+                b.lib.qc_flush(b.handle)
+            assert np.array_equal(a.amplitudes(), b.amplitudes()), rep
