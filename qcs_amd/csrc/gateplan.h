@@ -53,20 +53,29 @@ struct PlanGate {
 };
 
 // Program of a pass: layout records, each followed by its ops.
-// Op word: kind | cond1 << 8 | cond2 << 16 | words of the op << 24, then the
-// parameters in the state's precision.
+// Op word: kind | words of the op << 5 | u1 << 10 | u2 << 16 | l1 << 22 |
+// l2 << 25, then the parameters in the state's precision.  Conditions: bits
+// u1, u2 of the wave's uniform word (pass_uniform) and lane bits l1, l2 have to
+// be set.
 enum : uint8_t {
   kPDense = 0,     // + register bit: m[0..7]
   kPReal = 4,      // m00, m01, m10, m11 (real parts)
   kPAnti = 8,      // m01, m10
   kPDiag = 12,     // m00, m11
-  kPPhase = 16,    // m11; under conditions where cond1 / cond2 say so
+  kPPhase = 16,    // m11; under conditions
   kPEuler = 20,    // diag(a, conj a), [[c, -s], [s, c]], diag(b, conj b)
   kPCPhase = 24,   // + pair index of two register bits: m11
-  kPScale = 30,    // every amplitude, where cond1 and cond2 hold: m11
-  kPSelect = 31    // every amplitude: cond1 ? m11 : m00
+  kPScale = 30,    // every amplitude, under conditions: m11
+  kPSelect = 31    // every amplitude: conditions ? m11 : m00
 };
-// condition byte: thread bit b (< 16), or 64 + an index bit outside the tile
+// What a whole wave shares: the index bits outside the tile, above them the
+// thread bits past the lane's, and a bit that is always set.
+constexpr int kPLaneBits = 6, kPWaveBit = 40, kPAlways = 63;
+constexpr int kPNoLane = 7;
+constexpr uint64_t pass_uniform(uint64_t base, unsigned wave) {
+  return base | uint64_t(wave) << kPWaveBit | uint64_t(1) << kPAlways;
+}
+// condition: lane bit b, or 64 + a bit of the uniform word
 constexpr int kPNoCond = 255;
 
 // Layout record, in whole words (scalar loads are 32 bits and up).  A pair
@@ -482,7 +491,13 @@ inline IndexMap make_map(const std::vector<PlanGate> &gates, const std::vector<i
 template <typename T>
 inline void put_op(uint32_t *&w, int kind, int c1, int c2, const T *par, int npar) {
   const int words = 1 + npar * int(sizeof(T) / 4);
-  *w++ = uint32_t(kind) | uint32_t(c1) << 8 | uint32_t(c2) << 16 | uint32_t(words) << 24;
+  int u[2] = {kPAlways, kPAlways}, l[2] = {kPNoLane, kPNoLane}, nu = 0, nl = 0;
+  for (int c : {c1, c2}) {
+    if (c == kPNoCond) continue;
+    if (c < 64) l[nl++] = c;
+    else u[nu++] = c - 64;
+  }
+  *w++ = uint32_t(kind | words << 5 | u[0] << 10 | u[1] << 16 | l[0] << 22 | l[1] << 25);
   std::memcpy(w, par, size_t(npar) * sizeof(T));
   w += words - 1;
 }
@@ -492,7 +507,9 @@ template <typename T>
 inline void write_ops(const std::vector<PlanGate> &gates, const std::vector<int> &ops,
                       const LayoutMap &m, const int *pos, uint64_t tile, uint32_t *&w) {
   auto cond = [&](int q) {
-    return ((tile >> q) & 1) ? m.thread_bit(pos[q]) : 64 + q;
+    if (!((tile >> q) & 1)) return 64 + q;
+    const int b = m.thread_bit(pos[q]);
+    return b < kPLaneBits ? b : 64 + kPWaveBit + b - kPLaneBits;
   };
   auto reg = [&](int q) { return ((tile >> q) & 1) ? m.reg_bit(pos[q]) : -1; };
   for (size_t x = 0; x < ops.size(); ++x) {

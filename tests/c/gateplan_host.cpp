@@ -184,18 +184,23 @@ static void run_pass(Vec<T> &v, int n, const PassProgram &pp, uint64_t filled) {
       while (w < end) {
         const uint32_t h = w[0];
         const uint32_t *pw = w + 1;
-        w += h >> 24;
-        const int kind = int(h & 255), c1 = int((h >> 8) & 255), c2 = int((h >> 16) & 255);
-        if ((h >> 24) == 0 || w > end) fail("op length");
+        w += (h >> 5) & 31;
+        const int kind = int(h & 31);
+        if (((h >> 5) & 31) == 0 || w > end) fail("op length");
         for (int t = 0; t < nthr; ++t) {
           T *r = &vr[size_t(t) * kPAmps], *s = &vi[size_t(t) * kPAmps];
-          auto cond = [&](int c) {
-            if (c == kPNoCond) return true;
-            if (c >= 64 && c - 64 >= n) fail("condition");
-            if (c < 64 && c >= tb - kPRegBits) fail("condition");
-            return c < 64 ? ((t >> c) & 1) != 0 : ((base >> (c - 64)) & 1) != 0;
-          };
-          const bool on = cond(c1) && cond(c2);
+          const uint64_t uni = pass_uniform(base, unsigned(t >> kPLaneBits));
+          bool on = true;
+          for (int c : {int(h >> 10) & 63, int(h >> 16) & 63}) {
+            const bool wave = c >= kPWaveBit && c - kPWaveBit < tb - kPRegBits - kPLaneBits;
+            if (c != kPAlways && c >= n && !wave) fail("condition");
+            on = on && ((uni >> c) & 1);
+          }
+          for (int c : {int(h >> 22) & 7, int(h >> 25) & 7}) {
+            if (c == kPNoLane) continue;
+            if (c >= kPLaneBits || c >= tb - kPRegBits) fail("condition");
+            on = on && ((t >> c) & 1);
+          }
           if (kind < kPCPhase) {
             op1<T>(kind & ~3, r, s, kind & 3, pw, on);
             continue;
