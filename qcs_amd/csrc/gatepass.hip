@@ -11,8 +11,8 @@
 // from 270 to 20 ms.
 //
 // k_gate_pass.  One work-group per tile of 2^tb amplitudes; thread t holds 16
-// of them in registers, those that differ in the layout's four register
-// bits.  A layout change exchanges the tile through LDS, complex128 as two
+// (small states: 4) of them in registers, those that differ in the layout's
+// register bits.  A layout change exchanges the tile through LDS, complex128 as two
 // planes (all real parts, then all imaginary parts), so a 12-bit tile takes
 // 32 KiB: four work-groups of 256 threads fit a CU (128 registers a thread),
 // and one computes while another waits for HBM.  The arithmetic is that of gates.hip without the
@@ -48,9 +48,6 @@ namespace qcs {
 // vr[j], vi[j]: the amplitude whose register bits are the bits of j.  Every
 // index is a compile-time constant.
 
-template <typename T>
-using Regs = T[kPAmps];
-
 // Every product of a pair is formed before any sum: each result is then
 // defined after the last use of the inputs and takes an input's register, so
 // every op leaves each amplitude in the register it came in and the joins
@@ -59,10 +56,10 @@ using Regs = T[kPAmps];
 // waves a SIMD holds leave.
 __device__ __forceinline__ void pair_end() { __builtin_amdgcn_sched_barrier(0); }
 
-template <int Q, typename T>
-__device__ __forceinline__ void p_dense(Regs<T> &vr, Regs<T> &vi, const T (&m)[8]) {
+template <int Q, typename T, int N>
+__device__ __forceinline__ void p_dense(T (&vr)[N], T (&vi)[N], const T (&m)[8]) {
 #pragma unroll
-  for (int j = 0; j < kPAmps; ++j) {
+  for (int j = 0; j < N; ++j) {
     if (j & (1 << Q)) continue;
     const int k = j | (1 << Q);
     const T x0 = vr[j], y0 = vi[j], x1 = vr[k], y1 = vi[k];
@@ -79,10 +76,10 @@ __device__ __forceinline__ void p_dense(Regs<T> &vr, Regs<T> &vi, const T (&m)[8
 }
 
 // every imaginary part 0: {m00, m01, m10, m11}
-template <int Q, typename T>
-__device__ __forceinline__ void p_real(Regs<T> &vr, Regs<T> &vi, T m00, T m01, T m10, T m11) {
+template <int Q, typename T, int N>
+__device__ __forceinline__ void p_real(T (&vr)[N], T (&vi)[N], T m00, T m01, T m10, T m11) {
 #pragma unroll
-  for (int j = 0; j < kPAmps; ++j) {
+  for (int j = 0; j < N; ++j) {
     if (j & (1 << Q)) continue;
     const int k = j | (1 << Q);
     const T x0 = vr[j], y0 = vi[j], x1 = vr[k], y1 = vi[k];
@@ -97,10 +94,10 @@ __device__ __forceinline__ void p_real(Regs<T> &vr, Regs<T> &vi, T m00, T m01, T
 }
 
 // zero diagonal: out0 = (ar, ai) v1, out1 = (br, bi) v0
-template <int Q, typename T>
-__device__ __forceinline__ void p_anti(Regs<T> &vr, Regs<T> &vi, T ar, T ai, T br, T bi) {
+template <int Q, typename T, int N>
+__device__ __forceinline__ void p_anti(T (&vr)[N], T (&vi)[N], T ar, T ai, T br, T bi) {
 #pragma unroll
-  for (int j = 0; j < kPAmps; ++j) {
+  for (int j = 0; j < N; ++j) {
     if (j & (1 << Q)) continue;
     const int k = j | (1 << Q);
     const T x0 = vr[j], y0 = vi[j], x1 = vr[k], y1 = vi[k];
@@ -122,10 +119,10 @@ __device__ __forceinline__ void p_scale(T &vr, T &vi, T ar, T ai) {
 }
 
 // the amplitudes whose register bits include those of SET, times (ar, ai)
-template <int SET, typename T>
-__device__ __forceinline__ void p_phase(Regs<T> &vr, Regs<T> &vi, T ar, T ai) {
+template <int SET, typename T, int N>
+__device__ __forceinline__ void p_phase(T (&vr)[N], T (&vi)[N], T ar, T ai) {
 #pragma unroll
-  for (int j = 0; j < kPAmps; ++j) {
+  for (int j = 0; j < N; ++j) {
     if ((j & SET) == SET) {
       p_scale(vr[j], vi[j], ar, ai);
       if (j & 1) pair_end();
@@ -138,10 +135,10 @@ __device__ __forceinline__ void p_phase(Regs<T> &vr, Regs<T> &vi, T ar, T ai) {
   }
 }
 
-template <int Q, typename T>
-__device__ __forceinline__ void p_diag(Regs<T> &vr, Regs<T> &vi, T ar, T ai, T br, T bi) {
+template <int Q, typename T, int N>
+__device__ __forceinline__ void p_diag(T (&vr)[N], T (&vi)[N], T ar, T ai, T br, T bi) {
 #pragma unroll
-  for (int j = 0; j < kPAmps; ++j) {
+  for (int j = 0; j < N; ++j) {
     if (j & (1 << Q)) continue;
     const int k = j | (1 << Q);
     p_scale(vr[j], vi[j], ar, ai);
@@ -153,11 +150,11 @@ __device__ __forceinline__ void p_diag(Regs<T> &vr, Regs<T> &vi, T ar, T ai, T b
 // diag(ar + i ai, conj), [[c, s], [-s, c]], diag(br + i bi, conj), one after
 // the other: the products of the three gates, whose other entries are copies
 // and negations of these
-template <int Q, typename T>
-__device__ __forceinline__ void p_euler(Regs<T> &vr, Regs<T> &vi, T ar, T ai, T c, T s, T br,
+template <int Q, typename T, int N>
+__device__ __forceinline__ void p_euler(T (&vr)[N], T (&vi)[N], T ar, T ai, T c, T s, T br,
                                         T bi) {
 #pragma unroll
-  for (int j = 0; j < kPAmps; ++j) {
+  for (int j = 0; j < N; ++j) {
     if (j & (1 << Q)) continue;
     const int k = j | (1 << Q);
     p_scale(vr[j], vi[j], ar, ai);
@@ -284,8 +281,8 @@ __device__ __forceinline__ T own(T x) {
 
 // m11 on the amplitudes of SET in the lanes that meet the conditions: in the
 // others the factor is 1 (x * 1 - y * 0 is x)
-template <int SET, typename T>
-__device__ __forceinline__ void p_phase_if(uint32_t h, int tid, Regs<T> &vr, Regs<T> &vi, T ar,
+template <int SET, typename T, int N>
+__device__ __forceinline__ void p_phase_if(uint32_t h, int tid, T (&vr)[N], T (&vi)[N], T ar,
                                            T ai) {
   if (any_lane(h)) {
     p_phase<SET, T>(vr, vi, own(ar), own(ai));
@@ -296,8 +293,8 @@ __device__ __forceinline__ void p_phase_if(uint32_t h, int tid, Regs<T> &vr, Reg
 }
 
 // one-qubit gates on register bit Q
-template <int Q, typename T>
-__device__ __forceinline__ void p_op(int cls, Regs<T> &vr, Regs<T> &vi, const Par &w) {
+template <int Q, typename T, int N>
+__device__ __forceinline__ void p_op(int cls, T (&vr)[N], T (&vi)[N], const Par &w) {
   switch (cls) {
     case kPDense: {
       const T m[8] = {par<T>(w, 0), par<T>(w, 1), par<T>(w, 2), par<T>(w, 3),
@@ -339,10 +336,11 @@ struct Feed {
   }
 };
 
-template <typename T>
+template <typename T, int RB>
 __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
     const PassProgram by_value, typename Amp<T>::type *a) {
   typedef typename Amp<T>::type A;
+  constexpr int N = 1 << RB;
   // the first argument starts the kernel-argument segment
   const ProgramPtr prog = (ProgramPtr)__builtin_amdgcn_kernarg_segment_ptr();
   const int tb = int(prog->tb);
@@ -352,42 +350,42 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
   // taken by both halves, which store the same.)
   const int half = prog->nswaps == 0
                        ? 0
-                       : __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> (tb - kPRegBits));
-  const int tid = int(threadIdx.x) - (half << (tb - kPRegBits));
+                       : __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> (tb - RB));
+  const int tid = int(threadIdx.x) - (half << (tb - RB));
   // a tile of fewer than 1024 amplitudes still takes a whole wave, whose
   // lanes past the tile compute on copies and store nothing
-  const bool in = tid < (1 << (tb - kPRegBits));
+  const bool in = tid < (1 << (tb - RB));
   // amplitude index of the tile, and of the place it is stored in
   uint64_t base = pass_tile(prog, xcd_order(blockIdx.x, gridDim.x)), home = base;
   if (prog->nswaps != 0) {
     const uint64_t other = pass_home(prog, base);
     (half != 0 ? base : home) = other;
   }
-  T vr[kPAmps], vi[kPAmps];
+  T vr[N], vi[N];
   {
     // one thread address, plus a scalar offset per register (the masks of a
     // load share no bit); lanes past the tile read its first amplitudes,
     // their masks being zero
     const uint64_t i0 = base | xor_lanes<kPThrBits>(uint32_t(tid), prog->load_t);
     const char *p = reinterpret_cast<const char *>(a + i0);
-    A v[kPAmps];
+    A v[N];
     if ((prog->skip_t | prog->skip_r) == 0) {
 #pragma unroll
-      for (int j = 0; j < kPAmps; ++j)
+      for (int j = 0; j < N; ++j)
         v[j] = ld_stream(reinterpret_cast<const A *>(
-            p + xor_const<kPRegBits>(j, prog->load_r) * sizeof(A)));
+            p + xor_const<RB>(j, prog->load_r) * sizeof(A)));
     } else {
       const bool lane = ((i0 ^ prog->basis) & prog->skip_t) == 0;
 #pragma unroll
-      for (int j = 0; j < kPAmps; ++j) {
-        const uint64_t off = xor_const<kPRegBits>(j, prog->load_r);
+      for (int j = 0; j < N; ++j) {
+        const uint64_t off = xor_const<RB>(j, prog->load_r);
         v[j].x = v[j].y = T(0);
         if (((off ^ prog->basis) & prog->skip_r) == 0 && lane)
           v[j] = ld_stream(reinterpret_cast<const A *>(p + off * sizeof(A)));
       }
     }
 #pragma unroll
-    for (int j = 0; j < kPAmps; ++j) {
+    for (int j = 0; j < N; ++j) {
       vr[j] = v[j].x;
       vi[j] = v[j].y;
     }
@@ -407,7 +405,7 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
       if ((kind & ~3) == kPPhase) {
         if (!wave_meets(f.cur.h, uni)) continue;
         const T ar = par<T>(pw, 0), ai = par<T>(pw, 1);
-        switch (kind & 3) {
+        switch (kind & (RB == 4 ? 3 : 1)) {
           case 0: p_phase_if<1, T>(f.cur.h, tid, vr, vi, ar, ai); break;
           case 1: p_phase_if<2, T>(f.cur.h, tid, vr, vi, ar, ai); break;
           case 2: p_phase_if<4, T>(f.cur.h, tid, vr, vi, ar, ai); break;
@@ -416,11 +414,14 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
         continue;
       }
       if (kind < kPCPhase) {
-        switch (kind & 3) {
+        switch (kind & (RB == 4 ? 3 : 1)) {
           case 0: p_op<0, T>(kind & ~3, vr, vi, pw); break;
           case 1: p_op<1, T>(kind & ~3, vr, vi, pw); break;
-          case 2: p_op<2, T>(kind & ~3, vr, vi, pw); break;
-          default: p_op<3, T>(kind & ~3, vr, vi, pw); break;
+          case 2:
+            if constexpr (RB > 2) p_op<2, T>(kind & ~3, vr, vi, pw);
+            break;
+          default:
+            if constexpr (RB > 2) p_op<3, T>(kind & ~3, vr, vi, pw);
         }
         continue;
       }
@@ -445,10 +446,10 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
     if (++l == int(prog->nlayouts)) break;
     // exchange: written in this layout, through its index map, and read in
     // the next one
-    const LayoutPtr nxt = (LayoutPtr)w;
-    const uint32_t tx = fresh(uint32_t(tid)), lds0 = uint32_t(half) << (tb + 3);
-    uint32_t ws = xor_lanes<kPThrBits>(tx, lay->thr) >> 16 | lds0;
-    const uint32_t rs = (xor_lanes<kPThrBits>(tx, nxt->thr) & 0xffffu) | lds0;
+    const uint32_t both = xor_lanes<kPThrBits>(fresh(uint32_t(tid)), lay->thr);
+    const uint32_t lds0 = uint32_t(half) << (tb + 3);
+    uint32_t ws = both >> 16 | lds0;
+    uint32_t rs = (both & 0xffffu) | lds0;
     for (uint32_t k = 0; k < lay->nterm; ++k) {
       const uint32_t t = lay->term[k];
       if ((base >> (t & 63)) & 1) ws ^= t >> 16;
@@ -456,35 +457,49 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
     // byte offsets from the start of LDS, which is all dynamic here
     typedef __attribute__((address_space(3))) double *LdsDouble;
     typedef __attribute__((address_space(3))) f2v *LdsFloat2;
-    auto wslot = [&](int j) { return ws ^ (xor_const<kPRegBits>(j, lay->reg) >> 16); };
-    auto rslot = [&](int j) { return rs ^ (xor_const<kPRegBits>(j, nxt->reg) & 0xffffu); };
+    typedef __attribute__((address_space(3))) d2v *LdsDouble2;
+    auto wslot = [&](int j) { return ws ^ (xor_const<RB>(j, lay->reg) >> 16); };
+    auto rslot = [&](int j) { return rs ^ (xor_const<RB>(j, lay->reg) & 0xffffu); };
     __syncthreads();  // the reads of the exchange before
-    if constexpr (sizeof(T) == 8) {
+    if constexpr (sizeof(T) == 8 && RB < kPRegBits) {
+      // a small tile fits LDS with both parts side by side
       if (in) {
 #pragma unroll
-        for (int j = 0; j < kPAmps; ++j) *(LdsDouble)uintptr_t(wslot(j)) = vr[j];
+        for (int j = 0; j < N; ++j) *(LdsDouble2)uintptr_t(2 * wslot(j)) = d2v{vr[j], vi[j]};
       }
       __syncthreads();
 #pragma unroll
-      for (int j = 0; j < kPAmps; ++j)
+      for (int j = 0; j < N; ++j) {
+        const d2v x = *(LdsDouble2)uintptr_t(2 * rslot(j));
+        vr[j] = x.x;
+        vi[j] = x.y;
+      }
+    } else if constexpr (sizeof(T) == 8) {
+      if (in) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) *(LdsDouble)uintptr_t(wslot(j)) = vr[j];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < N; ++j)
         vr[j] = *(LdsDouble)uintptr_t(rslot(j));
       __syncthreads();
       if (in) {
 #pragma unroll
-        for (int j = 0; j < kPAmps; ++j) *(LdsDouble)uintptr_t(wslot(j)) = vi[j];
+        for (int j = 0; j < N; ++j) *(LdsDouble)uintptr_t(wslot(j)) = vi[j];
       }
       __syncthreads();
 #pragma unroll
-      for (int j = 0; j < kPAmps; ++j)
+      for (int j = 0; j < N; ++j)
         vi[j] = *(LdsDouble)uintptr_t(rslot(j));
     } else {
       if (in) {
 #pragma unroll
-        for (int j = 0; j < kPAmps; ++j) *(LdsFloat2)uintptr_t(wslot(j)) = f2v{vr[j], vi[j]};
+        for (int j = 0; j < N; ++j) *(LdsFloat2)uintptr_t(wslot(j)) = f2v{vr[j], vi[j]};
       }
       __syncthreads();
 #pragma unroll
-      for (int j = 0; j < kPAmps; ++j) {
+      for (int j = 0; j < N; ++j) {
         const f2v x = *(LdsFloat2)uintptr_t(rslot(j));
         vr[j] = x.x;
         vi[j] = x.y;
@@ -510,13 +525,13 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
   if (prog->store_add) {
     char *p = reinterpret_cast<char *>(a + i0);
 #pragma unroll
-    for (int j = 0; j < kPAmps; ++j)
-      st_stream(reinterpret_cast<A *>(p + xor_const<kPRegBits>(j, prog->store_r) * sizeof(A)),
+    for (int j = 0; j < N; ++j)
+      st_stream(reinterpret_cast<A *>(p + xor_const<RB>(j, prog->store_r) * sizeof(A)),
                 amp(j));
   } else {
 #pragma unroll
-    for (int j = 0; j < kPAmps; ++j)
-      st_stream(a + (i0 ^ xor_const<kPRegBits>(j, prog->store_r)), amp(j));
+    for (int j = 0; j < N; ++j)
+      st_stream(a + (i0 ^ xor_const<RB>(j, prog->store_r)), amp(j));
   }
 }
 
@@ -532,6 +547,15 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
 static int pass_tile_bits(int n) {
   return n <= kPMaxTile ? n : kPMaxTile - 1;
 }
+
+// Register bits of its layouts.  A state of up to 11 qubits is one work-group,
+// and with 16 amplitudes a thread one to four of its waves, each the whole
+// chain of ops long: 4 a thread give the arithmetic four times the SIMDs, at
+// the price of more exchanges, which a small tile does in one piece instead of
+// two planes (complex128 layered circuit, depth 8, 16 / 4 amplitudes: 8 qubits
+// 111 / 99 us, 10 qubits 142 / 124, 11 qubits 153 / 151; above, the work-group
+// would need more than its 512 threads).
+static int pass_reg_bits(int n) { return n <= kPThrBits + 2 ? 2 : kPRegBits; }
 
 // Two-norm bounds (log2) under which no amplitude can overflow: beyond them
 // the products by exact zeros are no longer zeros and the gates run one by
@@ -583,15 +607,20 @@ static int launch_pass(qcs_hip_state *s, const PassPick &pick,
   write_pass<T>(s->queue, pick, groups, s->n, tb, s->support, s->basis, &prog, s->filled);
   const int outer_bits = __builtin_popcountll(prog.outer);
   const int halves = prog.nswaps > 0 ? 2 : 1;
-  const int threads = std::max(64, halves << (tb - kPRegBits));
-  const size_t lds = prog.nlayouts > 1 ? size_t(8 * halves) << tb : 0;
+  const int threads = std::max(64, halves << (tb - pick.rb));
+  const size_t slot = pick.rb < kPRegBits ? sizeof(A) : 8;
+  const size_t lds = prog.nlayouts > 1 ? (slot * size_t(halves)) << tb : 0;
   TimedLaunch tl;
   const double amps = double(uint64_t(1) << (outer_bits + 2 * int(prog.nswaps) + tb));
   const double read = amps / double(uint64_t(1) << __builtin_popcountll(prog.skip_t | prog.skip_r));
   timing_begin(s, QCS_HIP_K_FUSED, (amps + read) * sizeof(A),
                6.0 * amps * double(pick.gates.size()), &tl);
-  hipLaunchKernelGGL(k_gate_pass<T>, dim3(unsigned(pass_work_groups(&prog, outer_bits))),
-                     dim3(unsigned(threads)), lds, s->stream, prog, static_cast<A *>(s->vec));
+  const dim3 grid(unsigned(pass_work_groups(&prog, outer_bits))), block{unsigned(threads)};
+  A *a = static_cast<A *>(s->vec);
+  if (pick.rb == 2)
+    hipLaunchKernelGGL((k_gate_pass<T, 2>), grid, block, lds, s->stream, prog, a);
+  else
+    hipLaunchKernelGGL((k_gate_pass<T, 4>), grid, block, lds, s->stream, prog, a);
   int rc = launch_check("k_gate_pass");
   if (rc) return rc;
   if (s->filled != ~uint64_t(0)) {
@@ -612,7 +641,8 @@ static int run_queue(qcs_hip_state *s, bool all) {
   const int tb = pass_tile_bits(s->n);
   const int words = s->precision == QCS_HIP_C128 ? 2 : 1;
   while (!q.empty() && (all || q.size() >= kQueueLow)) {
-    plan_pick(q, s->n, tb, kPassLowBits, words, 64, &pick, &groups, s->n > tb);
+    plan_pick(q, s->n, tb, kPassLowBits, words, 64, &pick, &groups, s->n > tb,
+              pass_reg_bits(s->n));
     if (!all && !pick.full && q.size() < kQueueMax) break;
     taken.clear();
     std::merge(pick.gates.begin(), pick.gates.end(), pick.swaps.begin(), pick.swaps.end(),

@@ -3,7 +3,7 @@
 // (no HIP), so tests can run the plans on the CPU.
 //
 // A pass holds a tile of 2^tb amplitudes in the registers of a work-group,
-// 16 to a thread: four of the tile's index bits select the register
+// 16 to a thread (rb = 4, fewer for small tiles): rb of the tile's index bits select the register
 // ("register bits"), the others the thread.  A gate that mixes amplitudes
 // needs its target among the register bits; a diagonal gate, and a control,
 // may sit anywhere, since an amplitude's index bits are known.  Between two
@@ -27,8 +27,7 @@
 
 namespace qcs {
 
-constexpr int kPRegBits = 4;               // register bits of a layout
-constexpr int kPAmps = 1 << kPRegBits;     // amplitudes per thread
+constexpr int kPRegBits = 4;               // register bits of a layout, at most
 constexpr int kPMaxTile = 13;              // tile bits: 512 threads x 16
 constexpr int kPThrBits = kPMaxTile - kPRegBits;
 constexpr int kPLineBits = 3;              // 8 amplitudes: a 128-byte line (complex128)
@@ -79,8 +78,9 @@ constexpr uint64_t pass_uniform(uint64_t base, unsigned wave) {
 constexpr int kPNoCond = 255;
 
 // Layout record, in whole words (scalar loads are 32 bits and up).  A pair
-// holds the LDS byte offset of a thread or register bit when the layout is
-// read, and in the upper half the one it is written to for the next layout.
+// belongs to the exchange that follows the layout: in the upper half the LDS
+// byte offset a thread or register bit of this layout is written to, in the
+// lower half the one it reads as a bit of the next layout.
 struct PassLayout {
   uint32_t thr[kPThrBits], reg[kPRegBits];
   uint32_t term[kPMaxTerms];  // index bit | offset << 16: written offsets change where the bit is set
@@ -105,6 +105,7 @@ struct PassProgram {
   uint32_t store_q[kPMaxTerms];
   // SWAPs of two index bits outside the tile (pairs of tiles change places)
   uint32_t nswaps, swaps[kPMaxSwaps];  // low bit | high bit << 8
+  uint32_t rb;                         // register bits
   uint32_t store_nterm;
   uint32_t store_add;  // the registers' masks share no bit with others: XOR is addition
   uint32_t words[kPWords + kPPad];
@@ -251,9 +252,10 @@ struct PassPick {
   bool full;               // the next gate does not fit: more gates would not change the pick
   std::vector<int> swaps;  // SWAPs of two qubits outside the tile, after the others
   uint64_t swapped;        // their qubits
+  int rb;                  // register bits of the layouts
 };
 
-// One group: ops on at most kPRegBits register qubits, then index maps.
+// One group: ops on at most rb register qubits, then index maps.
 struct PassGroup {
   std::vector<int> ops;   // indices into the gate list
   std::vector<int> maps;  // CNOTs and SWAPs, applied after the ops
@@ -263,7 +265,7 @@ struct PassGroup {
 // Appends gate g to the groups (opening a new one where it has to); returns
 // false when it cannot, because of the exchange's limit of outside terms.
 inline bool plan_add(std::vector<PassGroup> &gs, const std::vector<PlanGate> &gates, int i,
-                     uint64_t tile, int words_left) {
+                     uint64_t tile, int words_left, int rb) {
   const PlanGate &g = gates[size_t(i)];
   if (gs.empty()) gs.emplace_back();
   PassGroup *cur = &gs.back();
@@ -286,7 +288,7 @@ inline bool plan_add(std::vector<PassGroup> &gs, const std::vector<PlanGate> &ga
   }
   const uint64_t reg = g.need;  // the target of a gate that mixes amplitudes
   const bool fits = !(g.qubits & cur->mapped) &&
-                    __builtin_popcountll(cur->regs | reg) <= kPRegBits;
+                    __builtin_popcountll(cur->regs | reg) <= rb;
   if (!fits) {
     if (words_left < 2 * kPLayoutWords) return false;
     gs.emplace_back();
@@ -305,7 +307,7 @@ inline bool plan_add(std::vector<PassGroup> &gs, const std::vector<PlanGate> &ga
 // its qubits behind.
 inline void plan_pick(const std::vector<PlanGate> &gates, int n, int tb, int low,
                       int param_words, int scan, PassPick *out, std::vector<PassGroup> *groups,
-                      bool pairs = false) {
+                      bool pairs = false, int rb = kPRegBits) {
   uint64_t tile = (uint64_t(1) << (low < n ? low : n)) - 1;
   if (tb >= n) tile = (uint64_t(1) << n) - 1;
   uint64_t left = 0;  // qubits of the gates left behind
@@ -315,6 +317,7 @@ inline void plan_pick(const std::vector<PlanGate> &gates, int n, int tb, int low
   out->full = false;
   out->swaps.clear();
   out->swapped = 0;
+  out->rb = rb;
   groups->clear();
   // the layouts of the load and the store besides the groups'
   const int budget = kPWords - 2 * kPLayoutWords;
@@ -350,7 +353,7 @@ inline void plan_pick(const std::vector<PlanGate> &gates, int n, int tb, int low
   for (int q = 0; q < n && __builtin_popcountll(tile) < tb; ++q)
     tile |= (uint64_t(1) << q) & ~out->swapped;
   if (__builtin_popcountll(tile) < (tb < n ? tb : n)) {  // the swapped qubits have to fill it
-    plan_pick(gates, n, tb, low, param_words, scan, out, groups, false);
+    plan_pick(gates, n, tb, low, param_words, scan, out, groups, false, rb);
     return;
   }
   out->bits = tile;
@@ -361,7 +364,7 @@ inline void plan_pick(const std::vector<PlanGate> &gates, int n, int tb, int low
     const int i = out->gates[used];
     words += plan_op_words(gates[size_t(i)], param_words);
     const int room = budget - words - int(groups->size()) * kPLayoutWords;
-    if (room < kPLayoutWords || !plan_add(*groups, gates, i, tile, room)) {
+    if (room < kPLayoutWords || !plan_add(*groups, gates, i, tile, room, rb)) {
       out->full = true;
       break;
     }
@@ -384,14 +387,14 @@ inline void plan_pick(const std::vector<PlanGate> &gates, int n, int tb, int low
 struct LayoutMap {
   int reg[kPRegBits];  // tile positions of the register bits, ascending
   int thr[kPThrBits];  // tile positions of the thread bits
-  int nthr;
+  int nthr, nreg;
   int thread_bit(int pos) const {
     for (int b = 0; b < nthr; ++b)
       if (thr[b] == pos) return b;
     return -1;
   }
   int reg_bit(int pos) const {
-    for (int b = 0; b < kPRegBits; ++b)
+    for (int b = 0; b < nreg; ++b)
       if (reg[b] == pos) return b;
     return -1;
   }
@@ -400,10 +403,10 @@ struct LayoutMap {
 
 // `need`: tile positions.  Free register bits go to the highest positions,
 // which keeps the low ones for the lanes.
-inline LayoutMap make_layout(unsigned need, int tb) {
+inline LayoutMap make_layout(unsigned need, int tb, int rb) {
   LayoutMap m;
   unsigned regs = need;
-  for (int p = tb - 1; p >= 0 && __builtin_popcount(regs) < kPRegBits; --p)
+  for (int p = tb - 1; p >= 0 && __builtin_popcount(regs) < rb; --p)
     regs |= 1u << p;
   int r = 0;
   std::vector<int> rest;
@@ -412,6 +415,7 @@ inline LayoutMap make_layout(unsigned need, int tb) {
     else rest.push_back(p);
   }
   m.nthr = int(rest.size());
+  m.nreg = r;
   // lanes: the first four positions' bank vectors independent modulo 16,
   // five modulo 32, taking the lowest positions that are
   std::vector<int> order;
@@ -571,6 +575,7 @@ inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
                        uint64_t basis, PassProgram *pp, uint64_t filled = ~uint64_t(0)) {
   std::memset(pp, 0, offsetof(PassProgram, words));
   pp->tb = uint32_t(tb);
+  pp->rb = uint32_t(pick.rb);
   const uint64_t all = n < 64 ? (uint64_t(1) << n) - 1 : ~uint64_t(0);
   if (~filled & all) support = filled;
   support |= pick.swapped;
@@ -605,9 +610,9 @@ inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
   std::vector<Step> steps;
   const std::vector<int> none;
   const IndexMap ident = make_map(gates, none, pos, pick.bits);
-  const LayoutMap io = make_layout(0, tb);
+  const LayoutMap io = make_layout(0, tb, pick.rb);
   for (const PassGroup &g : groups)
-    steps.push_back(Step{make_layout(positions(g.regs), tb), &g,
+    steps.push_back(Step{make_layout(positions(g.regs), tb, pick.rb), &g,
                          make_map(gates, g.maps, pos, pick.bits)});
   if (!steps.front().m.io()) steps.insert(steps.begin(), Step{io, nullptr, ident});
   {
@@ -626,13 +631,13 @@ inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
   };
   const Step &first = steps.front(), &last = steps.back();
   for (int b = 0; b < first.m.nthr; ++b) pp->load_t[b] = index_mask(1 << first.m.thr[b]);
-  for (int b = 0; b < kPRegBits; ++b) pp->load_r[b] = index_mask(1 << first.m.reg[b]);
+  for (int b = 0; b < pick.rb; ++b) pp->load_r[b] = index_mask(1 << first.m.reg[b]);
   for (uint64_t m : pp->load_t) pp->skip_t |= m & ~filled;
   pp->skip_t |= pick.swapped & ~filled;  // (whole tiles)
   for (uint64_t m : pp->load_r) pp->skip_r |= m & ~filled;
   pp->basis = basis;
   for (int b = 0; b < last.m.nthr; ++b) pp->store_t[b] = index_mask(last.a.col[last.m.thr[b]]);
-  for (int b = 0; b < kPRegBits; ++b) pp->store_r[b] = index_mask(last.a.col[last.m.reg[b]]);
+  for (int b = 0; b < pick.rb; ++b) pp->store_r[b] = index_mask(last.a.col[last.m.reg[b]]);
   pp->store_nterm = uint32_t(last.a.nterm);
   for (int k = 0; k < last.a.nterm; ++k) {
     pp->store_q[k] = last.a.termq[k];
@@ -647,14 +652,15 @@ inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
     seen |= m;
   }
   uint32_t *w = pp->words;
-  for (const Step &s : steps) {
+  for (size_t x = 0; x < steps.size(); ++x) {
+    const Step &s = steps[x], &next = steps[x + 1 < steps.size() ? x + 1 : x];
     PassLayout l;
     std::memset(&l, 0, sizeof(l));
-    auto pair = [&](int p) {
-      return uint32_t(8 * pass_slot(1 << p)) | uint32_t(8 * pass_slot(s.a.col[p])) << 16;
+    auto pair = [&](int from, int to) {
+      return uint32_t(8 * pass_slot(1 << to)) | uint32_t(8 * pass_slot(s.a.col[from])) << 16;
     };
-    for (int b = 0; b < s.m.nthr; ++b) l.thr[b] = pair(s.m.thr[b]);
-    for (int b = 0; b < kPRegBits; ++b) l.reg[b] = pair(s.m.reg[b]);
+    for (int b = 0; b < s.m.nthr; ++b) l.thr[b] = pair(s.m.thr[b], next.m.thr[b]);
+    for (int b = 0; b < pick.rb; ++b) l.reg[b] = pair(s.m.reg[b], next.m.reg[b]);
     l.nterm = uint32_t(s.a.nterm);
     for (int k = 0; k < s.a.nterm; ++k)
       l.term[k] = uint32_t(s.a.termq[k]) | uint32_t(8 * pass_slot(s.a.termv[k])) << 16;

@@ -92,8 +92,8 @@ static T par(const uint32_t *w, int i) {
 }
 
 template <typename T>
-static void op1(int cls, T *vr, T *vi, int q, const uint32_t *w, bool on) {
-  for (int j = 0; j < kPAmps; ++j) {
+static void op1(int cls, T *vr, T *vi, int amps, int q, const uint32_t *w, bool on) {
+  for (int j = 0; j < amps; ++j) {
     if ((j >> q) & 1) continue;
     const int k = j | (1 << q);
     T x0 = vr[j], y0 = vi[j], x1 = vr[k], y1 = vi[k];
@@ -146,7 +146,9 @@ static void op1(int cls, T *vr, T *vi, int q, const uint32_t *w, bool on) {
 // One pass over the state, as k_gate_pass runs it.
 template <typename T>
 static void run_pass(Vec<T> &v, int n, const PassProgram &pp, uint64_t filled) {
-  const int tb = int(pp.tb), nthr = 1 << (tb - kPRegBits);
+  const int tb = int(pp.tb), kPRegBits = int(pp.rb), kPAmps = 1 << kPRegBits;
+  const int nthr = 1 << (tb - kPRegBits);
+  if (tb - kPRegBits > kPThrBits) fail("thread bits");
   const uint64_t N = uint64_t(1) << n;
   // the work-groups' tiles: with SWAPs outside the tile, pairs that change
   // places and tiles that stay
@@ -177,7 +179,7 @@ static void run_pass(Vec<T> &v, int n, const PassProgram &pp, uint64_t filled) {
       if (xor_bits<uint64_t>(uint32_t(t), pp.load_t, kPThrBits) != uint64_t(t)) fail("load line");
     const uint32_t *w = pp.words;
     for (uint32_t l = 0;;) {
-      PassLayout lay, nxt;
+      PassLayout lay;
       std::memcpy(&lay, w, sizeof(lay));
       w += kPLayoutWords;
       const uint32_t *end = w + lay.opwords;
@@ -202,11 +204,13 @@ static void run_pass(Vec<T> &v, int n, const PassProgram &pp, uint64_t filled) {
             on = on && ((t >> c) & 1);
           }
           if (kind < kPCPhase) {
-            op1<T>(kind & ~3, r, s, kind & 3, pw, on);
+            if ((1 << (kind & 3)) >= kPAmps) fail("register bit");
+            op1<T>(kind & ~3, r, s, kPAmps, kind & 3, pw, on);
             continue;
           }
           static const int sets[6] = {3, 5, 9, 6, 10, 12};
           const int set = kind < kPScale ? sets[kind - kPCPhase] : 0;
+          if (set >= kPAmps) fail("register bits");
           T ar = par<T>(pw, 0), ai = par<T>(pw, 1);
           if (kind == kPScale && !on) ar = T(1), ai = T(0);
           if (kind == kPSelect && on) ar = par<T>(pw, 2), ai = par<T>(pw, 3);
@@ -216,7 +220,6 @@ static void run_pass(Vec<T> &v, int n, const PassProgram &pp, uint64_t filled) {
         }
       }
       if (++l == pp.nlayouts) break;
-      std::memcpy(&nxt, w, sizeof(nxt));
       std::vector<T> lr(size_t(1) << tb), li(lr.size());
       std::vector<char> full(lr.size(), 0);
       for (int t = 0; t < nthr; ++t) {
@@ -234,9 +237,9 @@ static void run_pass(Vec<T> &v, int n, const PassProgram &pp, uint64_t filled) {
         }
       }
       for (int t = 0; t < nthr; ++t) {
-        const uint32_t rs = xor_bits<uint32_t>(uint32_t(t), nxt.thr, kPThrBits) & 0xffffu;
+        const uint32_t rs = xor_bits<uint32_t>(uint32_t(t), lay.thr, kPThrBits) & 0xffffu;
         for (int j = 0; j < kPAmps; ++j) {
-          uint32_t x = rs ^ (xor_bits<uint32_t>(uint32_t(j), nxt.reg, kPRegBits) & 0xffffu);
+          uint32_t x = rs ^ (xor_bits<uint32_t>(uint32_t(j), lay.reg, kPRegBits) & 0xffffu);
           if (x & 7) fail("read offset");
           x /= 8;
           if (x >= full.size() || full[x] != 1) fail("read slot");
@@ -280,7 +283,7 @@ static void run_pass(Vec<T> &v, int n, const PassProgram &pp, uint64_t filled) {
 }
 
 template <typename T>
-static int check(int n, int tb, int low, int count, int style, bool basis_state, bool unfilled, bool pairs) {
+static int check(int n, int tb, int low, int count, int style, bool basis_state, bool unfilled, bool pairs, int rb) {
   const uint64_t N = uint64_t(1) << n;
   std::vector<Gate> gates;
   std::vector<PlanGate> q;
@@ -356,7 +359,7 @@ static int check(int n, int tb, int low, int count, int style, bool basis_state,
   std::vector<PassGroup> groups;
   static PassProgram pp;
   while (!q.empty()) {
-    plan_pick(q, n, tb, low, int(sizeof(T) / 4), 64, &pick, &groups, pairs);
+    plan_pick(q, n, tb, low, int(sizeof(T) / 4), 64, &pick, &groups, pairs, rb);
     if (!pairs && !pick.swaps.empty()) fail("swaps");
     std::vector<int> taken = pick.gates;
     taken.insert(taken.end(), pick.swaps.begin(), pick.swaps.end());
@@ -390,7 +393,7 @@ static int check(int n, int tb, int low, int count, int style, bool basis_state,
 int main() {
   rng_state = 12345;
   long total = 0;
-  for (int n = 7; n <= 14; ++n)
+  for (int n = 7; n <= 13; ++n)
     for (int style = 0; style < 4; ++style)
       for (int rep = 0; rep < 6; ++rep) {
         // the whole state in a tile, then tiles smaller than it
@@ -398,8 +401,10 @@ int main() {
           for (int low = 3; low <= 4; ++low) {
             if (tb < n && tb < low + 4) continue;
             const int count = 20 + int(rnd() % 200);
-            total += check<double>(n, tb, low, count, style, rep % 3 > 0, rep % 3 > 1, rep > 2);
-            total += check<float>(n, tb, low, count, style, rep % 3 > 0, rep % 3 > 1, rep > 2);
+            for (int rb = 4; rb >= (low == 4 ? 2 : 4) && tb - rb <= kPThrBits; --rb) {
+              total += check<double>(n, tb, low, count, style, rep % 3 > 0, rep % 3 > 1, rep > 2, rb);
+              total += check<float>(n, tb, low, count, style, rep % 3 > 0, rep % 3 > 1, rep > 2, rb);
+            }
           }
       }
   if (swaps_set_aside < 100) fail("no pass moved its tiles");
