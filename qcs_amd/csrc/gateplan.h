@@ -166,9 +166,8 @@ inline int pass_bank(int p) {
   return v[p];
 }
 inline int pass_slot(int e) {
-  int s = 0;
-  for (int p = 0; p < kPMaxTile; ++p)
-    if ((e >> p) & 1) s ^= (1 << p) ^ (p >= 5 ? pass_bank(p) : 0);
+  int s = e;
+  for (e >>= 5; e; e &= e - 1) s ^= pass_bank(5 + __builtin_ctz(unsigned(e)));
   return s;
 }
 
@@ -408,25 +407,24 @@ inline LayoutMap make_layout(unsigned need, int tb, int rb) {
   unsigned regs = need;
   for (int p = tb - 1; p >= 0 && __builtin_popcount(regs) < rb; --p)
     regs |= 1u << p;
-  int r = 0;
-  std::vector<int> rest;
+  int r = 0, rest[kPMaxTile], nrest = 0;
   for (int p = 0; p < tb; ++p) {
     if ((regs >> p) & 1) m.reg[r++] = p;
-    else rest.push_back(p);
+    else rest[nrest++] = p;
   }
-  m.nthr = int(rest.size());
+  m.nthr = nrest;
   m.nreg = r;
   // lanes: the first four positions' bank vectors independent modulo 16,
   // five modulo 32, taking the lowest positions that are
-  std::vector<int> order;
-  std::vector<char> used(rest.size(), 0);
+  int norder = 0;  // m.thr
+  bool used[kPMaxTile] = {false};
   int basis[5] = {0, 0, 0, 0, 0};
   for (int want = 0, mask = 15; want < 5; ++want) {
     if (want == 4) {
       mask = 31;  // redo the basis in the larger space
       for (int &b : basis) b = 0;
-      for (int p : order) {
-        int v = pass_bank(p);
+      for (int b = 0; b < norder; ++b) {
+        int v = pass_bank(m.thr[b]);
         for (int k = 4; k >= 0; --k)
           if ((v >> k) & 1) {
             if (!basis[k]) { basis[k] = v; break; }
@@ -434,7 +432,7 @@ inline LayoutMap make_layout(unsigned need, int tb, int rb) {
           }
       }
     }
-    for (size_t x = 0; x < rest.size(); ++x) {
+    for (int x = 0; x < nrest; ++x) {
       if (used[x]) continue;
       int v = pass_bank(rest[x]) & mask;
       for (int k = 4; k >= 0; --k)
@@ -443,13 +441,12 @@ inline LayoutMap make_layout(unsigned need, int tb, int rb) {
       for (int k = 4; k >= 0; --k)
         if ((v >> k) & 1) { basis[k] = v; break; }
       used[x] = 1;
-      order.push_back(rest[x]);
+      m.thr[norder++] = rest[x];
       break;
     }
   }
-  for (size_t x = 0; x < rest.size(); ++x)
-    if (!used[x]) order.push_back(rest[x]);
-  for (int b = 0; b < m.nthr; ++b) m.thr[b] = order[size_t(b)];
+  for (int x = 0; x < nrest; ++x)
+    if (!used[x]) m.thr[norder++] = rest[x];
   return m;
 }
 
@@ -596,8 +593,7 @@ inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
     }
   auto positions = [&](uint64_t qubits) {
     unsigned r = 0;
-    for (int q = 0; q < 64; ++q)
-      if (((qubits & pick.bits) >> q) & 1) r |= 1u << pos[q];
+    for (qubits &= pick.bits; qubits; qubits &= qubits - 1) r |= 1u << pos[__builtin_ctzll(qubits)];
     return r;
   };
   // the layouts: the groups', with one of the load and one of the store
@@ -608,6 +604,7 @@ inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
     IndexMap a;
   };
   std::vector<Step> steps;
+  steps.reserve(groups.size() + 2);
   const std::vector<int> none;
   const IndexMap ident = make_map(gates, none, pos, pick.bits);
   const LayoutMap io = make_layout(0, tb, pick.rb);
@@ -625,8 +622,7 @@ inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
   pp->nlayouts = uint32_t(steps.size());
   auto index_mask = [&](int e) {
     uint64_t r = 0;
-    for (int p = 0; p < tb; ++p)
-      if ((e >> p) & 1) r |= uint64_t(1) << bits[p];
+    for (; e; e &= e - 1) r |= uint64_t(1) << bits[__builtin_ctz(unsigned(e))];
     return r;
   };
   const Step &first = steps.front(), &last = steps.back();
