@@ -341,6 +341,7 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
     const PassProgram by_value, typename Amp<T>::type *a) {
   typedef typename Amp<T>::type A;
   constexpr int N = 1 << RB;
+  constexpr int TH = RB < kPRegBits ? kPThrBits : kPMaxTile - RB;  // thread bits
   // the first argument starts the kernel-argument segment
   const ProgramPtr prog = (ProgramPtr)__builtin_amdgcn_kernarg_segment_ptr();
   const int tb = int(prog->tb);
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
     // one thread address, plus a scalar offset per register (the masks of a
     // load share no bit); lanes past the tile read its first amplitudes,
     // their masks being zero
-    const uint64_t i0 = base | xor_lanes<kPThrBits>(uint32_t(tid), prog->load_t);
+    const uint64_t i0 = base | xor_lanes<TH>(uint32_t(tid), prog->load_t);
     const char *p = reinterpret_cast<const char *>(a + i0);
     A v[N];
     if ((prog->skip_t | prog->skip_r) == 0) {
@@ -446,7 +447,7 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
     if (++l == int(prog->nlayouts)) break;
     // exchange: written in this layout, through its index map, and read in
     // the next one
-    const uint32_t both = xor_lanes<kPThrBits>(fresh(uint32_t(tid)), lay->thr);
+    const uint32_t both = xor_lanes<TH>(fresh(uint32_t(tid)), lay->thr);
     const uint32_t lds0 = uint32_t(half) << (tb + 3);
     uint32_t ws = both >> 16 | lds0;
     uint32_t rs = (both & 0xffffu) | lds0;
@@ -513,7 +514,7 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
     __syncthreads();
   }
   if (!in) return;
-  uint64_t i0 = home ^ xor_lanes<kPThrBits>(fresh(uint32_t(tid)), prog->store_t);
+  uint64_t i0 = home ^ xor_lanes<TH>(fresh(uint32_t(tid)), prog->store_t);
   for (uint32_t k = 0; k < prog->store_nterm; ++k)
     if ((base >> prog->store_q[k]) & 1) i0 ^= prog->store_term[k];
   auto amp = [&](int j) {
@@ -537,25 +538,26 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
 
 // ---- the queue of plain gates --------------------------------------------------
 
-// Tile of a pass over an n-qubit state.  A state of up to 13 qubits is one
-// tile, so a pass ends only where its program is full.  Larger states take
-// 12-bit tiles: 256 threads, four work-groups to a CU, which overlap their
-// HBM and arithmetic phases better than two of 512 (complex128 layered
-// circuit, all passes, 13 / 12 bits: 16 qubits 0.36 / 0.27 ms, 20 qubits
-// 0.54 / 0.48, 24 qubits 1.73 / 1.80, 28 qubits 24.5 / 21.8; 11 bits 0.30 at
-// 16 qubits, 25.7 at 28).
-static int pass_tile_bits(int n) {
-  return n <= kPMaxTile ? n : kPMaxTile - 1;
+// Tile of a pass over an n-qubit state, and register bits of its layouts.
+//
+// Large states: 12 bits with 16 amplitudes a thread, 256 threads, five
+// work-groups to a CU, which overlap their HBM and arithmetic phases
+// (complex128 layered circuit, 24 and 28 qubits, 13-bit tiles 1.73 and 24.5
+// ms, 12 bits 1.80 and 21.8, 11 bits 25.7 at 28).
+//
+// Up to 19 qubits such tiles leave most SIMDs idle and each wave is a long
+// chain: 10 bits with 4 amplitudes a thread spread the arithmetic 16 times as
+// wide, at the price of more exchanges and, above 12 qubits, of more passes
+// (complex128 layered circuits, 12 bits and 16 amplitudes / 10 and 4: 13
+// qubits 358 / 266 us, 14: 314 / 281, 16: 358 / 321, 17: 396 / 368, 19: 425 /
+// 404, 20: 483 / 468, 21: 519 / 567; complex64 14: 293 / 278, 19: 363 / 354,
+// 20: 420 / 433).  A state of up to 12 qubits is one tile, so a pass ends only
+// where its program is full, with 4 amplitudes a thread while 512 threads
+// hold it (10 qubits 16 / 4 amplitudes 142 / 124 us, 8 qubits 111 / 99).
+static int pass_tile_bits(int n) { return n <= kPMaxTile ? n : n < 20 ? 10 : kPMaxTile; }
+static int pass_reg_bits(int n) {
+  return pass_tile_bits(n) <= kPThrBits + 2 ? 2 : kPRegBits;
 }
-
-// Register bits of its layouts.  A state of up to 11 qubits is one work-group,
-// and with 16 amplitudes a thread one to four of its waves, each the whole
-// chain of ops long: 4 a thread give the arithmetic four times the SIMDs, at
-// the price of more exchanges, which a small tile does in one piece instead of
-// two planes (complex128 layered circuit, depth 8, 16 / 4 amplitudes: 8 qubits
-// 111 / 99 us, 10 qubits 142 / 124, 11 qubits 153 / 151; above, the work-group
-// would need more than its 512 threads).
-static int pass_reg_bits(int n) { return n <= kPThrBits + 2 ? 2 : kPRegBits; }
 
 // Two-norm bounds (log2) under which no amplitude can overflow: beyond them
 // the products by exact zeros are no longer zeros and the gates run one by

@@ -28,8 +28,8 @@
 namespace qcs {
 
 constexpr int kPRegBits = 4;               // register bits of a layout, at most
-constexpr int kPMaxTile = 13;              // tile bits: 512 threads x 16
-constexpr int kPThrBits = kPMaxTile - kPRegBits;
+constexpr int kPMaxTile = 12;              // tile bits, at most
+constexpr int kPThrBits = 9;               // thread bits, at most
 constexpr int kPLineBits = 3;              // 8 amplitudes: a 128-byte line (complex128)
 constexpr int kPMaxSwaps = 16;             // SWAPs of two bits outside the tile per pass
 constexpr int kPMaxTerms = 6;              // controls outside the tile per exchange
@@ -162,7 +162,7 @@ constexpr uint64_t pass_home(const P prog, uint64_t base) {
 // that 32 lanes whose positions have independent vectors use 32 slots that
 // differ modulo 32.
 inline int pass_bank(int p) {
-  static const int v[kPMaxTile] = {1, 2, 4, 8, 16, 1, 2, 4, 8, 16, 9, 18, 5};
+  static const int v[kPMaxTile] = {1, 2, 4, 8, 16, 1, 2, 4, 8, 16, 9, 18};
   return v[p];
 }
 inline int pass_slot(int e) {
