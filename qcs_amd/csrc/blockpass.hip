@@ -17,7 +17,7 @@
 // Launch variants (chosen per block by the autotuner, see qcs_hip_set_tuning,
 // and by the state's size, block_variant_for): TB 12 / 256 threads, or TB 13 /
 // 256 or 512 threads; with or without software pipelining (the next tile's
-// loads issued before the current tile's MFMA work); TB 10 on one wave for
+// loads issued before the current tile's MFMA work); TB 10 on two waves for
 // small states.  All use non-temporal global accesses and, when the
 //   state has >= 8 tiles, an XCD-aware tile order (work-group i runs on XCD
 //   i % 8, so XCD x takes the contiguous x-th eighth of the tiles).
@@ -56,11 +56,14 @@ __global__ __launch_bounds__(NTH) void k_fused_mfma(float2 *__restrict__ a,
   constexpr int CS = C + 1;                   // LDS row stride (float2), padded
   constexpr int MT = (RR + 31) / 32;          // 32-row blocks of the output
   constexpr int NW = NTH / 64;
-  constexpr int CT = C / (32 * NW);           // 32-column MFMA tiles per wave
+  constexpr int CW = NW < C / 32 ? NW : C / 32;  // waves across the columns
+  constexpr int RW = NW / CW;                 // and across the row blocks
+  constexpr int CT = C / (32 * CW);           // 32-column MFMA tiles per wave
+  constexpr int MW = MT / RW;                 // row blocks per wave
   constexpr int TBITS = __builtin_ctz(NTH) + 1;
   constexpr int IT = (1 << TB) / (2 * NTH);
   constexpr int IB = TB - TBITS;
-  static_assert(CT >= 1, "at least one column tile per wave");
+  static_assert(CW * RW == NW && MW >= 1, "work for every wave");
   // real and imaginary parts in separate planes: a half-wave reads one part
   // of 32 consecutive columns, 32 distinct 4-byte banks
   __shared__ float lre[R * CS], lim[R * CS];
@@ -68,10 +71,11 @@ __global__ __launch_bounds__(NTH) void k_fused_mfma(float2 *__restrict__ a,
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int h = lane >> 5, l32 = lane & 31;
 
-  float wa[MT][R];  // A operand: lane holds W[mt*32 + l32][2s + h]
+  const int cw = RW == 1 ? wave : wave % CW, mt0 = RW == 1 ? 0 : wave / CW * MW;
+  float wa[MW][R];  // A operand: lane holds W[mt*32 + l32][2s + h]
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int row = mt * 32 + l32;
+  for (int mt = 0; mt < MW; ++mt) {
+    const int row = (mt0 + mt) * 32 + l32;
 #pragma unroll
     for (int s = 0; s < R; ++s) wa[mt][s] = (row < RR) ? W[row * RR + 2 * s + h] : 0.0f;
   }
@@ -154,13 +158,15 @@ __global__ __launch_bounds__(NTH) void k_fused_mfma(float2 *__restrict__ a,
     }
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
-      const int col = (wave * CT + ct) * 32 + l32;
+      const int col = (cw * CT + ct) * 32 + l32;
       float b[R];
 #pragma unroll
       for (int s = 0; s < R; ++s) b[s] = bpl[s * CS + col];
-      floatx16 acc[MT];
+      // a wave of the other rows reads the columns that this one writes
+      if (RW > 1) __syncthreads();
+      floatx16 acc[MW];
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
+      for (int mt = 0; mt < MW; ++mt) {
         acc[mt] = floatx16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f,
                            0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -168,10 +174,10 @@ __global__ __launch_bounds__(NTH) void k_fused_mfma(float2 *__restrict__ a,
           acc[mt] = __builtin_amdgcn_mfma_f32_32x32x2f32(wa[mt][s], b[s], acc[mt], 0, 0, 0);
       }
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
+      for (int mt = 0; mt < MW; ++mt)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int r0 = mt * 16 + 4 * q + 2 * h;
+          const int r0 = (mt0 + mt) * 16 + 4 * q + 2 * h;
           if (r0 < R) {
             lre[r0 * CS + col] = acc[mt][4 * q];
             lim[r0 * CS + col] = acc[mt][4 * q + 1];
@@ -236,9 +242,12 @@ static void launch_k(qcs_hip_state *s, const float *W, const BlockGeom &g,
                      r.count, r.outer, r.fixed);
 }
 
-// one-wave tiles, for states too small to fill the chip with larger ones; not
-// among the variants a caller can name
-constexpr int kBlockTb10_64 = 16;
+// 10-bit tiles on two waves, for states too small to fill the chip with larger
+// ones; not among the variants a caller can name.  A five-qubit block on such a
+// tile is 64 matrix instructions in a row, 1.8 us of a 6 us launch, so its two
+// row blocks go to a wave each (whole flushes, one wave / two: 12 qubits 188 /
+// 166 us, 18 qubits 286 / 260, 20 qubits 497 / 493).
+constexpr int kBlockTb10 = 16;
 
 template <int K>
 static void launch_variant(qcs_hip_state *s, const float *W, const int *targets,
@@ -253,8 +262,8 @@ static void launch_variant(qcs_hip_state *s, const float *W, const int *targets,
     case QCS_HIP_BLOCK_TB13_256_PIPE:
       launch_k<K, 13, 256, true>(s, W, make_geom(s->n, K, targets, 13), 512);
       break;
-    case kBlockTb10_64:
-      launch_k<K, 10, 64, false>(s, W, make_geom(s->n, K, targets, 10), 4096);
+    case kBlockTb10:
+      launch_k<K, 10, 128, false>(s, W, make_geom(s->n, K, targets, 10), 4096);
       break;
     default:
       launch_k<K, 13, 512, true>(s, W, make_geom(s->n, K, targets, 13), 512);
@@ -265,14 +274,14 @@ static void launch_variant(qcs_hip_state *s, const float *W, const int *targets,
 // The variant a state of this size runs.  13-bit tiles on 512 threads need
 // many tiles to fill 256 CUs, and pay their barriers and operand loads for
 // them: whole flushes of the layered circuit, one-wave 10-bit tiles / 13-bit
-// tiles on 256 / on 512 threads: 18 qubits 286 / 499 / 659 us, 20 qubits
-// 521 / 607 / 788, 21 qubits 832 / 722 / 930, 23 qubits 1280 / 1163 / 1392,
+// tiles on 256 / on 512 threads: 18 qubits 286 / 499 / 659 us (two waves:
+// 260), 20 qubits 521 / 607 / 788, 21 qubits 832 / 722 / 930, 23 qubits 1280 / 1163 / 1392,
 // 26 qubits 5407 / 5258 / 5045, 28 qubits 18.3 / 17.1 / 16.1 ms.  (10 and 11
 // qubits ran k_fused_valu: 10 qubits 358 us.)
 int block_variant_for(const qcs_hip_state *s, int variant) {
-  if (s->n < 12) return kBlockTb10_64;
+  if (s->n < 12) return kBlockTb10;
   if (variant == QCS_HIP_BLOCK_TB13_512_PIPE && s->n < 25)
-    variant = s->n < 21 ? kBlockTb10_64 : QCS_HIP_BLOCK_TB13_256_PIPE;
+    variant = s->n < 21 ? kBlockTb10 : QCS_HIP_BLOCK_TB13_256_PIPE;
   if (variant == QCS_HIP_BLOCK_TB13_256_PIPE && s->n < 13) return QCS_HIP_BLOCK_TB12_256_PIPE;
   return variant;
 }
@@ -280,7 +289,7 @@ int block_variant_for(const qcs_hip_state *s, int variant) {
 // amplitudes that launch_block_mfma would read and write
 double block_mfma_amps(const qcs_hip_state *s, int k, const int *targets, int variant) {
   const int v = block_variant_for(s, variant);
-  const int tb = v == kBlockTb10_64 ? 10
+  const int tb = v == kBlockTb10 ? 10
                  : v == QCS_HIP_BLOCK_TB12_256 || v == QCS_HIP_BLOCK_TB12_256_PIPE ? 12 : 13;
   return double(tile_range(s, geom_mask(make_geom(s->n, k, targets, tb), tb), true).count << tb);
 }
