@@ -273,7 +273,7 @@ static void launch_variant(qcs_hip_state *s, const float *W, const int *targets,
 
 // The variant a state of this size runs.  13-bit tiles on 512 threads need
 // many tiles to fill 256 CUs, and pay their barriers and operand loads for
-// them: whole flushes of the layered circuit, one-wave 10-bit tiles / 13-bit
+// them: whole flushes of the layered circuit, 10-bit tiles on one wave / 13-bit
 // tiles on 256 / on 512 threads: 18 qubits 286 / 499 / 659 us (two waves:
 // 260), 20 qubits 521 / 607 / 788, 21 qubits 832 / 722 / 930, 23 qubits 1280 / 1163 / 1392,
 // 26 qubits 5407 / 5258 / 5045, 28 qubits 18.3 / 17.1 / 16.1 ms.  (10 and 11
