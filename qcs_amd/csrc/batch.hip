@@ -1755,10 +1755,16 @@ int batch_run(qcs_hip_batch *b, const qcs_hip_batch_circuit *cs, int nc,
         ops += resident ? 0.0 : 2.0;
       }
     }
-    // (a unit of complex64 work takes 2.8 times a unit of complex128 work:
-    // measured per layer at 20 qubits, 2.71 against 5.52 ms for 240 against
-    // 1392 units an amplitude)
-    cost[i] = (c.precision == QCS_HIP_C128 ? 16.0 : 8.0 * 2.8) *
+    // A unit of complex64 work takes 2.8 times a unit of complex128 work
+    // (measured per layer at 20 qubits, 2.71 against 5.52 ms for 240 against
+    // 1392 units an amplitude), and 4.8 times where other work-groups stream
+    // their states at the same time: with 2.8 the complex64 parts of a batch
+    // of 256 circuits of 10-18 qubits ran 3.5 to 5 ms where the complex128
+    // parts ran 2.5 to 3, and were still running when the rest had finished
+    // (kernel, three batches, 2.8 / 3.9 / 4.5 / 5.0 / 6.4: 7.5 / 7.1 / 6.8 /
+    // 6.8 / 7.0, 7.5 / 7.0 / 6.8 / 6.7 / 6.8, 8.1 / 7.3 / 7.2 / 7.1 / 7.4 ms).
+    const double unit = c.precision == QCS_HIP_C128 ? 1.0 : resident ? 2.8 : 4.8;
+    cost[i] = unit * double(amp) *
               double(uint64_t(1) << c.num_qubits) * (ops + 1.0);
   }
   const int nch_cap = int(std::max<uint64_t>(
