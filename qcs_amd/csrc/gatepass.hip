@@ -443,7 +443,8 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
           if (wave_meets(f.cur.h, uni)) p_phase_if<0, T>(f.cur.h, tid, vr, vi, ar, ai);
       }
     }
-    w = f.end;
+    const Words terms = f.end;
+    w = terms + lay->nterm;
     if (++l == int(prog->nlayouts)) break;
     // exchange: written in this layout, through its index map, and read in
     // the next one
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
     uint32_t ws = both >> 16 | lds0;
     uint32_t rs = (both & 0xffffu) | lds0;
     for (uint32_t k = 0; k < lay->nterm; ++k) {
-      const uint32_t t = lay->term[k];
+      const uint32_t t = terms[k];
       if ((base >> (t & 63)) & 1) ws ^= t >> 16;
     }
     // byte offsets from the start of LDS, which is all dynamic here
@@ -547,17 +548,15 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
 //
 // Up to 19 qubits such tiles leave most SIMDs idle and each wave is a long
 // chain: 10 bits with 4 amplitudes a thread spread the arithmetic 16 times as
-// wide, at the price of more exchanges and, above 12 qubits, of more passes
-// (complex128 layered circuits, 12 bits and 16 amplitudes / 10 and 4: 13
-// qubits 358 / 266 us, 14: 314 / 281, 16: 358 / 321, 17: 396 / 368, 19: 425 /
-// 404, 20: 483 / 468, 21: 519 / 567; complex64 14: 293 / 278, 19: 363 / 354,
-// 20: 420 / 433).  A state of up to 12 qubits is one tile, so a pass ends only
-// where its program is full, with 4 amplitudes a thread while 512 threads
-// hold it (10 qubits 16 / 4 amplitudes 142 / 124 us, 8 qubits 111 / 99).
+// wide, at the price of more exchanges and of more passes (layered circuits, 12
+// bits and 16 amplitudes / 10 and 4, complex128, 13 qubits: 358 / 266 us, 14:
+// 314 / 281, 16: 358 / 321, 17: 396 / 368, 19: 425 / 404, 20: equal, 21: 519 /
+// 567; complex64 13: 278 / 262, 14: 293 / 278, 19: 363 / 354, 20: 420 / 433).
+// A state of up to 12 qubits is one tile, so a pass ends only where its program
+// is full, with 4 amplitudes a thread while 512 threads hold it (10 qubits 16 /
+// 4 amplitudes 142 / 124 us, 8 qubits 111 / 99).
 static int pass_tile_bits(int n) { return n <= kPMaxTile ? n : n < 20 ? 10 : kPMaxTile; }
-static int pass_reg_bits(int n) {
-  return pass_tile_bits(n) <= kPThrBits + 2 ? 2 : kPRegBits;
-}
+static int pass_reg_bits(int tb) { return tb <= kPThrBits + 2 ? 2 : kPRegBits; }
 
 // Two-norm bounds (log2) under which no amplitude can overflow: beyond them
 // the products by exact zeros are no longer zeros and the gates run one by
@@ -639,13 +638,17 @@ static int run_queue(qcs_hip_state *s, bool all) {
   PassPick pick;
   std::vector<PassGroup> groups;
   std::vector<int> taken;  // the pick's gates and SWAPs
+  bool open = false;  // the last pick would take more gates
   int rc = 0;
   const int tb = pass_tile_bits(s->n);
   const int words = s->precision == QCS_HIP_C128 ? 2 : 1;
   while (!q.empty() && (all || q.size() >= kQueueLow)) {
     plan_pick(q, s->n, tb, kPassLowBits, words, 64, &pick, &groups, s->n > tb,
-              pass_reg_bits(s->n));
-    if (!all && !pick.full && q.size() < kQueueMax) break;
+              pass_reg_bits(tb));
+    if (!all && !pick.full && q.size() < kQueueMax) {
+      open = true;
+      break;
+    }
     taken.clear();
     std::merge(pick.gates.begin(), pick.gates.end(), pick.swaps.begin(), pick.swaps.end(),
                std::back_inserter(taken));
@@ -677,7 +680,7 @@ static int run_queue(qcs_hip_state *s, bool all) {
     }
     q.resize(keep);
   }
-  s->queue_mark = q.size() + kQueueStep;
+  s->queue_mark = std::max(kQueueLow, q.size() + (open ? kQueueStep : kQueueNext));
   return rc;
 }
 

@@ -83,9 +83,9 @@ constexpr int kPNoCond = 255;
 // lower half the one it reads as a bit of the next layout.
 struct PassLayout {
   uint32_t thr[kPThrBits], reg[kPRegBits];
-  uint32_t term[kPMaxTerms];  // index bit | offset << 16: written offsets change where the bit is set
-  uint32_t nterm;
-  uint32_t opwords;           // words of the ops that follow the record
+  // words that follow the record: ops, then terms of the exchange (index bit |
+  // offset << 16: written offsets change where the bit is set)
+  uint32_t nterm, opwords;
 };
 constexpr int kPLayoutWords = int(sizeof(PassLayout) / 4);
 
@@ -361,7 +361,9 @@ inline void plan_pick(const std::vector<PlanGate> &gates, int n, int tb, int low
   words = 0;
   for (; used < out->gates.size(); ++used) {
     const int i = out->gates[used];
-    words += plan_op_words(gates[size_t(i)], param_words);
+    const PlanGate &g = gates[size_t(i)];
+    words += plan_op_words(g, param_words);
+    if (g.cls == kGCnot && !((tile >> g.c) & 1)) ++words;  // a term, at most
     const int room = budget - words - int(groups->size()) * kPLayoutWords;
     if (room < kPLayoutWords || !plan_add(*groups, gates, i, tile, room, rb)) {
       out->full = true;
@@ -657,13 +659,14 @@ inline void write_pass(const std::vector<PlanGate> &gates, const PassPick &pick,
     };
     for (int b = 0; b < s.m.nthr; ++b) l.thr[b] = pair(s.m.thr[b], next.m.thr[b]);
     for (int b = 0; b < pick.rb; ++b) l.reg[b] = pair(s.m.reg[b], next.m.reg[b]);
-    l.nterm = uint32_t(s.a.nterm);
-    for (int k = 0; k < s.a.nterm; ++k)
-      l.term[k] = uint32_t(s.a.termq[k]) | uint32_t(8 * pass_slot(s.a.termv[k])) << 16;
+    // (the last layout's map is the store's)
+    l.nterm = x + 1 < steps.size() ? uint32_t(s.a.nterm) : 0;
     uint32_t *rec = w;
     w += kPLayoutWords;
     if (s.g) write_ops<T>(gates, s.g->ops, s.m, pos, pick.bits, w);
     l.opwords = uint32_t(w - rec - kPLayoutWords);
+    for (uint32_t k = 0; k < l.nterm; ++k)
+      *w++ = uint32_t(s.a.termq[k]) | uint32_t(8 * pass_slot(s.a.termv[k])) << 16;
     std::memcpy(rec, &l, sizeof(l));
   }
 }

@@ -725,9 +725,11 @@ __global__ __launch_bounds__(kThreads) void k_sample_wide(
 // two lanes (real and imaginary part) and rewrites the state once, where a
 // sweep per round moved 2 N s each time.  Any starting state is allowed.  The
 // recurrence runs on pairs of doubles, so it adds no error of its own and an
-// amplitude is rounded once instead of every round (14 qubits, 100 rounds from
-// the H layer: 1.1e-15 off the closed form, which is the layer's own error; in
-// plain doubles 2.0e-15).  27 qubits, 16 rounds: 11.7 -> 0.98 ms; 14 qubits,
+// amplitude is rounded once instead of every round: from the H layer, 4 to 19
+// qubits and up to 571 rounds, the marked probability is 7.0e-16 off the closed
+// form on average and 3.0e-15 at most, which is the layer's own error, where a
+// sweep per round was 8.9e-16 and 1.7e-14 off (14 qubits, 100 rounds, the
+// recurrence in plain doubles: 2.0e-15, in pairs 1.1e-15).  27 qubits, 16 rounds: 11.7 -> 0.98 ms; 14 qubits,
 // 100 rounds: 0.70 -> 0.032 ms, 0.26 us of it a round.
 
 // partial sums of the amplitudes other than m

@@ -219,13 +219,15 @@ static void run_pass(Vec<T> &v, int n, const PassProgram &pp, uint64_t filled) {
             if ((j & set) == set) cmul(ar, ai, r[j], s[j], r[j], s[j]);
         }
       }
+      const uint32_t *terms = w;
+      w += lay.nterm;
       if (++l == pp.nlayouts) break;
       std::vector<T> lr(size_t(1) << tb), li(lr.size());
       std::vector<char> full(lr.size(), 0);
       for (int t = 0; t < nthr; ++t) {
         uint32_t ws = xor_bits<uint32_t>(uint32_t(t), lay.thr, kPThrBits) >> 16;
         for (uint32_t k = 0; k < lay.nterm; ++k)
-          if ((base >> (lay.term[k] & 63)) & 1) ws ^= lay.term[k] >> 16;
+          if ((base >> (terms[k] & 63)) & 1) ws ^= terms[k] >> 16;
         for (int j = 0; j < kPAmps; ++j) {
           uint32_t x = ws ^ (xor_bits<uint32_t>(uint32_t(j), lay.reg, kPRegBits) >> 16);
           if (x & 7) fail("write offset");
