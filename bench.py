@@ -1037,7 +1037,7 @@ def run_mode(hip, ops, n, mode, args, steps, warmup, tune):
         step()
     hip.qcs_hip_device_sync()
     T = (time.perf_counter() - t0) / steps
-    f_ms, f_n, _, f_flops = timing(hip, state, qcs_amd.K_FUSED)
+    f_ms, f_n, f_bytes, f_flops = timing(hip, state, qcs_amd.K_FUSED)
     c_ms, _, _, _ = timing(hip, state, qcs_amd.K_COMPOSE)
     hip.qcs_hip_timing_enable(state, 0)
     avg_ms = f_ms / max(f_n, 1)
@@ -1059,7 +1059,8 @@ def run_mode(hip, ops, n, mode, args, steps, warmup, tune):
         "compose_ms_per_step": c_ms / steps,
         "launches": f_n,
         "avg_launch_ms": avg_ms,
-        "hbm_gbs": 2.0 * N * 8.0 / (avg_ms * 1e-3) / 1e9,
+        # (the amplitudes of tiles known to be zero are neither moved nor counted)
+        "hbm_gbs": f_bytes / max(f_ms, 1e-9) / 1e6,
         "tflops": flops_per_launch / (avg_ms * 1e-3) / 1e12,
     }
     return fused, r

@@ -97,7 +97,8 @@ void qc_swap(t_q_circuit *circuit, int qubit_a, int qubit_b);
 /* Apply a gate list in order: gate i is the qc_* call of ops[i] on
  * targets[i], with controls[i] (CNOT, CPHASE; the other qubit of a SWAP) and
  * params[i] (the angle), as if called one by one.  Stops at the first
- * unknown code; returns the number of gates applied. */
+ * unknown code; returns the number of gates applied (0 where an array is
+ * NULL). */
 long qc_apply_gates(t_q_circuit *circuit, const int *ops, const int *targets,
                     const int *controls, const double *params, long count);
 

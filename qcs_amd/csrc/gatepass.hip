@@ -3,27 +3,29 @@
 // A gate by itself reads and writes the state once (gates.hip: bound by HBM,
 // 5.8 TB/s in place).  A pass reads it once, runs the gates of gateplan.h's
 // program on it and writes it once, so the cost of a gate becomes its
-// arithmetic: a pass of the 28-qubit layered circuit (694 gates in 21 passes)
-// takes 1.5-2.1 ms, where each gate by itself took 1.2 ms.  The passes are
-// bound by FP64 multiplies and adds (VALU 95 % busy at the 1.9 GHz the card
-// holds under them; 288 of the 344 instructions per RZ RY RZ), HBM below it at
-// 4-5.7 TB/s.  The circuit went from 863 to 36 ms, the 28-qubit QFT (448 gates)
-// from 270 to 20 ms.
+// arithmetic: a pass of the 28-qubit layered circuit (694 gates in 22 passes)
+// takes 1.5-2.4 ms, where each gate by itself took 1.2 ms.  The passes are
+// bound by FP64 multiplies and adds (VALU 88-93 % busy at the 1.9 GHz the card
+// holds under them; 288 of about 330 instructions per RZ RY RZ), HBM below it
+// at 3.6-5.6 TB/s.  The circuit went from 863 to 36 ms, the 28-qubit QFT of any
+// state (476 gates with its preparation) from 269 to 14 ms.
 //
 // k_gate_pass.  One work-group per tile of 2^tb amplitudes; thread t holds 16
 // (small states: 4) of them in registers, those that differ in the layout's
-// register bits.  A layout change exchanges the tile through LDS, complex128 as two
-// planes (all real parts, then all imaginary parts), so a 12-bit tile takes
-// 32 KiB: four work-groups of 256 threads fit a CU (128 registers a thread),
-// and one computes while another waits for HBM.  The arithmetic is that of gates.hip without the
-// products by exact-zero entries, which add only signed zeros; the
-// amplitudes compare equal to the per-gate kernels' (bound_gate
+// register bits.  A layout change exchanges the tile through LDS, complex128 as
+// two planes (all real parts, then all imaginary parts), so a 12-bit tile takes
+// 32 KiB: five work-groups of 256 threads fit a CU (96 registers a thread), and
+// one computes while another waits for HBM.  The arithmetic is that of
+// gates.hip without the products by exact-zero entries, which add only signed
+// zeros; the amplitudes compare equal to the per-gate kernels' (bound_gate
 // keeps states whose amplitudes could overflow out).
 //
 // A state that starts as a basis state is zero wherever an index bit no gate
 // has mixed yet differs from the basis index; tiles of zeros are left alone
 // (28 qubits, H on every qubit and three layers: 21.5 -> 18.4 ms, with cheaper
-// addresses; the QFT of a basis state 15.4 -> 5.0 ms).
+// addresses; the QFT of a basis state 15.4 -> 5.0 ms), and those that no pass
+// has written yet are not read (launch_basis_start): 1.4 ms for that QFT.
+//
 // A SWAP of two bits outside the tile moves whole tiles: a work-group of two
 // halves reads a tile and the one it changes places with and stores each in
 // the other's place, so a bit reversal, which took four passes, takes one (28

@@ -430,6 +430,7 @@ void qc_swap(t_q_circuit *circuit, int qubit_a, int qubit_b) {
 long qc_apply_gates(t_q_circuit *circuit, const int *ops, const int *targets,
                     const int *controls, const double *params, long count) {
   long i;
+  if (!ops || !targets || !controls || !params) return 0;
   for (i = 0; i < count; i++) {
     const int t = targets[i], k = controls[i];
     const double a = params[i];

@@ -75,3 +75,4 @@ def test_counts_the_gates_applied():
         assert q.qc_apply_gates(c.handle, *args, 0) == 0
         assert q.qc_get_num_gates(c.handle) == 2
         assert q.qc_apply_gates(None, *args, 1) == 1
+        assert q.qc_apply_gates(c.handle, None, *args[1:], 1) == 0
