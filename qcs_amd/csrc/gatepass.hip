@@ -342,10 +342,9 @@ struct Feed {
 // are under way, all of them before one wait: a launch finds none there, and
 // read as the program gets to them each is a trip to L2 in a chain that a small
 // grid does not hide (8 and 10 qubits 89 -> 81 and 116 -> 105 us, 17 qubits 255 ->
-// 244, 20 qubits 405 -> 374).  Larger grids have their lines after the first
-// work-groups; one 12-bit tile's ops are long enough to hide the trips (12
-// qubits 162 -> 169).
-constexpr unsigned kWarmGrid = 512;
+// 244).  With 4 amplitudes a thread a grid has 512 work-groups at most (19
+// qubits); the ops of 16 amplitudes a thread are long enough to hide the trips
+// (12 qubits 162 -> 169, a 20-qubit circuit with its histogram 630 -> 657).
 __device__ __forceinline__ void warm_program(Words w) {
   static_assert(52 * 64 + 4 <= kPWords * 4, "inside the program");
   uint32_t x;
@@ -432,7 +431,7 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
           v[j] = ld_stream(reinterpret_cast<const A *>(p + off * sizeof(A)));
       }
     }
-    if (gridDim.x <= kWarmGrid && (RB < kPRegBits || gridDim.x > 1)) warm_program(prog->words);
+    if constexpr (RB < kPRegBits) warm_program(prog->words);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       vr[j] = v[j].x;
