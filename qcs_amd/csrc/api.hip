@@ -11,6 +11,7 @@
 #include <new>
 
 #include "internal.h"
+#include "normbound.h"
 
 namespace qcs {
 
@@ -212,16 +213,6 @@ static int copy_out(qcs_hip_state *s, const void *dev, long off, long count,
   return 0;
 }
 
-static uint64_t or_bits(const double *x, long n) {
-  uint64_t r = 0;
-  for (long i = 0; i < n; ++i) {
-    uint64_t b;
-    std::memcpy(&b, x + i, 8);
-    r |= b;
-  }
-  return r;
-}
-
 int validate_blocks(int n, const qcs_hip_block *blocks, int num_blocks,
                     const qcs_hip_gate *gates, int num_gates) {
   if (num_blocks < 0 || num_gates < 0 || (num_blocks > 0 && !blocks) ||
@@ -405,11 +396,11 @@ int qcs_hip_write(qcs_hip_state *s, long offset, long count, const double *in) {
   const size_t chunk_amps = size_t(1) << 20;
   if ((rc = ensure_pinned(s, chunk_amps * 16))) return rc;
   if (count > 0) s->support = ~uint64_t(0);
-  uint64_t exps = 0;  // the exponent bits of every value, or-ed
+  uint64_t bits = 0;
   for (long done = 0; done < count;) {
     const long m = long(std::min<size_t>(chunk_amps, size_t(count - done)));
     QCS_HIP_TRY(hipStreamSynchronize(s->stream));  // staging buffer free
-    exps |= or_bits(in + 2 * done, 2 * m);
+    bits |= or_bits(in + 2 * done, 2 * m);
     if (s->precision == QCS_HIP_C128) {
       std::memcpy(s->host, in + 2 * done, size_t(m) * 16);
     } else {
@@ -421,20 +412,9 @@ int qcs_hip_write(qcs_hip_state *s, long offset, long count, const double *in) {
                                hipMemcpyHostToDevice, s->stream));
     done += m;
   }
-  if (count > 0) {
-    // |x| < 2 for every value unless some exponent says otherwise
-    double top = 2.0;
-    if (((exps >> 52) & 0x7ff) >= 0x400) {
-      top = 0.0;
-      for (long i = 0; i < 2 * count; ++i)
-        if (!(std::fabs(in[i]) <= top)) top = std::fabs(in[i]);
-    }
-    const double b = std::log2(top) + 0.5 * std::log2(2.0 * double(count));
-    // the amplitudes left as they were keep their bound
-    const double old = uint64_t(count) == s->size ? b : s->log2_bound;
-    bound_reset(s, (old > b ? old : b) + 0.5);
-    if (!(b < 1e300)) bound_reset(s, b);  // infinite or NaN
-  }
+  if (count > 0)
+    bound_reset(s, bound_after_write(s->log2_bound, written_bound(in, count, bits),
+                                     uint64_t(count) == s->size));
   QCS_HIP_TRY(hipStreamSynchronize(s->stream));
   return 0;
 }
