@@ -38,11 +38,12 @@ inline double written_bound(const double *in, long count, uint64_t bits) {
 }
 
 // The bound after such a write: `old` is the bound before it, which the
-// amplitudes left as they were keep unless the `whole` state was written.
+// amplitudes left as they were keep unless the `whole` state was written.  A
+// NaN (a matrix with one was applied) bounds nothing, before and after.
 inline double bound_after_write(double old, double written, bool whole) {
   if (whole) old = written;
   if (!(written < 1e300)) return written;  // infinite
-  return (old > written ? old : written) + 0.5;
+  return (old <= written ? written : old) + 0.5;
 }
 
 }  // namespace qcs

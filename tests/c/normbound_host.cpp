@@ -36,6 +36,19 @@ int main() {
       check(bound(v) < 1e300 && bound(v) >= std::log2(x), "finite, and at least the largest value");
     }
   check(bound({1e300, nan, 1.0, 1.0}) > 900.0, "a large value before NaN");
+  // a part of the state written: what was unbounded stays so, what was bounded
+  // keeps the larger bound; the whole state written: the new values' bound
+  for (double old : {nan, -nan, inf}) {
+    check(!(qcs::bound_after_write(old, 3.0, false) < 1e300), "an unbounded rest");
+    check(qcs::bound_after_write(old, 3.0, true) < 1e300, "all of it replaced");
+  }
+  for (double old : {-20.0, 0.0, 700.0})
+    for (double w : {-20.0, 0.0, 700.0}) {
+      const double want = 0.5 * std::log2(std::exp2(2 * old) + std::exp2(2 * w));
+      const double b = qcs::bound_after_write(old, w, false);
+      check(b < 1e300 && (want > 1e300 || b >= want - 1e-12), "both parts together");
+      check(!(qcs::bound_after_write(old, inf, false) < 1e300), "an unbounded part");
+    }
   if (!bad) std::printf("ok\n");
   return bad != 0;
 }

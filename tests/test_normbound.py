@@ -1,6 +1,7 @@
 """The norm bound that keeps states with infinite, NaN or huge amplitudes out
 of the gate passes: its rule for written amplitudes on the CPU, and on the
 device the gates after such a write."""
+import ctypes
 import os
 import shutil
 import subprocess
@@ -36,10 +37,10 @@ def real_gates():
     return ops
 
 
-def gates_equal_one_by_one(prepare, n=8):
+def gates_equal_one_by_one(prepare, ops=None, n=8):
     """``prepare`` sets both states up; the parts are compared each by itself
     (numpy calls two complex numbers with any NaN equal)."""
-    ops = real_gates()
+    ops = ops or real_gates()
     with qcs_amd.Circuit(n) as a, qcs_amd.Circuit(n) as b:
         prepare(a)
         prepare(b)
@@ -59,3 +60,22 @@ def test_finite_values_after_a_bad_one(qlib, bad):
     v[0] = bad  # (1e300: the NaN after it)
     v[1] = bad if bad != 1e300 else np.nan
     gates_equal_one_by_one(lambda c: c.set_amplitudes(v))
+
+
+@pytest.mark.gpu
+def test_part_of_a_nan_state_written(qlib):
+    """A matrix with a NaN leaves half the state NaN; writing one amplitude
+    does not make the rest finite.  Y and RZ have zeros in places where the
+    per-gate kernels multiply NaN by them."""
+    hip, _ = qlib
+    m = (ctypes.c_double * 8)(1, 0, 0, 0, 0, 0, np.nan, 0)
+    one = (ctypes.c_double * 2)(0.5, 0.25)
+
+    def prepare(c):
+        for q in range(c.n):
+            c.h(q)
+        assert hip.qcs_hip_apply_1q(c.device_state, c.n - 1, m) == 0
+        assert hip.qcs_hip_write(c.device_state, 0, 1, one) == 0
+
+    gates_equal_one_by_one(
+        prepare, C.Ops().add(C.H, 0).add(C.Y, 7).add(C.RZ, 6, -1, 0.3).add(C.H, 3))
