@@ -727,7 +727,7 @@ static int run_queue(qcs_hip_state *s, bool all) {
     }
     q.resize(keep);
   }
-  s->queue_mark = std::max(kQueueLow, q.size() + (open ? kQueueStep : kQueueNext));
+  s->queue_mark = queue_next_look(q.size(), open);
   return rc;
 }
 

@@ -17,6 +17,7 @@
 // and cost no arithmetic.
 #pragma once
 
+#include <algorithm>
 #include <cmath>
 #include <cstddef>
 #include <cstdint>
@@ -35,6 +36,18 @@ constexpr int kPMaxSwaps = 16;             // SWAPs of two bits outside the tile
 constexpr int kPMaxTerms = 6;              // controls outside the tile per exchange
 constexpr int kPWords = 848;               // program words of a pass
 constexpr int kPPad = 17;                  // words read past the last op
+
+// The queue of gates that are not launched yet.
+constexpr size_t kQueueLow = 96;     // gates kept back to plan the next pass
+constexpr size_t kQueueStep = 64;    // gates to the next look at a queue whose pass is still open,
+constexpr size_t kQueueNext = 8;     // and after one that launched what it could (64: the device
+                                     // waited for the next pass, 17 qubits 283 -> 270 us)
+constexpr size_t kQueueMax = 1024;   // a queue of this size is launched from, open or not
+// The size at which a queue is next looked at: now it holds `size` gates, and
+// `open` if its next pass would take more of them.
+inline size_t queue_next_look(size_t size, bool open) {
+  return std::min(kQueueMax, std::max(kQueueLow, size + (open ? kQueueStep : kQueueNext)));
+}
 
 // A gate as the planner sees it.  kGCuDense (a controlled matrix that is
 // neither X nor a phase; no qc_* gate makes one) is not planned: it runs by

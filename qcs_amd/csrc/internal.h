@@ -30,11 +30,6 @@ constexpr int kPassMinQubits = 7;
 constexpr int kPassLowBits = 4;      // tiles always hold these index bits: 256-byte runs
                                      // (28 qubits: 21.8 ms; 3 bits 22.7, 5 bits 24.4)
 constexpr int kPassBigState = 18;    // from here on launches cost less than traffic
-constexpr size_t kQueueLow = 96;     // gates kept back to plan the next pass
-constexpr size_t kQueueStep = 64;    // gates to the next look at a queue whose pass is still open,
-constexpr size_t kQueueNext = 8;     // and after one that launched what it could (64: the device
-                                     // waited for the next pass, 17 qubits 283 -> 270 us)
-constexpr size_t kQueueMax = 1024;   // the queue never grows beyond this
 
 struct TimedLaunch {
   hipEvent_t start;
