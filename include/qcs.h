@@ -214,6 +214,10 @@ int qc_batch_get_amplitudes(t_q_batch *batch, int circuit, long offset,
  * run replayed a captured graph, else 0. */
 int qc_batch_last_timing(t_q_batch *batch, double *kernel_ms,
                          double *total_ms);
+/* Work items of the last run (more than circuits where several work-groups
+ * shared one) and how many of the batch's runs so far had to be repeated
+ * with a work-group per circuit.  Returns 0 or a negative QCS_HIP_E* code. */
+int qc_batch_last_sharing(t_q_batch *batch, int *items, int *fallbacks);
 /* Plan of the circuits with `num_qubits` qubits: LDS tile bits (complex128
  * <= 13, complex64 <= 14; a state of at most that many qubits stays on
  * chip) and, for fused circuits, the fusion width 1..5.  0 keeps the

@@ -404,6 +404,12 @@ int qcs_hip_batch_read_state(qcs_hip_batch *b, int circuit, long offset,
  * launch sequence, in ms; whether the last run replayed a captured graph */
 int qcs_hip_batch_last_timing(qcs_hip_batch *b, double *kernel_ms,
                               double *total_ms, int *graph_replayed);
+/* How the last run was shared out: the queue items its results came from
+ * (more than circuits where work-groups shared one), and how many of the
+ * batch's runs so far were repeated with a work-group per circuit because
+ * the parts of a circuit had not met (work of others held the device).
+ * No reference counterpart. */
+int qcs_hip_batch_last_sharing(qcs_hip_batch *b, int *items, int *fallbacks);
 
 #ifdef __cplusplus
 }

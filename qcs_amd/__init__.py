@@ -224,6 +224,12 @@ class Batch:
         replayed = self.lib.qc_batch_last_timing(self._b, ctypes.byref(k), ctypes.byref(t))
         return k.value, t.value, bool(replayed)
 
+    def last_sharing(self):
+        """Work items of the last run, and runs so far repeated unshared."""
+        items, fallbacks = ctypes.c_int(), ctypes.c_int()
+        self.lib.qc_batch_last_sharing(self._b, ctypes.byref(items), ctypes.byref(fallbacks))
+        return items.value, fallbacks.value
+
     def set_plan(self, fused, num_qubits, tile_bits=0, fuse_k=0):
         rc = self.lib.qc_batch_set_plan(self._b, int(bool(fused)), num_qubits, tile_bits, fuse_k)
         if rc != 0:

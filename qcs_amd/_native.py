@@ -124,6 +124,7 @@ _HIP_PROTOS = {
     "qcs_hip_batch_rerun": (c_int, [c_void_p, c_long, P(c_double), P(c_long)]),
     "qcs_hip_batch_read_state": (c_int, [c_void_p, c_int, c_long, c_long, P(c_double)]),
     "qcs_hip_batch_last_timing": (c_int, [c_void_p, P(c_double), P(c_double), P(c_int)]),
+    "qcs_hip_batch_last_sharing": (c_int, [c_void_p, P(c_int), P(c_int)]),
 }
 
 _Q = c_void_p  # t_q_circuit *
@@ -191,6 +192,7 @@ _QCS_PROTOS = {
     "qc_batch_run_shots": (c_int, [c_void_p, P(_Q), c_int, c_int, P(P(c_int))]),
     "qc_batch_get_amplitudes": (c_int, [c_void_p, c_int, c_long, c_long, P(c_double)]),
     "qc_batch_last_timing": (c_int, [c_void_p, P(c_double), P(c_double)]),
+    "qc_batch_last_sharing": (c_int, [c_void_p, P(c_int), P(c_int)]),
     "qc_batch_set_plan": (c_int, [c_void_p, c_int, c_int, c_int, c_int]),
     "qc_batch_set_threads": (c_int, [c_void_p, c_int]),
     "qc_autotune": (c_int, [_Q]),

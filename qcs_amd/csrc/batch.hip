@@ -1125,6 +1125,7 @@ struct qcs_hip_batch {
   std::vector<uint64_t> last_off;
   float kernel_ms = -1.0f, total_ms = -1.0f;
   int replayed = 0;
+  int fallbacks = 0;  // runs repeated without sharing
 };
 
 namespace qcs {
@@ -1605,6 +1606,7 @@ static int submit(qcs_hip_batch *b, bool rerun, int nb, bool build_graph) {
     b->last_grid = std::min(b->last_grid, k);
     drop_graph(b);
     b->replayed = 0;
+    ++b->fallbacks;
     if ((rc = enqueue_run(b, L, nc, 0, shots, b->last_tile_bytes, b->last_nch_cap, b->last_grid,
                           true, false)))
       return rc;
@@ -2102,6 +2104,13 @@ int qcs_hip_batch_last_timing(qcs_hip_batch *b, double *kernel_ms,
   if (kernel_ms) *kernel_ms = b->kernel_ms;
   if (total_ms) *total_ms = b->total_ms;
   if (graph_replayed) *graph_replayed = b->replayed;
+  return 0;
+}
+
+int qcs_hip_batch_last_sharing(qcs_hip_batch *b, int *items, int *fallbacks) {
+  if (!b) return fail(QCS_HIP_EINVAL, "null batch");
+  if (items) *items = b->has_last ? b->last_nitems : 0;
+  if (fallbacks) *fallbacks = b->fallbacks;
   return 0;
 }
 

@@ -548,3 +548,8 @@ int qc_batch_last_timing(t_q_batch *batch, double *kernel_ms,
     return 0;
   return replayed;
 }
+
+int qc_batch_last_sharing(t_q_batch *batch, int *items, int *fallbacks) {
+  if (!batch) return QCS_HIP_EINVAL;
+  return qcs_hip_batch_last_sharing(batch->dev, items, fallbacks);
+}
