@@ -1068,9 +1068,10 @@ __global__ void k_batch_reset(unsigned *queue, unsigned *sync, int nc) {
 // ---- host side ---------------------------------------------------------------------
 
 // byte offsets of the regions of the descriptor block (device and pinned
-// staging alike)
+// staging alike); `order` holds the queue items, `alone` those of a run with a
+// work-group per circuit (where circuits are shared)
 struct BatchLayout {
-  size_t circ, order, sync, pass, gate, group, block, hgate, hblock, u, total;
+  size_t circ, order, alone, sync, pass, gate, group, block, hgate, hblock, u, total;
 };
 
 // one host thread's share of a run's device ops (gates, register groups,
@@ -1125,7 +1126,10 @@ struct qcs_hip_batch {
   std::vector<uint64_t> last_off;
   float kernel_ms = -1.0f, total_ms = -1.0f;
   int replayed = 0;
-  int fallbacks = 0;  // runs repeated without sharing
+  // runs repeated without sharing: all of them, and those since a shared run
+  // last succeeded; the runs to come that do not try to share
+  int fallbacks = 0, failed = 0, unshared = 0;
+  int ran_items = 0;  // of the last run
 };
 
 namespace qcs {
@@ -1474,13 +1478,13 @@ static unsigned part_spin_limit() {
 }
 
 template <int NTH>
-static int launch_batch(qcs_hip_batch *b, const BatchLayout &L, int nitems,
+static int launch_batch(qcs_hip_batch *b, const BatchLayout &L, size_t order, int nitems,
                         uint64_t shots, int tile_bytes, int nch_cap, int grid) {
   char *d = static_cast<char *>(b->d_desc);
   hipLaunchKernelGGL(k_batch<NTH>, dim3(unsigned(grid)), dim3(NTH),
                      size_t(tile_bytes) + 2 * sizeof(double) * size_t(nch_cap),
                      b->stream, reinterpret_cast<const BCirc *>(d + L.circ),
-                     reinterpret_cast<const BItem *>(d + L.order), nitems,
+                     reinterpret_cast<const BItem *>(d + order), nitems,
                      reinterpret_cast<const BPass *>(d + L.pass),
                      reinterpret_cast<const BGate *>(d + L.gate),
                      reinterpret_cast<const BGroup *>(d + L.group),
@@ -1508,20 +1512,22 @@ static int batch_occupancy(int nth, int lds_bytes, int *per_cu) {
   }
 }
 
-static int batch_launch(qcs_hip_batch *b, int nth, const BatchLayout &L, int nitems,
+static int batch_launch(qcs_hip_batch *b, int nth, const BatchLayout &L, size_t order, int nitems,
                         uint64_t shots, int tile_bytes, int nch_cap, int grid) {
   switch (nth) {
-    case 256: return launch_batch<256>(b, L, nitems, shots, tile_bytes, nch_cap, grid);
-    default: return launch_batch<512>(b, L, nitems, shots, tile_bytes, nch_cap, grid);
+    case 256: return launch_batch<256>(b, L, order, nitems, shots, tile_bytes, nch_cap, grid);
+    default: return launch_batch<512>(b, L, order, nitems, shots, tile_bytes, nch_cap, grid);
   }
 }
 
 // The launch sequence of one run on b->stream: uploads, composition, queue
 // reset, the persistent kernel, the download of the sampled indices.  A
-// rerun uploads only the uniforms and keeps the composed blocks.
-static int enqueue_run(qcs_hip_batch *b, const BatchLayout &L, int nc, int nb,
-                       uint64_t shots, int tile_bytes, int nch_cap, int grid,
+// rerun uploads only the uniforms and keeps the composed blocks.  `alone`: a
+// work-group per circuit, none shared.
+static int enqueue_run(qcs_hip_batch *b, const BatchLayout &L, int nc, int nb, bool alone,
                        bool timed, bool rerun) {
+  const uint64_t shots = uint64_t(b->last_shots);
+  const int nitems = alone ? nc : b->last_nitems;
   char *d = static_cast<char *>(b->d_desc);
   const size_t ubytes = sizeof(double) * size_t(nc) * size_t(shots);
   if (!rerun)
@@ -1542,8 +1548,10 @@ static int enqueue_run(qcs_hip_batch *b, const BatchLayout &L, int nc, int nb,
                      reinterpret_cast<unsigned *>(d + L.sync), nc);
   if ((rc = launch_check("k_batch_reset"))) return rc;
   if (timed) QCS_HIP_TRY(hipEventRecord(b->ev[1], b->stream));
-  if ((rc = batch_launch(b, b->nth, L, b->last_nitems, shots, tile_bytes, nch_cap, grid)))
+  if ((rc = batch_launch(b, b->nth, L, alone ? L.alone : L.order, nitems, shots,
+                         b->last_tile_bytes, b->last_nch_cap, std::min(b->last_grid, nitems))))
     return rc;
+  b->ran_items = nitems;
   if (timed) QCS_HIP_TRY(hipEventRecord(b->ev[2], b->stream));
   if (ubytes)
     QCS_HIP_TRY(hipMemcpyAsync(b->h_out, b->d_out, ubytes, hipMemcpyDeviceToHost,
@@ -1559,8 +1567,10 @@ static int enqueue_run(qcs_hip_batch *b, const BatchLayout &L, int nc, int nb,
 static int submit(qcs_hip_batch *b, bool rerun, int nb, bool build_graph) {
   const BatchLayout &L = b->last_layout;
   const int nc = b->last_nc;
-  const uint64_t shots = uint64_t(b->last_shots);
-  const bool use_graph = (b->flags & QCS_HIP_BATCH_GRAPH) != 0;
+  const bool shared = b->last_nitems > nc;
+  bool alone = shared && b->unshared > 0;
+  if (alone) --b->unshared;
+  const bool use_graph = (b->flags & QCS_HIP_BATCH_GRAPH) != 0 && !alone;
   hipGraph_t *graph = rerun ? &b->rerun_graph : &b->graph;
   hipGraphExec_t *exec = rerun ? &b->rerun_exec : &b->exec;
   int rc;
@@ -1573,8 +1583,7 @@ static int submit(qcs_hip_batch *b, bool rerun, int nb, bool build_graph) {
       *exec = nullptr;
       *graph = nullptr;
       QCS_HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-      rc = enqueue_run(b, L, nc, nb, shots, b->last_tile_bytes, b->last_nch_cap,
-                       b->last_grid, false, rerun);
+      rc = enqueue_run(b, L, nc, nb, false, false, rerun);
       hipGraph_t g = nullptr;
       const hipError_t e = hipStreamEndCapture(b->stream, &g);
       if (rc) {
@@ -1588,31 +1597,27 @@ static int submit(qcs_hip_batch *b, bool rerun, int nb, bool build_graph) {
       b->replayed = 1;
     }
     QCS_HIP_TRY(hipGraphLaunch(*exec, b->stream));
+    b->ran_items = b->last_nitems;
   } else {
-    if ((rc = enqueue_run(b, L, nc, nb, shots, b->last_tile_bytes, b->last_nch_cap,
-                          b->last_grid, true, rerun)))
-      return rc;
+    if ((rc = enqueue_run(b, L, nc, nb, alone, true, rerun))) return rc;
   }
   QCS_HIP_TRY(hipEventRecord(b->ev[3], b->stream));
   QCS_HIP_TRY(hipStreamSynchronize(b->stream));
-  if (*b->h_flag != 0u && b->last_nitems > nc) {
+  if (*b->h_flag != 0u && shared && !alone) {
     // the parts of a circuit were not on the device together (work of other
-    // processes holds it): once more, a work-group per circuit
-    BItem *items = reinterpret_cast<BItem *>(b->h_stage + L.order);
-    int k = 0;
-    for (int i = 0; i < b->last_nitems; ++i)
-      if (items[i].part == 0) items[k++] = BItem{items[i].circ, 0, 1, 0};
-    b->last_nitems = k;
-    b->last_grid = std::min(b->last_grid, k);
-    drop_graph(b);
-    b->replayed = 0;
+    // processes holds it): once more, a work-group per circuit.  The plan
+    // keeps its shares, but as the wait for parts that do not come is several
+    // seconds, each failure in a row doubles the runs that go without.
     ++b->fallbacks;
-    if ((rc = enqueue_run(b, L, nc, 0, shots, b->last_tile_bytes, b->last_nch_cap, b->last_grid,
-                          true, false)))
-      return rc;
+    b->failed = std::min(b->failed + 1, 7);
+    b->unshared = (1 << (b->failed - 1)) - 1;
+    alone = true;
+    b->replayed = 0;
+    if ((rc = enqueue_run(b, L, nc, 0, true, true, true))) return rc;
     QCS_HIP_TRY(hipEventRecord(b->ev[3], b->stream));
     QCS_HIP_TRY(hipStreamSynchronize(b->stream));
   }
+  if (shared && !alone) b->failed = 0;
   if (*b->h_flag != 0u)
     return fail(QCS_HIP_EDEVICE, "batch: the work-groups sharing a circuit did not all "
                                  "reach a pass boundary in time");
@@ -1805,7 +1810,7 @@ int batch_run(qcs_hip_batch *b, const qcs_hip_batch_circuit *cs, int nc,
   }
   // queue items, the longest parts first; the parts of a shared circuit are
   // consecutive
-  std::vector<BItem> items;
+  std::vector<BItem> items, alone;
   {
     std::vector<int> idx(static_cast<size_t>(nc));
     for (int i = 0; i < nc; ++i) idx[size_t(i)] = i;
@@ -1815,6 +1820,12 @@ int batch_run(qcs_hip_batch *b, const qcs_hip_batch_circuit *cs, int nc,
     items.reserve(size_t(nc));
     for (int i : idx)
       for (int j = 0; j < shares[size_t(i)]; ++j) items.push_back(BItem{i, j, shares[size_t(i)], 0});
+    if (items.size() > size_t(nc)) {
+      std::stable_sort(idx.begin(), idx.end(),
+                       [&](int a, int c) { return cost[size_t(a)] > cost[size_t(c)]; });
+      alone.reserve(size_t(nc));
+      for (int i : idx) alone.push_back(BItem{i, 0, 1, 0});
+    }
   }
   const int nitems = int(items.size());
   const int grid = std::min(nitems, resident);
@@ -1829,6 +1840,7 @@ int batch_run(qcs_hip_batch *b, const qcs_hip_batch_circuit *cs, int nc,
   };
   L.circ = take(sizeof(BCirc) * size_t(nc));
   L.order = take(sizeof(BItem) * size_t(nitems));
+  L.alone = take(sizeof(BItem) * alone.size());
   L.sync = take(sizeof(unsigned) * size_t(nc));
   L.pass = take(sizeof(BPass) * size_t(np));
   L.gate = take(sizeof(BGate) * n_gate);
@@ -1923,6 +1935,7 @@ int batch_run(qcs_hip_batch *b, const qcs_hip_batch_circuit *cs, int nc,
   if (shots > 0)
     std::memcpy(h + L.u, u, sizeof(double) * size_t(nc) * size_t(shots));
   std::memcpy(h + L.order, items.data(), sizeof(BItem) * items.size());
+  if (!alone.empty()) std::memcpy(h + L.alone, alone.data(), sizeof(BItem) * alone.size());
 
   const double t2 = host_ms();
   std::vector<long> key = {b->generation, nc, nitems, np, nb, long(n_cgate), long(n_gate),
@@ -2109,7 +2122,7 @@ int qcs_hip_batch_last_timing(qcs_hip_batch *b, double *kernel_ms,
 
 int qcs_hip_batch_last_sharing(qcs_hip_batch *b, int *items, int *fallbacks) {
   if (!b) return fail(QCS_HIP_EINVAL, "null batch");
-  if (items) *items = b->has_last ? b->last_nitems : 0;
+  if (items) *items = b->has_last ? b->ran_items : 0;
   if (fallbacks) *fallbacks = b->fallbacks;
   return 0;
 }
