@@ -7,11 +7,14 @@ from splitmix64(seed 2); 2,410 gates) on a complex64 state resident in HBM:
 reset to |0...0>, record the gates through the qc_* API, flush (fusion plan,
 FP64 composition of the fused unitaries on the device, tile programs that
 apply several fused blocks per HBM pass on the FP32 matrix cores, FP64
-renormalisation).  value = gates * 2^30 / step time.
+renormalisation).  value = gates * 2^30 / step time: the circuit's nominal
+updates, whether or not an amplitude was known to be zero (the first passes
+of a step leave such tiles alone; the roofline counts only what was run).
 
 Beside it, in the same process:
   * the plain FP64 form of the same circuit (complex128, the gates' own
-    arithmetic, many gates per HBM pass), for the speedup and for 1 - F / max-abs of the fused state;
+    arithmetic, many gates per HBM pass), for the speedup and for 1 - F /
+    max-abs of the fused state;
   * the dominant kernel's roofline: average duration of the fused
     matrix-core kernel from HIP events recorded on the state's stream inside
     the timed steps; tile programs are bound by the FP32 matrix cores
@@ -126,6 +129,40 @@ def moved(hip, state, cls):
     if hip.qcs_hip_timing_moved(state, cls, ctypes.byref(mv)) != 0:
         raise RuntimeError(hip.qcs_hip_last_error())
     return mv.value
+
+
+def class_rates(ms, launches, nbytes, prefix):
+    """Average launch, GB/s and share of the memory's peak of a kernel class
+    from its total ms and bytes; None where nothing was launched."""
+    gbs = nbytes / (ms * 1e-3) / 1e9 if launches and ms > 0.0 else None
+    return {prefix + "_avg_ms": ms / launches if launches else None, prefix + "_gbs": gbs,
+            prefix + "_hbm_frac": None if gbs is None else gbs / HBM_PEAK_GBS}
+
+
+def plain_rates(one, cu, passes, moved_one, moved_cu, step_s):
+    """The plain form's rates from (ms, launches, bytes) of its one-qubit
+    kernels, its controlled kernels and its gate passes.  The passes run most
+    gates; the per-gate kernels only what is left over by itself."""
+    out = {}
+    for prefix, (ms, launches, nbytes), mv in (("k_1q", one, moved_one), ("k_cu", cu, moved_cu)):
+        out.update(class_rates(ms, launches, nbytes, prefix))
+        # what HBM moved: whole 128-byte lines (a controlled gate on qubit 0,
+        # 1 or 2 reads and writes every line, twice its algorithmic bytes)
+        lines = class_rates(ms, launches, mv, "moved")
+        out[prefix + "_moved_gbs"] = lines["moved_gbs"]
+        out[prefix + "_moved_hbm_frac"] = lines["moved_hbm_frac"]
+    # many gates per sweep over the state: the passes' own bytes
+    gp = class_rates(*passes, "x")
+    out["gate_passes"] = {"launches": passes[1], "avg_ms": gp["x_avg_ms"], "gbs": gp["x_gbs"],
+                          "hbm_frac": gp["x_hbm_frac"]}
+    # the plain form as a whole: the bytes of every launch that ran gates,
+    # over those launches' time and over the step's wall time
+    ms, launches, nbytes = (sum(x) for x in zip(one, cu, passes))
+    whole = class_rates(ms, launches, nbytes, "gate_kernels")
+    out["gate_kernels_gbs"] = whole["gate_kernels_gbs"]
+    out["gate_kernels_hbm_frac"] = whole["gate_kernels_hbm_frac"]
+    out["step_hbm_frac"] = nbytes / step_s / 1e9 / HBM_PEAK_GBS if launches else None
+    return out
 
 
 def cpu_model():
@@ -441,7 +478,9 @@ def bench_qft(args):
     |b>, b uniform from splitmix64 seed 1.  A step is: set |b>, apply the
     gates, wait.  Plain complex128 (value) and fused FP32 tile programs beside
     it; one 65536-amplitude range is checked against the closed form
-    exp(2 pi i rev(b) rev(y) / N) / sqrt(N)."""
+    exp(2 pi i rev(b) rev(y) / N) / sqrt(N).  value counts gates * 2^n, though
+    most of those amplitudes are known to be zero and left alone: from a basis
+    state the passes start with one tile."""
     import math
     import numpy as np
     import qcs_amd
@@ -483,6 +522,7 @@ def bench_qft(args):
     m1, n1, b1, _ = timing(hip, st, qcs_amd.K_1Q)
     m2, n2, b2, _ = timing(hip, st, qcs_amd.K_CU)
     m3, n3, b3, _ = timing(hip, st, qcs_amd.K_FUSED)
+    one, cu, gp = (class_rates(*x, "k") for x in ((m1, n1, b1), (m2, n2, b2), (m3, n3, b3)))
     off = 12345678 % (N - (1 << 16))
     y = np.arange(off, off + (1 << 16), dtype=np.int64)
     ref = np.exp(2j * np.pi * ((int(rev(np.array([b]))[0]) * rev(y)) % N) / N) / math.sqrt(N)
@@ -508,13 +548,10 @@ def bench_qft(args):
                    "qubits": n, "gates": G},
         "gates_per_s": G / tp,
         "closed_form_max_abs_err": err,
-        "k_1q": {"launches": n1, "avg_ms": m1 / max(n1, 1),
-                 "gbs": (b1 / max(n1, 1)) / (m1 / max(n1, 1) * 1e-3) / 1e9 if n1 else None},
-        "k_cu_and_swap": {"launches": n2, "avg_ms": m2 / max(n2, 1),
-                          "gbs_algorithmic": (b2 / max(n2, 1)) / (m2 / max(n2, 1) * 1e-3) / 1e9
-                          if n2 else None},
-        "gate_passes": {"launches": n3, "avg_ms": m3 / max(n3, 1),
-                        "gbs": b3 / (m3 * 1e-3) / 1e9 if n3 else None},
+        "k_1q": {"launches": n1, "avg_ms": one["k_avg_ms"], "gbs": one["k_gbs"]},
+        "k_cu_and_swap": {"launches": n2, "avg_ms": cu["k_avg_ms"],
+                          "gbs_algorithmic": cu["k_gbs"]},
+        "gate_passes": {"launches": n3, "avg_ms": gp["k_avg_ms"], "gbs": gp["k_gbs"]},
         "fused_fp32_tiles": {"ms_per_step": tf * 1e3, "amp_updates_per_s": G * N / tf,
                              "fused_blocks": blocks, "hbm_passes": passes,
                              "one_minus_f": omf, "max_abs_err": mx},
@@ -1201,30 +1238,8 @@ def main():
             "ms": Tp * 1e3,
             "amp_updates_per_s": G * N / Tp,
             "gates_per_s": G / Tp,
-            "k_1q_avg_ms": m1 / max(n1, 1),
-            "k_1q_gbs": (b1 / max(n1, 1)) / (m1 / max(n1, 1) * 1e-3) / 1e9 if n1 else None,
-            "k_cu_avg_ms": m2 / max(n2, 1),
-            "k_cu_gbs": (b2 / max(n2, 1)) / (m2 / max(n2, 1) * 1e-3) / 1e9 if n2 else None,
+            **plain_rates((m1, n1, b1), (m2, n2, b2), (m3, n3, b3), mv1, mv2, Tp),
         }
-        # many gates per sweep over the state: the passes' own bytes
-        result["plain_fp64"]["gate_passes"] = {
-            "launches": n3, "avg_ms": m3 / max(n3, 1),
-            "gbs": b3 / (m3 * 1e-3) / 1e9 if n3 else None,
-            "hbm_frac": b3 / (m3 * 1e-3) / 1e9 / HBM_PEAK_GBS if n3 else None}
-        result["plain_fp64"]["k_1q_hbm_frac"] = (result["plain_fp64"]["k_1q_gbs"] or 0) / HBM_PEAK_GBS
-        # the plain form as a whole: algorithmic bytes of every gate over the
-        # gate kernels' time, and over the step's wall time
-        if n1 + n2:
-            gk = (b1 + b2) / ((m1 + m2) * 1e-3) / 1e9
-            result["plain_fp64"]["gate_kernels_gbs"] = gk
-            result["plain_fp64"]["gate_kernels_hbm_frac"] = gk / HBM_PEAK_GBS
-            result["plain_fp64"]["step_hbm_frac"] = (b1 + b2) / Tp / 1e9 / HBM_PEAK_GBS
-        # what HBM moved: whole 128-byte lines (a controlled gate on qubit 0,
-        # 1 or 2 reads and writes every line, twice its algorithmic bytes)
-        for key, mv, ms_, n_ in (("k_1q", mv1, m1, n1), ("k_cu", mv2, m2, n2)):
-            gbs = mv / (ms_ * 1e-3) / 1e9 if n_ else None
-            result["plain_fp64"][key + "_moved_gbs"] = gbs
-            result["plain_fp64"][key + "_moved_hbm_frac"] = (gbs or 0) / HBM_PEAK_GBS
         result["speedup_vs_plain_fp64"] = Tp / m["ms_per_step"] * 1e3
         result["one_minus_f"] = omf
         result["max_abs_err"] = mx
