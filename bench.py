@@ -732,10 +732,8 @@ def bench_config5(args):
         out["grover_33q_c128"] = {
             "h_layer_ms": t_h * 1e3, "rounds": k, "rounds_ms": t_r * 1e3,
             "ms_per_round": t_r / k * 1e3,
-            # the reference's round: a sum, then a read+write update (3*N*s);
-            # here that is what all rounds together move (the sums follow by
-            # recurrence)
-            "round_gbs": 3 * N * sb / (t_r / k) / 1e9,
+            # what all rounds together move: a sum, then a read+write update
+            # (the rounds' sums follow by recurrence)
             "moved_gbs": 3 * N * sb / t_r / 1e9,
             "moved_hbm_frac": 3 * N * sb / t_r / 1e9 / HBM_PEAK_GBS,
             "marked": m, "p_marked": p, "p_marked_analytic": want,
