@@ -361,10 +361,8 @@ int qcs_hip_state_set_basis(qcs_hip_state *s, long basis) {
   if ((rc = check_state(s)) || (rc = queue_flush(s, false))) return rc;
   if (basis < 0 || uint64_t(basis) >= s->size)
     return fail(QCS_HIP_EINVAL, "basis %ld outside 2^%d", basis, s->n);
+  if ((rc = launch_basis_start(s, uint64_t(basis)))) return rc;
   bound_reset(s, 0.0);
-  s->support = 0;
-  s->basis = uint64_t(basis);
-  if ((rc = launch_basis_start(s))) return rc;
   if (s->scratch && (rc = launch_fill_basis(s, s->scratch, 0, 0))) return rc;
   return 0;
 }

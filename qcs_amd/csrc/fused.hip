@@ -221,11 +221,15 @@ static int apply_block(qcs_hip_state *s, int k, const int *targets,
   timing_begin(s, QCS_HIP_K_FUSED, 2.0 * amps * double(s->amp_bytes),
                8.0 * double(1 << k) * amps, &tl);
   if (s->precision == QCS_HIP_C64 && s->n >= 10) {
-    if ((rc = launch_block_mfma(s, k, targets, W, s->block_variant[k]))) return rc;
+    rc = launch_block_mfma(s, k, targets, W, s->block_variant[k]);
   } else {
     if (s->precision == QCS_HIP_C128) launch_valu<double>(s, k, U, targets);
     else launch_valu<float>(s, k, U, targets);
-    if ((rc = launch_check("k_fused_valu"))) return rc;
+    rc = launch_check("k_fused_valu");
+  }
+  if (rc) {
+    s->support = ~uint64_t(0);
+    return rc;
   }
   for (int q = 0; q < k; ++q) s->support |= uint64_t(1) << targets[q];
   return timing_end(s, &tl);

@@ -717,6 +717,7 @@ static int run_queue(qcs_hip_state *s, bool all) {
     }
     if (rc) {
       q.clear();  // the state is no longer what the rest would act on
+      s->support = ~uint64_t(0);
       break;
     }
     for (int i : taken) s->support |= plan_spread(q[size_t(i)]);

@@ -535,19 +535,30 @@ int launch_fill_basis(qcs_hip_state *s, void *buf, uint64_t basis, int one) {
 // one amplitude's.
 constexpr uint64_t kStartBytes = uint64_t(1) << 24;
 
-int launch_basis_start(qcs_hip_state *s) {
-  s->filled = ~uint64_t(0);
-  if (!s->queued || s->size * s->amp_bytes < kStartBytes)
-    return launch_fill_basis(s, s->vec, s->basis, 1);
-  if (s->precision == QCS_HIP_C128)
-    hipLaunchKernelGGL(k_fill<double>, dim3(1), dim3(kThreads), 0, s->stream,
-                       static_cast<double2 *>(s->vec) + s->basis, 1, 0, 1);
-  else
-    hipLaunchKernelGGL(k_fill<float>, dim3(1), dim3(kThreads), 0, s->stream,
-                       static_cast<float2 *>(s->vec) + s->basis, 1, 0, 1);
-  const int rc = launch_check("k_fill");
-  if (!rc) s->filled = 0;
-  return rc;
+// (What is known of the state changes only with the launch: after a failed
+// one it is what it was, but for amplitudes that may have become zero or one.)
+int launch_basis_start(qcs_hip_state *s, uint64_t basis) {
+  const bool whole = !s->queued || s->size * s->amp_bytes < kStartBytes;
+  int rc;
+  if (whole) {
+    rc = launch_fill_basis(s, s->vec, basis, 1);
+  } else {
+    if (s->precision == QCS_HIP_C128)
+      hipLaunchKernelGGL(k_fill<double>, dim3(1), dim3(kThreads), 0, s->stream,
+                         static_cast<double2 *>(s->vec) + basis, 1, 0, 1);
+    else
+      hipLaunchKernelGGL(k_fill<float>, dim3(1), dim3(kThreads), 0, s->stream,
+                         static_cast<float2 *>(s->vec) + basis, 1, 0, 1);
+    rc = launch_check("k_fill");
+  }
+  if (rc) {
+    s->support = ~uint64_t(0);
+    return rc;
+  }
+  s->support = 0;
+  s->basis = basis;
+  s->filled = whole ? ~uint64_t(0) : 0;
+  return 0;
 }
 
 int launch_fill_rest(qcs_hip_state *s) {
@@ -560,8 +571,9 @@ int launch_fill_rest(qcs_hip_state *s) {
   else
     hipLaunchKernelGGL(k_fill_rest<float>, dim3(g), dim3(kThreads), 0, s->stream,
                        static_cast<float2 *>(s->vec), s->size, s->filled, s->basis);
-  s->filled = ~uint64_t(0);
-  return launch_check("k_fill_rest");
+  const int rc = launch_check("k_fill_rest");
+  if (!rc) s->filled = ~uint64_t(0);
+  return rc;
 }
 
 }  // namespace qcs

@@ -93,7 +93,8 @@ struct qcs_hip_state {
   std::vector<qcs::PlanGate> queue;
   size_t queue_mark = qcs::kQueueLow;
   // amplitudes whose index differs from `basis` in a bit outside `support`
-  // are zero (all bits: nothing is known); gate passes skip their tiles
+  // are zero (all bits: nothing is known, as after a launch that failed and
+  // may yet have run); gate passes skip their tiles
   uint64_t support = 0, basis = 0;
   // memory holds only the amplitudes that agree with `basis` outside `filled`,
   // the others being zero; gate passes fill the rest as they grow the support,
@@ -143,7 +144,7 @@ int launch_1q(qcs_hip_state *s, int target, const double m[8]);
 int launch_cu(qcs_hip_state *s, int control, int target, const double m[8]);
 int launch_swap(qcs_hip_state *s, int a, int b);
 int launch_fill_basis(qcs_hip_state *s, void *buf, uint64_t basis, int one);
-int launch_basis_start(qcs_hip_state *s);
+int launch_basis_start(qcs_hip_state *s, uint64_t basis);
 int launch_fill_rest(qcs_hip_state *s);
 // kernels in gatepass.hip: a plain gate is queued, and launched together
 // with others on its tile; queue_flush launches what is queued

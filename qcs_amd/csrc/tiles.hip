@@ -1718,8 +1718,8 @@ int tiles_apply(qcs_hip_state *s, const qcs_hip_pass *passes, int np,
     else
       rc = split ? launch_tp<512, true, 0>(s, dp, p, db, tiles, nbp)
                  : launch_tp<512, false, 0>(s, dp, p, db, tiles, nbp);
+    s->support |= rc ? ~uint64_t(0) : targets;
     if (rc) return rc;
-    s->support |= targets;
     if ((rc = timing_end(s, &tl))) return rc;
     if (norm_partials && p == last_pass) *norm_partials = fs ? -1 : parts;
     if (scale_ahead && p == prev_pass && parts > 0 &&

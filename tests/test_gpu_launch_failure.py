@@ -1,0 +1,52 @@
+"""What is known of a state's zeros after a launch that reports a failure.
+
+The failure is injected on the host (QCS_HIP_INJECT_FAULT=launch:N: the N-th
+launch check of the process fails although the kernel ran), so the amplitudes
+may or may not have spread: the passes that follow must not leave tiles out
+as zeros.  Each case runs in a child process; the device never faults."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+# H on the qubits of the first launch, which reports the failure, then H on
+# the others: the uniform state if the launch ran and is not taken for lost
+CHILD = r"""
+import sys
+sys.path.insert(0, %r)
+import numpy as np
+import qcs_amd
+n, option, first, rest = 14, %d, %s, %s
+c = qcs_amd.Circuit(n, option)
+q, h = c.lib, c.handle
+for t in first:
+    q.qc_h(h, t)
+q.qc_flush(h)
+print("ERR", q.qc_last_error(h), flush=True)
+for t in rest:
+    q.qc_h(h, t)
+q.qc_flush(h)
+a = c.amplitudes()
+print("OFF", float(np.max(np.abs(a - 2.0 ** (-n / 2)))), flush=True)
+"""
+
+
+@pytest.mark.parametrize("option,launch,tol", [(0x0, 2, 1e-15), (0x1, 3, 1e-8)])
+def test_a_failed_launch_leaves_no_tile_out(qlib, option, launch, tol):
+    # launch checks: 1 = |0> fill of qc_create; complex128: 2 = the pass of the
+    # first gates, on one tile of 10 bits; fused complex64: 2 = the composition,
+    # 3 = the block of the first five
+    first = list(range(10)) if option == 0 else list(range(5, 10))
+    rest = [10, 11, 12, 13] + [q for q in range(5) if q not in first]
+    code = CHILD % (ROOT, option, first, rest)
+    env = dict(os.environ, QCS_HIP_INJECT_FAULT=f"launch:{launch}")
+    p = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True,
+                       timeout=120)
+    assert p.returncode == 0, p.stderr
+    assert "ERR -4" in p.stdout and p.stderr.count("injected failure") == 1, p.stdout + p.stderr
+    assert float(p.stdout.split("OFF ")[1].split()[0]) <= tol
