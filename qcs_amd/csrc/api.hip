@@ -358,13 +358,17 @@ int qcs_hip_state_flags(const qcs_hip_state *s) { return s ? s->flags : 0; }
 
 int qcs_hip_state_set_basis(qcs_hip_state *s, long basis) {
   int rc;
-  if ((rc = check_state(s)) || (rc = queue_flush(s, false))) return rc;
+  if ((rc = check_state(s))) return rc;
+  const int earlier = queue_flush(s, false);
   if (basis < 0 || uint64_t(basis) >= s->size)
     return fail(QCS_HIP_EINVAL, "basis %ld outside 2^%d", basis, s->n);
+  // a failure of the gates queued before is reported, but what replaces the
+  // state goes on
+  if (earlier) queue_drop(s);
   if ((rc = launch_basis_start(s, uint64_t(basis)))) return rc;
   bound_reset(s, 0.0);
   if (s->scratch && (rc = launch_fill_basis(s, s->scratch, 0, 0))) return rc;
-  return 0;
+  return earlier;
 }
 
 int qcs_hip_sync(qcs_hip_state *s) {
@@ -390,7 +394,12 @@ int qcs_hip_read_scratch(qcs_hip_state *s, long offset, long count,
 
 int qcs_hip_write(qcs_hip_state *s, long offset, long count, const double *in) {
   int rc;
-  if ((rc = ready(s)) || (rc = check_range(s, offset, count, in))) return rc;
+  if ((rc = check_state(s))) return rc;
+  const int earlier = queue_flush(s, true);
+  const bool whole = uint64_t(count) == s->size;
+  if (earlier && !whole) return earlier;
+  if ((rc = check_range(s, offset, count, in))) return rc;
+  if (earlier) queue_drop(s);  // (as in qcs_hip_state_set_basis)
   const size_t chunk_amps = size_t(1) << 20;
   if ((rc = ensure_pinned(s, chunk_amps * 16))) return rc;
   if (count > 0) s->support = ~uint64_t(0);
@@ -411,10 +420,10 @@ int qcs_hip_write(qcs_hip_state *s, long offset, long count, const double *in) {
     done += m;
   }
   if (count > 0)
-    bound_reset(s, bound_after_write(s->log2_bound, written_bound(in, count, bits),
-                                     uint64_t(count) == s->size));
+    bound_reset(s, bound_after_write(s->log2_bound, written_bound(in, count, bits), whole));
+  if (whole) s->filled = ~uint64_t(0);
   QCS_HIP_TRY(hipStreamSynchronize(s->stream));
-  return 0;
+  return earlier;
 }
 
 int qcs_hip_apply_1q(qcs_hip_state *s, int target, const double m[8]) {

@@ -742,6 +742,12 @@ int queue_flush(qcs_hip_state *s, bool fill) try {
   return fail(QCS_HIP_ENOMEM, "planning the queued gates: out of host memory");
 }
 
+// what could not be launched, given up
+void queue_drop(qcs_hip_state *s) {
+  std::lock_guard<std::mutex> lock(s->queue_mu);
+  s->queue.clear();
+}
+
 int queue_gate(qcs_hip_state *s, int kind, int target, int control, const double *m) try {
   if (!s->queued) return launch_gate(s, kind, target, control, m);
   std::lock_guard<std::mutex> lock(s->queue_mu);

@@ -150,6 +150,7 @@ int launch_fill_rest(qcs_hip_state *s);
 // with others on its tile; queue_flush launches what is queued
 int queue_gate(qcs_hip_state *s, int kind, int target, int control, const double *m);
 int queue_flush(qcs_hip_state *s, bool fill);
+void queue_drop(qcs_hip_state *s);
 // the bound of the state's two-norm that decides whether gates may be queued
 void bound_reset(qcs_hip_state *s, double log2_norm);
 void bound_normalized(qcs_hip_state *s);

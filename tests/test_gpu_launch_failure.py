@@ -1,4 +1,5 @@
-"""What is known of a state's zeros after a launch that reports a failure.
+"""States after a launch that reports a failure: what is known of their zeros,
+and the calls that replace them.
 
 The failure is injected on the host (QCS_HIP_INJECT_FAULT=launch:N: the N-th
 launch check of the process fails although the kernel ran), so the amplitudes
@@ -50,3 +51,41 @@ def test_a_failed_launch_leaves_no_tile_out(qlib, option, launch, tol):
     assert p.returncode == 0, p.stderr
     assert "ERR -4" in p.stdout and p.stderr.count("injected failure") == 1, p.stdout + p.stderr
     assert float(p.stdout.split("OFF ")[1].split()[0]) <= tol
+
+
+REPLACE = r"""
+import sys
+sys.path.insert(0, %r)
+import ctypes
+import numpy as np
+import qcs_amd
+n, how = 8, %r
+c = qcs_amd.Circuit(n)
+q, h = c.lib, c.handle
+for t in range(n):
+    q.qc_h(h, t)
+want = np.zeros(1 << n, np.complex128)
+want[5] = 1.0
+if how == "basis":
+    c.set_basis_state(5)
+else:
+    q.qc_set_amplitudes(h, 0, 1 << n, want.ctypes.data_as(ctypes.POINTER(ctypes.c_double)))
+print("ERR", q.qc_last_error(h), flush=True)
+a = c.amplitudes()
+c.h(0)
+c.h(0)
+print("SAME", bool(np.array_equal(a, want)), abs(c.amplitudes()[5] - 1.0) < 1e-15, flush=True)
+"""
+
+
+@pytest.mark.parametrize("how", ["basis", "write"])
+def test_a_replaced_state_does_not_need_the_gates_before(qlib, how):
+    """The queued gates' failure (launch check 2) is reported by the call that
+    launches them, a reset or a write of the whole state, which still does
+    what it was called for."""
+    env = dict(os.environ, QCS_HIP_INJECT_FAULT="launch:2")
+    p = subprocess.run([sys.executable, "-c", REPLACE % (ROOT, how)], env=env,
+                       capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0, p.stderr
+    assert "ERR -4" in p.stdout and p.stderr.count("injected failure") == 1, p.stdout + p.stderr
+    assert "SAME True True" in p.stdout, p.stdout
