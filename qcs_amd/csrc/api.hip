@@ -330,6 +330,7 @@ int qcs_hip_state_create(qcs_hip_state **out, int num_qubits, int precision,
     return rc;
   }
   if (num_qubits >= kPassMinQubits && !(flags & QCS_HIP_COMPAT)) {
+    s->queued = true;  // before another thread's qcs_hip_device_sync sees the state
     try {
       std::lock_guard<std::mutex> lock(g_states_mu);
       g_states.push_back(s);
@@ -337,7 +338,6 @@ int qcs_hip_state_create(qcs_hip_state **out, int num_qubits, int precision,
       free_state(s);
       return fail(QCS_HIP_ENOMEM, "host allocation failed");
     }
-    s->queued = true;
   }
   *out = s;
   return 0;
