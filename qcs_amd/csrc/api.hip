@@ -261,15 +261,18 @@ int qcs_hip_device_available(void) {
 }
 
 int qcs_hip_device_sync(void) {
-  int dev = 0, rc;
+  int dev = 0, rc = 0;
   QCS_HIP_TRY(hipGetDevice(&dev));
   {
+    // one state's failure keeps neither the others' gates nor the wait back
     std::lock_guard<std::mutex> lock(g_states_mu);
-    for (qcs_hip_state *s : g_states)
-      if (s->device == dev && (rc = queue_flush(s, false))) return rc;
+    for (qcs_hip_state *s : g_states) {
+      const int r = s->device == dev ? queue_flush(s, false) : 0;
+      if (r) rc = r;
+    }
   }
   QCS_HIP_TRY(hipDeviceSynchronize());
-  return 0;
+  return rc;
 }
 
 int qcs_hip_device_name(char *buf, int len) {

@@ -89,3 +89,36 @@ def test_a_replaced_state_does_not_need_the_gates_before(qlib, how):
     assert p.returncode == 0, p.stderr
     assert "ERR -4" in p.stdout and p.stderr.count("injected failure") == 1, p.stdout + p.stderr
     assert "SAME True True" in p.stdout, p.stdout
+
+
+SYNC = r"""
+import sys
+sys.path.insert(0, %r)
+import time
+import qcs_amd
+hip, q = qcs_amd.load()
+a, b = qcs_amd.Circuit(8), qcs_amd.Circuit(28)
+b.flush()
+for t in range(8):
+    a.h(t)
+for t in range(28):
+    b.h(t)
+    b.ry(t, 0.3)
+t0 = time.perf_counter()
+rc = hip.qcs_hip_device_sync()
+t1 = time.perf_counter()
+b.flush()
+t2 = time.perf_counter()
+print("RC", rc, "FIRST", t1 - t0 > t2 - t1, flush=True)
+"""
+
+
+def test_device_sync_waits_for_every_state(qlib):
+    """Launch check 3 is the pass of the first state; the second one's passes
+    (4 GiB, milliseconds) are launched and waited for all the same, so the
+    flush after it finds nothing to do."""
+    env = dict(os.environ, QCS_HIP_INJECT_FAULT="launch:3")
+    p = subprocess.run([sys.executable, "-c", SYNC % ROOT], env=env, capture_output=True,
+                       text=True, timeout=120)
+    assert p.returncode == 0, p.stderr
+    assert "RC -4 FIRST True" in p.stdout, p.stdout + p.stderr
