@@ -679,14 +679,16 @@ static int launch_pass(qcs_hip_state *s, const PassPick &pick,
 }
 
 // Launches passes from the head of the queue: all of it, or only those that
-// further gates would not change, while enough is left to plan the next.
+// further gates would not change, while enough is left to plan the next.  A
+// launch that fails loses its own gates, as a gate's own launch would; those
+// behind it still run, and the first failure is the result.
 static int run_queue(qcs_hip_state *s, bool all) {
   std::vector<PlanGate> &q = s->queue;
   PassPick pick;
   std::vector<PassGroup> groups;
   std::vector<int> taken;  // the pick's gates and SWAPs
   bool open = false;  // the last pick would take more gates
-  int rc = 0;
+  int first_rc = 0;
   const int tb = pass_tile_bits(s->n);
   const int words = s->precision == QCS_HIP_C128 ? 2 : 1;
   while (!q.empty() && (all || q.size() >= kQueueLow)) {
@@ -699,27 +701,26 @@ static int run_queue(qcs_hip_state *s, bool all) {
     taken.clear();
     std::merge(pick.gates.begin(), pick.gates.end(), pick.swaps.begin(), pick.swaps.end(),
                std::back_inserter(taken));
+    int rc;
     double traffic = 0.0;
     for (int i : taken) traffic += plan_gate_traffic(q[size_t(i)]);
     if (taken.size() <= 1 || (s->n >= kPassBigState && traffic <= 2.0)) {
       // the per-gate kernels move no more than the pass would
       if (taken.empty()) taken.push_back(0);
-      rc = launch_fill_rest(s);
+      const int fill_rc = rc = launch_fill_rest(s);
       for (int i : taken) {
-        if (rc) break;
+        if (fill_rc) break;  // memory is not the state yet
         const PlanGate &g = q[size_t(i)];
         const int kind = g.cls == kGSwap ? QCS_HIP_G_SWAP : g.c >= 0 ? QCS_HIP_G_CU : QCS_HIP_G_1Q;
-        rc = launch_gate(s, kind, g.t, g.c, g.m);
+        const int gate_rc = launch_gate(s, kind, g.t, g.c, g.m);
+        if (gate_rc && !rc) rc = gate_rc;
       }
     } else {
       rc = s->precision == QCS_HIP_C128 ? launch_pass<double>(s, pick, groups, tb)
                                         : launch_pass<float>(s, pick, groups, tb);
     }
-    if (rc) {
-      q.clear();  // the state is no longer what the rest would act on
-      s->support = ~uint64_t(0);
-      break;
-    }
+    if (rc && !first_rc) first_rc = rc;
+    if (rc) s->support = ~uint64_t(0);
     for (int i : taken) s->support |= plan_spread(q[size_t(i)]);
     size_t keep = 0, x = 0;
     for (size_t i = 0; i < q.size(); ++i) {
@@ -729,7 +730,7 @@ static int run_queue(qcs_hip_state *s, bool all) {
     q.resize(keep);
   }
   s->queue_mark = queue_next_look(q.size(), open);
-  return rc;
+  return first_rc;
 }
 
 // (the planner's vectors may throw; the queue is whole either way)
@@ -737,7 +738,8 @@ int queue_flush(qcs_hip_state *s, bool fill) try {
   if (!s->queued) return 0;
   std::lock_guard<std::mutex> lock(s->queue_mu);
   const int rc = s->queue.empty() ? 0 : run_queue(s, true);
-  return rc || !fill ? rc : launch_fill_rest(s);
+  const int fill_rc = fill ? launch_fill_rest(s) : 0;
+  return rc ? rc : fill_rc;
 } catch (const std::exception &) {
   return fail(QCS_HIP_ENOMEM, "planning the queued gates: out of host memory");
 }
@@ -754,10 +756,11 @@ int queue_gate(qcs_hip_state *s, int kind, int target, int control, const double
   if (kind != QCS_HIP_G_SWAP) bound_gate(s, m);
   const PlanGate g = plan_gate(kind, target, control, m);
   if (g.cls == kGCuDense || !bounded(s)) {
-    int rc = s->queue.empty() ? 0 : run_queue(s, true);
-    if (!rc) rc = launch_fill_rest(s);
+    const int earlier = s->queue.empty() ? 0 : run_queue(s, true);
+    int rc = launch_fill_rest(s);
     s->support = ~uint64_t(0);  // 0 times infinity
-    return rc ? rc : launch_gate(s, kind, target, control, m);
+    if (!rc) rc = launch_gate(s, kind, target, control, m);
+    return earlier ? earlier : rc;
   }
   s->queue.push_back(g);
   return s->queue.size() >= s->queue_mark ? run_queue(s, false) : 0;

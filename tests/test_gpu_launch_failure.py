@@ -122,3 +122,33 @@ def test_device_sync_waits_for_every_state(qlib):
                        text=True, timeout=120)
     assert p.returncode == 0, p.stderr
     assert "RC -4 FIRST True" in p.stdout, p.stdout + p.stderr
+
+
+BEHIND = r"""
+import sys
+sys.path.insert(0, %r)
+import numpy as np
+import qcs_amd
+n = 14
+c = qcs_amd.Circuit(n)
+for t in range(10):
+    c.h(t)
+for t in range(10, n):
+    c.x(t)
+c.flush()
+print("ERR", c.lib.qc_last_error(c.handle), flush=True)
+want = np.zeros(1 << n)
+want[15 << 10:] = 2.0 ** -5
+print("OFF", float(np.max(np.abs(c.amplitudes() - want))), flush=True)
+"""
+
+
+def test_gates_behind_a_failed_launch_still_run(qlib):
+    """Launch check 2 is the pass of the H gates, which runs and reports a
+    failure; the X gates are a pass of their own behind it."""
+    env = dict(os.environ, QCS_HIP_INJECT_FAULT="launch:2")
+    p = subprocess.run([sys.executable, "-c", BEHIND % ROOT], env=env, capture_output=True,
+                       text=True, timeout=120)
+    assert p.returncode == 0, p.stderr
+    assert "ERR -4" in p.stdout and p.stderr.count("injected failure") == 1, p.stdout + p.stderr
+    assert float(p.stdout.split("OFF ")[1].split()[0]) <= 1e-15
