@@ -93,8 +93,12 @@ int qcs_hip_read_scratch(qcs_hip_state *s, long offset, long count,
  * queues the gate; gates are launched together, several to a sweep over the
  * state, while later ones are still being queued, and what is left when an
  * entry point reads or changes the state otherwise, waits for it
- * (qcs_hip_sync, qcs_hip_device_sync) or destroys it.  A launch failure is
- * reported by the call that launches.  A program that waits with HIP's own
+ * (qcs_hip_sync, qcs_hip_device_sync) or destroys it.  The first are launched
+ * when 96 are queued, and never do more than 1024 wait, so a program that
+ * works on the host between gates has them launched later than its calls.  A
+ * launch failure is reported by the call that launches; it loses the gates of
+ * that launch, the others run, and a reset or a write of the whole state
+ * still does what it was called for.  A program that waits with HIP's own
  * calls instead of these has to call one of these first. */
 int qcs_hip_apply_1q(qcs_hip_state *s, int target, const double m[8]);
 /* qcs_hip_apply_cu replaces q_apply_2q_gate / q_apply_2q_gate_gpu
@@ -298,10 +302,13 @@ int qcs_hip_apply_passes_normalize(qcs_hip_state *s, const qcs_hip_pass *passes,
 #define QCS_HIP_BLOCK_TB12_256_PIPE 1 /* same, next tile's loads pipelined */
 #define QCS_HIP_BLOCK_TB13_256_PIPE 2 /* 8192-amplitude tiles, 256 threads */
 #define QCS_HIP_BLOCK_TB13_512_PIPE 3 /* 8192-amplitude tiles, 512 threads
-                                         (default); states of up to 24
-                                         qubits, which such tiles do not
-                                         fill the device with, run smaller
-                                         work-groups under this value */
+                                         (default) */
+/* States that such tiles do not fill the device with run other work-groups:
+ * under value 3 (named or by default) those of up to 20 qubits 1024-amplitude
+ * tiles on 128 threads and those of 21 to 24 the kernel of value 2; of 12
+ * qubits value 2 is that of value 1; of 10 and 11 every value runs the
+ * 1024-amplitude tiles, below 10 a kernel without matrix cores.  The results are the same bits under every value, and
+ * qcs_hip_get_tuning answers the value that was set. */
 int qcs_hip_set_tuning(qcs_hip_state *s, int knob, int value);
 /* the current value of a knob (what the autotuner chose, or the default) */
 int qcs_hip_get_tuning(qcs_hip_state *s, int knob, int *value);

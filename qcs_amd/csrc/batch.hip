@@ -1769,7 +1769,9 @@ int batch_run(qcs_hip_batch *b, const qcs_hip_batch_circuit *cs, int nc,
     // of 256 circuits of 10-18 qubits ran 3.5 to 5 ms where the complex128
     // parts ran 2.5 to 3, and were still running when the rest had finished
     // (kernel, three batches, 2.8 / 3.9 / 4.5 / 5.0 / 6.4: 7.5 / 7.1 / 6.8 /
-    // 6.8 / 7.0, 7.5 / 7.0 / 6.8 / 6.7 / 6.8, 8.1 / 7.3 / 7.2 / 7.1 / 7.4 ms).
+    // 6.8 / 7.0, 7.5 / 7.0 / 6.8 / 6.7 / 6.8, 8.1 / 7.3 / 7.2 / 7.1 / 7.4 ms;
+    // 2.8 / 4.8 with 512 circuits 8.2 / 7.6, with 4096 of 10-20 qubits 303.9 /
+    // 303.1).
     const double unit = c.precision == QCS_HIP_C128 ? 1.0 : resident ? 2.8 : 4.8;
     cost[i] = unit * double(amp) *
               double(uint64_t(1) << c.num_qubits) * (ops + 1.0);

@@ -399,8 +399,9 @@ __global__ __launch_bounds__(1 << kPThrBits, 5) void k_gate_pass(
                        ? 0
                        : __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> (tb - RB));
   const int tid = int(threadIdx.x) - (half << (tb - RB));
-  // a tile of fewer than 1024 amplitudes still takes a whole wave, whose
-  // lanes past the tile compute on copies and store nothing
+  // a tile of fewer than 64 threads (7 qubits, 4 amplitudes a thread) still
+  // takes a whole wave, whose lanes past the tile compute on copies and store
+  // nothing
   const bool in = tid < (1 << (tb - RB));
   // amplitude index of the tile, and of the place it is stored in
   uint64_t base = pass_tile(prog, xcd_order(blockIdx.x, gridDim.x)), home = base;

@@ -75,7 +75,7 @@ enum : uint8_t {
   kPAnti = 8,      // m01, m10
   kPDiag = 12,     // m00, m11
   kPPhase = 16,    // m11; under conditions
-  kPEuler = 20,    // diag(a, conj a), [[c, -s], [s, c]], diag(b, conj b)
+  kPEuler = 20,    // diag(a, conj a), [[c, s], [-s, c]], diag(b, conj b)
   kPCPhase = 24,   // + pair index of two register bits: m11
   kPScale = 30,    // every amplitude, under conditions: m11
   kPSelect = 31    // every amplitude: conditions ? m11 : m00

@@ -27,8 +27,11 @@ constexpr int kMaxQubits = 34;
 // Queue of plain gates (gatepass.hip).  A state of up to 6 qubits fits one
 // amplitude per lane of a wave: its gates launch one by one.
 constexpr int kPassMinQubits = 7;
-constexpr int kPassLowBits = 4;      // tiles always hold these index bits: 256-byte runs
-                                     // (28 qubits: 21.8 ms; 3 bits 22.7, 5 bits 24.4)
+// Tiles always hold these index bits: 256-byte runs (28 qubits: 21.8 ms; 3
+// bits 22.7, 5 bits 24.4).  Timed at 28 qubits only: states that fit the
+// caches run more passes for it (17 qubits, 12 layers: 31, with 3 bits 26; 20
+// qubits, 10 layers: 22 with either), which has not been timed.
+constexpr int kPassLowBits = 4;
 constexpr int kPassBigState = 18;    // from here on launches cost less than traffic
 
 struct TimedLaunch {

@@ -725,11 +725,16 @@ __global__ __launch_bounds__(kThreads) void k_sample_wide(
 // two lanes (real and imaginary part) and rewrites the state once, where a
 // sweep per round moved 2 N s each time.  Any starting state is allowed.  The
 // recurrence runs on pairs of doubles, so it adds no error of its own and an
-// amplitude is rounded once instead of every round: from the H layer, 4 to 19
-// qubits and up to 571 rounds, the marked probability is 7.0e-16 off the closed
-// form on average and 3.0e-15 at most, which is the layer's own error, where a
-// sweep per round was 8.9e-16 and 1.7e-14 off (14 qubits, 100 rounds, the
-// recurrence in plain doubles: 2.0e-15, in pairs 1.1e-15).  27 qubits, 16 rounds: 11.7 -> 0.98 ms; 14 qubits,
+// amplitude is rounded once instead of every round: from random states of 8 to
+// 16 qubits the amplitudes are 1.8e-17 off the exact rounds on average and
+// 1.8e-16 at most, with a sweep per round 1.1e-16 and 3.1e-15 (emulated; with
+// A, which is summed in plain doubles, in pairs too 1.0e-17 and 5.5e-17).  From
+// the H layer the layer's own error stays: 4 to 19 qubits and up to 571 rounds,
+// the marked probability is 7.0e-16 off the closed form on average and 3.0e-15
+// at most, with a sweep per round 8.9e-16 and 1.7e-14.  At some sizes the
+// sweeps' roundings happened to offset the layer's (14 qubits, 100 rounds:
+// 9.0e-16, now 1.13e-15, which an exact A leaves as it is; in plain doubles the
+// recurrence gave 2.0e-15).  27 qubits, 16 rounds: 11.7 -> 0.98 ms; 14 qubits,
 // 100 rounds: 0.70 -> 0.032 ms, 0.26 us of it a round.
 
 // partial sums of the amplitudes other than m
@@ -769,7 +774,7 @@ __global__ __launch_bounds__(kThreads) void k_gsum_partial(
 }
 
 // A sum of two doubles and its rounding error (Knuth); pairs added with
-// about 100 significant bits.
+// about 100 significant bits (Joldes, Muller, Popescu 2017, algorithm 6).
 struct Pair {
   double h, l;
 };
@@ -1185,7 +1190,7 @@ static int measure_seq_impl(qcs_hip_state *s, int count, const int *qubits,
 // had; nothing has been launched then.
 static int measure_low(qcs_hip_state *s, int count, const double *u, int *outcomes, bool *done) {
   double2 *a = static_cast<double2 *>(s->vec);
-  // two rows a work-group at least, so that the partials stay a small part
+  // four rows a work-group at least, so that the partials stay a small part
   // of what is read
   auto blocks = [](uint64_t rows) {
     const uint64_t b = rows / 4;
